@@ -358,7 +358,7 @@ def test_the_top_level_holds_only_what_belongs_there():
     tracked = subprocess.check_output(["git", "-C", ROOT, "ls-files"], text=True).splitlines()
     top = sorted({path.split("/")[0] for path in tracked})
     expected = {".gitignore", ".gpurunignore", "README.md", "DESIGN.md", "INTEGRATION.md", "SURVEY.md", "BASELINE.md", "BASELINE.json",
-                "VERDICT.md", "ADVICE.md", "__graft_entry__.py", "bench.py", "cudadma_amd", "include", "oracle", "profiles", "tests"}
+                "VERDICT.md", "ADVICE.md", "__graft_entry__.py", "bench.py", "cudadma_amd", "include", "oracle", "perf", "profiles", "tests"}
     records = re.compile(r"^(BENCH|GPUTEST|MULTICHIP|SCALE|COPYCHECK|PROGRESS)(_r\d+)?\.(json|jsonl)$")
     strays = [name for name in top if name not in expected and not records.match(name)]
     assert not strays, f"unexpected entries at the repository root: {strays}"
