@@ -59,6 +59,7 @@ struct GridState {
   int row0, col0;        // slot of this thread in round 0
   int drow, dcol;        // slot advance per round
   int rounds, steps, sure_rounds;
+  int whole_rounds;      // dcol == 0: leading rounds in which every thread has a row
 
   __host__ __device__ __forceinline__ void init(const int alignment, const int max_lds, const int e, const int n,
                                        const int t, const int tid)
@@ -74,6 +75,7 @@ struct GridState {
     rounds = ceil_div(n * W, t);
     steps = ceil_div(rounds, max_lds);
     sure_rounds = (W == LPE) ? (n * W) / t : 0;
+    whole_rounds = (dcol == 0 && drow > 0) ? n / drow : 0;
   }
   __host__ __device__ __forceinline__ GridCursor begin() const { return GridCursor{row0, col0}; }
   __host__ __device__ __forceinline__ void advance(GridCursor& c) const

@@ -231,6 +231,9 @@ private:
     m_dst_stride = dst_stride;
   }
 
+  // Some chunk slots of every row hold nothing (rows are not a power of two, or a multiple of 64, chunks long).
+  __device__ __forceinline__ bool padded_rows() const { return m_grid.W != m_grid.LPE; }
+
   // The direct path needs the 64 lanes of a wavefront to land on 64 consecutive
   // chunks of LDS: rows at least one wavefront wide, or unpadded rows packed
   // back to back.  Otherwise the register path is taken.
@@ -256,17 +259,33 @@ private:
       // one offset instead of a 64-bit address per load in flight, and the per-load part is scalar arithmetic.
       if (m_grid.dcol == 0) {
         const long long lane_part = (long long)(m_grid.row0 * m_src_stride + m_grid.col0 * ALIGNMENT);
+        // the same value in every lane (object parameters are); saying so keeps it in scalar registers
+        auto rows_down = [&](const int round) __attribute__((always_inline)) {
+          const unsigned long long bytes = (unsigned long long)((long long)(round * m_grid.drow) * (long long)m_src_stride);
+          return (long long)(((unsigned long long)scalar_u32((unsigned)(bytes >> 32)) << 32) | (unsigned long long)scalar_u32((unsigned)bytes));
+        };
+        if (padded_rows()) {
+          // Threads on the padding of a row have no column in any round, so they are sent around all loads of the step at
+          // once; whether a thread has a row only matters in the last round.  A branch of its own around every load lets the
+          // compiler reuse the registers of one load's address for the next, and it pays for that with s_waitcnt vmcnt(0)
+          // between the loads, one load in flight at a time
+          // (2-D stencil example, 960 x 160 x 200, tiles of 12 rows of 320 B: 561 us with the branches, 264 without).
+          if (m_grid.col0 < m_grid.LPE) {
+            const int bytes = m_grid.chunk_bytes(ALIGNMENT, cur);
+#pragma unroll
+            for (int k = 0; k < MAX_LDS; ++k) {
+              const int round = step * MAX_LDS + k;
+              if (round < m_grid.whole_rounds || m_grid.row0 + round * m_grid.drow < m_grid.N)
+                load_chunk<ALIGNMENT, ALIGNMENT, GLOBAL_LOAD, LOAD_QUAL>(m_buf[k], m_src + rows_down(round) + lane_part, bytes);
+            }
+          }
+          return;
+        }
 #pragma unroll
         for (int k = 0; k < MAX_LDS; ++k) {
-          if (m_grid.live(step * MAX_LDS + k, cur)) {
-            // the same value in every lane (object parameters are); saying so keeps it in scalar registers
-            const long long rows_down = (long long)((step * MAX_LDS + k) * m_grid.drow) * (long long)m_src_stride;
-            const long long uniform = (long long)(
-                ((unsigned long long)__builtin_amdgcn_readfirstlane((unsigned)((unsigned long long)rows_down >> 32)) << 32) |
-                (unsigned long long)__builtin_amdgcn_readfirstlane((unsigned)(unsigned long long)rows_down));
-            load_chunk<ALIGNMENT, ALIGNMENT, GLOBAL_LOAD, LOAD_QUAL>(m_buf[k], m_src + uniform + lane_part,
+          if (m_grid.live(step * MAX_LDS + k, cur))
+            load_chunk<ALIGNMENT, ALIGNMENT, GLOBAL_LOAD, LOAD_QUAL>(m_buf[k], m_src + rows_down(step * MAX_LDS + k) + lane_part,
                                                                      m_grid.chunk_bytes(ALIGNMENT, cur));
-          }
           m_grid.advance(cur);
         }
         return;
@@ -286,6 +305,22 @@ private:
   __device__ __forceinline__ void store_step(char* dst, const int step, hipdma::detail::GridCursor& cur) const
   {
     using namespace hipdma::detail;
+    if (m_grid.dcol == 0 && padded_rows()) {
+      // as in load_step: the column is looked at once, the row in the last round
+      if (m_grid.col0 < m_grid.LPE) {
+        const int bytes = m_grid.chunk_bytes(ALIGNMENT, cur);
+#pragma unroll
+        for (int k = 0; k < MAX_LDS; ++k) {
+          if (step * MAX_LDS + k < m_grid.whole_rounds || cur.row < m_grid.N)
+            store_chunk<ALIGNMENT, ALIGNMENT, STORE_QUAL>(
+                m_buf[k], dst + cur.row * m_dst_stride + lds_col<store_is_swizzled(STORE_QUAL)>(cur) * ALIGNMENT, bytes);
+          cur.row += m_grid.drow;
+        }
+      } else {
+        cur.row += MAX_LDS * m_grid.drow;
+      }
+      return;
+    }
 #pragma unroll
     for (int k = 0; k < MAX_LDS; ++k) {
       if (m_grid.live(step * MAX_LDS + k, cur))
