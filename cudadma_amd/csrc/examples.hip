@@ -35,8 +35,7 @@ const char* const kGemvNames[] = {
 };
 
 // ---- 2-D stencil ----
-constexpr int kTileX = 32, kTileY = 4, kRadius = 4;
-constexpr int kStencilDma = 64, kStencilBpt = 64, kStencilAlign = 16;
+constexpr int kUnitX = 32, kUnitY = 4, kRadius = 4;     // the dimensions are multiples of the reference's tile
 const char* const kStencilNames[] = {
   "warp specialized, single buffer",
   "warp specialized, double buffer",
@@ -45,33 +44,48 @@ const char* const kStencilNames[] = {
   "non warp specialized, double buffer",
 };
 
-template<int REACH>
-void launch_stencil(int variant, dim3 grid, hipStream_t s, const float2* src, float2* dst, int offset, int row_stride,
-                    int slice_stride, int z_steps)
+template<typename TILE, int REACH>
+void launch_stencil(int variant, hipStream_t s, const float2* src, float2* dst, examples::StencilGrid g, int dimz)
 {
-  constexpr int kCompute = kTileX * kTileY;
+  g.tiles_x = (g.dimx + TILE::kX - 1) / TILE::kX;
+  g.tiles_y = (g.dimy + TILE::kY - 1) / TILE::kY;
+  g.items = g.tiles_x * g.tiles_y * dimz;
+  // As many workgroups as share the pairs evenly, in whole rounds over the eight XCDs, up to `per_cu` per compute unit: one
+  // 23 KiB tile of loads in flight is what volumes beyond the caches run best with (960 x 160 x 200: 95 us with one
+  // workgroup per compute unit, 113 / 128 / 120 with two / three / four), and with the flat tile (9 KiB) four of them (133 / 98 /
+  // 130 us with two / four / six).
+  const int per_cu = TILE::kY >= 32 ? 1 : 4;
+  const int most = workloads::persistent_grid(g.items, per_cu);
+  const int rounds = (g.items + most - 1) / most;
+  int grid = (g.items + rounds - 1) / rounds;
+  if (grid > 8) grid = (grid + 7) / 8 * 8;
+  const dim3 blocks((unsigned)grid);
+  constexpr int kCompute = TILE::kComputeThreads, kDma = TILE::kDmaThreads;
   switch (variant) {
-    case 0:
-      hipLaunchKernelGGL((stencil_2D_warp_specialized_single_buffer<kStencilAlign, kStencilBpt, kTileX, kTileY, kRadius, REACH, kStencilDma>),
-                         grid, dim3(kCompute + kStencilDma), 0, s, src, dst, offset, row_stride, slice_stride, z_steps);
-      break;
-    case 1:
-      hipLaunchKernelGGL((stencil_2D_warp_specialized_double_buffer<kStencilAlign, kStencilBpt, kTileX, kTileY, kRadius, REACH, kStencilDma>),
-                         grid, dim3(kCompute + 2 * kStencilDma), 0, s, src, dst, offset, row_stride, slice_stride, z_steps);
-      break;
-    case 2:
-      hipLaunchKernelGGL((stencil_2D_warp_specialized_manual_buffer<kStencilAlign, kStencilBpt, kTileX, kTileY, kRadius, REACH, kStencilDma>),
-                         grid, dim3(kCompute + kStencilDma), 0, s, src, dst, offset, row_stride, slice_stride, z_steps);
-      break;
-    case 3:
-      hipLaunchKernelGGL((stencil_2D_non_warp_specialized_single_buffer<kStencilAlign, kStencilBpt, kTileX, kTileY, kRadius, REACH>),
-                         grid, dim3(kCompute), 0, s, src, dst, offset, row_stride, slice_stride, z_steps);
-      break;
-    default:
-      hipLaunchKernelGGL((stencil_2D_non_warp_specialized_double_buffer<kStencilAlign, kStencilBpt, kTileX, kTileY, kRadius, REACH>),
-                         grid, dim3(kCompute), 0, s, src, dst, offset, row_stride, slice_stride, z_steps);
-      break;
+    case 0: hipLaunchKernelGGL((stencil_2D_warp_specialized_single_buffer<TILE, REACH>), blocks, dim3(kCompute + kDma), 0, s, src, dst, g); break;
+    case 1: hipLaunchKernelGGL((stencil_2D_warp_specialized_double_buffer<TILE, REACH>), blocks, dim3(kCompute + 2 * kDma), 0, s, src, dst, g); break;
+    case 2: hipLaunchKernelGGL((stencil_2D_warp_specialized_manual_buffer<TILE, REACH>), blocks, dim3(kCompute + kDma), 0, s, src, dst, g); break;
+    case 3: hipLaunchKernelGGL((stencil_2D_non_warp_specialized_single_buffer<TILE, REACH>), blocks, dim3(kCompute), 0, s, src, dst, g); break;
+    default: hipLaunchKernelGGL((stencil_2D_non_warp_specialized_double_buffer<TILE, REACH>), blocks, dim3(kCompute), 0, s, src, dst, g); break;
   }
+}
+
+typedef StencilTile<64, 32, 4, kRadius, 128> LargeTile;
+typedef StencilTile<64, 8, 2, kRadius, 64> FlatTile;
+typedef StencilTile<32, 4, 1, kRadius, 64> SmallTile;
+
+template<int REACH>
+void launch_stencil(int variant, hipStream_t s, const float2* src, float2* dst, const examples::StencilGrid& g, int dimz)
+{
+  // Tall tiles read 1.4 cells per cell computed, flat ones 2.25, most of them from the L2: worth 3 to 8 % once the volume
+  // lies beyond the Infinity Cache (960 x 160 x 200: 95 against 98 us, 512 x 512 x 100: 80 against 85).  Where the caches hold
+  // it the flat tiles spread the work better (128 x 512 x 58: 14.7 against 16.9 us), and where 32 does not divide the height the
+  // rows computed twice cost more (960 x 164 x 100: 53 against 58 us).
+  const bool beyond_caches = 16LL * g.dimx * g.dimy * dimz > (192LL << 20);
+  const bool even = (g.dimy + 31) / 32 * 32 == (g.dimy + 7) / 8 * 8;
+  if (g.dimx >= 64 && g.dimy >= 32 && beyond_caches && even) launch_stencil<LargeTile, REACH>(variant, s, src, dst, g, dimz);
+  else if (g.dimx >= 64 && g.dimy >= 8) launch_stencil<FlatTile, REACH>(variant, s, src, dst, g, dimz);
+  else launch_stencil<SmallTile, REACH>(variant, s, src, dst, g, dimz);
 }
 
 template<typename T, int N> constexpr int count_of(T (&)[N]) { return N; }
@@ -181,7 +195,7 @@ extern "C" int cudadma_example_stencil2d(int variant, const float* d_src, float*
     return CUDADMA_ERANGE;
   }
   CUDADMA_REQUIRE(dimx > 0 && dimy > 0 && dimz > 0, "dimensions must be positive (%d x %d x %d)", dimx, dimy, dimz);
-  CUDADMA_REQUIRE((dimx % kTileX) == 0 && (dimy % kTileY) == 0, "dimx must be a multiple of %d and dimy of %d", kTileX, kTileY);
+  CUDADMA_REQUIRE((dimx % kUnitX) == 0 && (dimy % kUnitY) == 0, "dimx must be a multiple of %d and dimy of %d", kUnitX, kUnitY);
   CUDADMA_REQUIRE(variant == 0 || variant == 3 || (dimz % 2) == 0, "dimz (%d) must be even for the variants with two buffers", dimz);
   CUDADMA_REQUIRE(d_src != nullptr && d_dst != nullptr, "NULL pointer");
   CUDADMA_REQUIRE(cudadma_host::aligned_to(d_src, 16) && cudadma_host::aligned_to(d_dst, 8), "src must be 16-byte, dst 8-byte aligned");
@@ -189,14 +203,12 @@ extern "C" int cudadma_example_stencil2d(int variant, const float* d_src, float*
   const long long slice_stride = (dimy + 2 * kRadius) * row_stride;
   const long long offset = kRadius * slice_stride + kRadius * row_stride + kRadius;
   CUDADMA_REQUIRE(slice_stride * (dimz + 2 * kRadius) <= 0x7fffffffLL / 8, "volume too large for int element offsets");
-  const dim3 grid(dimx / kTileX, dimy / kTileY);
   hipStream_t s = (hipStream_t)stream;
   const float2* src = reinterpret_cast<const float2*>(d_src);
   float2* dst = reinterpret_cast<float2*>(d_dst);
-  if (full_cross)
-    launch_stencil<kRadius>(variant, grid, s, src, dst, (int)offset, (int)row_stride, (int)slice_stride, dimz);
-  else
-    launch_stencil<kRadius - 1>(variant, grid, s, src, dst, (int)offset, (int)row_stride, (int)slice_stride, dimz);
+  const examples::StencilGrid g = {dimx, dimy, 0, 0, (int)offset, (int)row_stride, (int)slice_stride, 0, cudadma_host::aligned_to(d_dst, 16)};
+  if (full_cross) launch_stencil<kRadius>(variant, s, src, dst, g, dimz);
+  else launch_stencil<kRadius - 1>(variant, s, src, dst, g, dimz);
   CUDADMA_HIP_CHECK(hipGetLastError());
   return CUDADMA_OK;
 }

@@ -118,6 +118,29 @@ def test_stencil2d(dev, variant, full_cross, dims):
     assert np.array_equal(ddst.cpu().numpy().ravel(), want)
 
 
+# every tile shape, and dimensions that the tile does not divide (its last tile moves back to fit): 32 x 4 below 64 columns or 8
+# rows, 64 x 8 above, 64 x 32 where the volume exceeds the caches
+@pytest.mark.parametrize("variant", range(5))
+@pytest.mark.parametrize("full_cross", [False, True])
+@pytest.mark.parametrize("dims", [(32, 20, 2), (96, 4, 6), (64, 8, 2), (96, 12, 4), (160, 36, 6), (64, 44, 130), (288, 60, 740)])
+def test_stencil2d_tile_shapes(dev, variant, full_cross, dims):
+    O = ol.load()
+    dimx, dimy, dimz = dims
+    r = ex.STENCIL2D_RADIUS
+    shape = (dimz + 2 * r, dimy + 2 * r, dimx + 2 * r, 2)
+    src = ol.uniform(int(np.prod(shape)), 33)
+    want = np.full(src.size, -7.0, dtype=np.float32)
+    O.oracle_stencil2d(ptr(src), ptr(want), dimx, dimy, dimz, r, r if full_cross else r - 1)
+    dsrc = torch.from_numpy(src).to(dev).view(shape)
+    buf = torch.full((src.size + 2,), -7.0, dtype=torch.float32, device=dev)
+    for first in (0, 2):                                   # a destination that is 16-byte aligned, and one that is 8-byte aligned
+        ddst = buf[first:first + src.size].view(shape)
+        ex.stencil2d(dsrc, ddst, variant, full_cross)
+        torch.cuda.synchronize()
+        assert np.array_equal(ddst.cpu().numpy().ravel(), want)
+        buf.fill_(-7.0)
+
+
 def test_stencil2d_argument_checks(dev):
     r = ex.STENCIL2D_RADIUS
     odd = torch.zeros((3 + 2 * r, 4 + 2 * r, 32 + 2 * r, 2), dtype=torch.float32, device=dev)
