@@ -25,14 +25,35 @@ const char* const kSaxpyNames[] = {
 constexpr int kGemvCompute = 128;
 constexpr int kGemvDmaPerLd = 64;
 constexpr int kGemvVecElmts = 256;          // columns per hand-off when only the vector is staged
-constexpr int kGemvPanelCols = 32;          // columns per hand-off when the matrix panel is staged too
+constexpr int kGemvPanelCols = 32;          // columns per hand-off when the matrix panel is staged too (variant 3: the unit of m)
 constexpr int kGemvMatLds = 2;              // DMA wavefronts on the matrix panel
 const char* const kGemvNames[] = {
   "vector staged by cudaDMASequential, one buffer",
   "vector staged by two cudaDMASequential on shared DMA threads",
   "vector by cudaDMASequential + 32-column panel by cudaDMAStrided, one buffer each",
-  "vector by cudaDMASequential + 32-column panel by cudaDMAStrided, two buffers each",
+  "vector by cudaDMASequential + panel of 32 to 256 columns by CudaDMAStrided, two buffers each",
 };
+
+template<int ROWS, int COLS, int VEC_DMA, int MAT_DMA>
+void launch_sgemv_panels(hipStream_t s, int n, int m, float alpha, const float* a, int lda, const float* x, float* y)
+{
+  hipLaunchKernelGGL((sgemvn_both_double<ROWS, COLS, VEC_DMA, MAT_DMA>), dim3((n + ROWS - 1) / ROWS),
+                     dim3((sgemv_both_double_threads<ROWS, VEC_DMA, MAT_DMA>())), 0, s, n, m, alpha, a, lda, x, y);
+}
+
+// The narrowest row tile that gives no compute unit a second workgroup: a row is one chain of multiply-adds whatever the tile, so
+// more and narrower workgroups share the bytes (4096 x 4096: 30 / 31 / 36 / 59 us with tiles of 16 / 32 / 64 / 128 rows); beyond one
+// workgroup per compute unit the memory counts, and with it the length of the pieces of a column (8192 x 8192: 100 / 60 / 70 us with
+// 16 / 32 / 64 rows, 16384 x 16384: 344 / 206 / 170).  A panel needs m >= its columns; what is shorter, and strides at which
+// the 31 rows a DMA thread may lie into a column group overflow 32 bits, go through the panel of 32 columns.
+void launch_sgemv_double(hipStream_t s, int n, int m, float alpha, const float* a, int lda, const float* x, float* y)
+{
+  const int cus = workloads::device_cus();
+  if (m < 256 || lda > (1 << 24)) launch_sgemv_panels<kGemvCompute, kGemvPanelCols, kGemvDmaPerLd, kGemvMatLds * kGemvDmaPerLd>(s, n, m, alpha, a, lda, x, y);
+  else if ((n + 15) / 16 <= cus) launch_sgemv_panels<16, 256, 64, 128>(s, n, m, alpha, a, lda, x, y);
+  else if ((n + 31) / 32 <= cus) launch_sgemv_panels<32, 256, 64, 128>(s, n, m, alpha, a, lda, x, y);
+  else launch_sgemv_panels<64, 128, 64, 256>(s, n, m, alpha, a, lda, x, y);
+}
 
 // ---- 2-D stencil ----
 constexpr int kUnitX = 32, kUnitY = 4, kRadius = 4;     // the dimensions are multiples of the reference's tile
@@ -178,10 +199,7 @@ extern "C" int cudadma_example_sgemv(int variant, int n, int m, float alpha, con
       hipLaunchKernelGGL((sgemvn_both_single<kGemvCompute, kGemvDmaPerLd, kGemvPanelCols, kGemvMatLds>), dim3(grid),
                          dim3(kGemvCompute + (1 + kGemvMatLds) * kGemvDmaPerLd), 0, s, n, m, alpha, d_a, lda, d_x, d_y);
       break;
-    default:
-      hipLaunchKernelGGL((sgemvn_both_double<kGemvCompute, kGemvDmaPerLd, kGemvPanelCols, kGemvMatLds>), dim3(grid),
-                         dim3(kGemvCompute + 2 * (1 + kGemvMatLds) * kGemvDmaPerLd), 0, s, n, m, alpha, d_a, lda, d_x, d_y);
-      break;
+    default: launch_sgemv_double(s, n, m, alpha, d_a, lda, d_x, d_y); break;
   }
   CUDADMA_HIP_CHECK(hipGetLastError());
   return CUDADMA_OK;

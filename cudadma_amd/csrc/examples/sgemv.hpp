@@ -17,6 +17,8 @@
 
 namespace examples {
 
+typedef float f32x4_t __attribute__((ext_vector_type(4)));
+
 // Vector staged in one buffer; the matrix is read straight from global memory.
 // Launch with COMPUTE_THREADS + DMA_THREADS_PER_LD threads.
 template<int COMPUTE_THREADS, int DMA_THREADS_PER_LD, int VEC_ELMTS>
@@ -139,60 +141,118 @@ __global__ void sgemvn_both_single(int n, int m, float alpha, const float* __res
 }
 
 // Vector and matrix panel staged through two buffers each, four objects on
-// disjoint DMA wavefronts.
-// Launch with COMPUTE_THREADS + 2 * (1 + MAT_LDS) * DMA_THREADS_PER_LD threads.
-template<int COMPUTE_THREADS, int DMA_THREADS_PER_LD, int VEC_ELMTS, int MAT_LDS>
-__global__ void sgemvn_both_double(int n, int m, float alpha, const float* __restrict__ A, int lda,
-                                   const float* __restrict__ x, float* __restrict__ y)
+// disjoint DMA wavefronts.  A workgroup owns ROWS rows; the panels hold COLS columns,
+// and the last one is moved back to end with column m - 1, its columns that were
+// summed before are skipped (m >= COLS, m and COLS multiples of 32).
+//
+// What bounds it: a row's sum is one chain of multiply-adds in ascending column order, 8 cycles each (4096 columns:
+// 14 us), and the wavefront that runs it also issues 12 LDS reads per 16 columns (160 cycles per 16 columns with the LDS to
+// itself, 230 next to the DMA wavefronts).  4096 x 4096: 59 us with panels of 128 rows x 32 columns (32 workgroups,
+// 128 hand-offs), 30 with 16 x 256.  Fewer DMA wavefronts leave too few bytes in flight (one per panel: 40 us).
+// Launch with sgemv_both_double_threads<ROWS, VEC_DMA, MAT_DMA>() threads.
+template<int ROWS, int VEC_DMA_THREADS, int MAT_DMA_THREADS>
+constexpr int sgemv_both_double_threads() { return (ROWS < 64 ? 64 : ROWS) + 2 * (VEC_DMA_THREADS + MAT_DMA_THREADS); }
+
+// 16 columns of a panel on their way from LDS to the chain of a compute thread.
+template<int ROWS>
+struct SgemvBlock {
+  float a[16];
+  f32x4_t x[4];
+  __device__ __forceinline__ void load(const float* mat, const float* vec, const int row, const int col)
+  {
+    // one base address per group of columns that the offsets of ds_read2_b32 or ds_read2st64_b32 reach
+    constexpr int kReach = ROWS == 32 ? 8 : 16;
+#pragma unroll
+    for (int g = 0; g < 16; g += kReach) {
+      int base = (col + g) * ROWS + row;
+      asm("" : "+v"(base));
+#pragma unroll
+      for (int j = 0; j < kReach; ++j) a[g + j] = mat[base + j * ROWS];
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j) x[j] = *(const f32x4_t*)(vec + col + 4 * j);
+  }
+  __device__ __forceinline__ float chain(float res) const
+  {
+#pragma unroll
+    for (int j = 0; j < 16; ++j) res = __builtin_fmaf(a[j], x[j / 4][j % 4], res);
+    return res;
+  }
+};
+
+// Sums the columns [first, COLS) of a panel; both are multiples of 32.
+// The reads of one block go out back to back under the sums of the other: read and multiply-add in turn issue at
+// half the speed (266 against 160 cycles per 16 columns), and left alone the scheduler reads a block right before it is needed.
+template<int ROWS, int COLS>
+__device__ __forceinline__ float sgemv_panel(const float* mat, const float* vec, const int row, const int first, float res)
 {
-  __shared__ __attribute__((aligned(16))) float buff0[VEC_ELMTS];
-  __shared__ __attribute__((aligned(16))) float buff1[VEC_ELMTS];
-  __shared__ __attribute__((aligned(16))) float mat0[VEC_ELMTS][COMPUTE_THREADS];
-  __shared__ __attribute__((aligned(16))) float mat1[VEC_ELMTS][COMPUTE_THREADS];
+  SgemvBlock<ROWS> even, odd;
+  even.load(mat, vec, row, first);
+  for (int c = first; c < COLS; c += 32) {
+    odd.load(mat, vec, row, c + 16);
+    __builtin_amdgcn_sched_barrier(0);
+    res = even.chain(res);
+    __builtin_amdgcn_sched_barrier(0);
+    even.load(mat, vec, row, c + 32 < COLS ? c + 32 : 0);
+    __builtin_amdgcn_sched_barrier(0);
+    res = odd.chain(res);
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  return res;
+}
 
-  typedef cudaDMASequential<true, 16, 4 * VEC_ELMTS, DMA_THREADS_PER_LD> vec_dma_t;
-  typedef cudaDMAStrided<true, 16, 4 * COMPUTE_THREADS, MAT_LDS * DMA_THREADS_PER_LD, VEC_ELMTS> mat_dma_t;
-  constexpr int kMatThreads = MAT_LDS * DMA_THREADS_PER_LD;
-  vec_dma_t dma_vec_0(1, COMPUTE_THREADS, COMPUTE_THREADS);
-  vec_dma_t dma_vec_1(2, COMPUTE_THREADS, COMPUTE_THREADS + DMA_THREADS_PER_LD);
-  mat_dma_t dma_mat_0(3, COMPUTE_THREADS, COMPUTE_THREADS + 2 * DMA_THREADS_PER_LD, 4 * lda);
-  mat_dma_t dma_mat_1(4, COMPUTE_THREADS, COMPUTE_THREADS + 2 * DMA_THREADS_PER_LD + kMatThreads, 4 * lda);
+template<int ROWS, int COLS, int VEC_DMA_THREADS, int MAT_DMA_THREADS>
+__global__ __launch_bounds__((sgemv_both_double_threads<ROWS, VEC_DMA_THREADS, MAT_DMA_THREADS>()))
+void sgemvn_both_double(int n, int m, float alpha, const float* __restrict__ A, int lda, const float* __restrict__ x,
+                        float* __restrict__ y)
+{
+  constexpr int kCompute = ROWS < 64 ? 64 : ROWS;       // with fewer rows the rest of the wavefront doubles them
+  __shared__ __attribute__((aligned(16))) float buff0[COLS];
+  __shared__ __attribute__((aligned(16))) float buff1[COLS];
+  __shared__ __attribute__((aligned(16))) float mat0[COLS * ROWS];
+  __shared__ __attribute__((aligned(16))) float mat1[COLS * ROWS];
 
-  if (threadIdx.x < COMPUTE_THREADS) {
+  // a thread holds its share of a panel in registers: the next panel is on its way while this one is read
+  constexpr int kMatBytes = 4 * ROWS * COLS / MAT_DMA_THREADS;
+  typedef cudaDMASequential<true, 16, 4 * COLS, VEC_DMA_THREADS> vec_dma_t;
+  typedef CudaDMAStrided<true, 16, kMatBytes, 4 * ROWS, MAT_DMA_THREADS, COLS> mat_dma_t;
+  vec_dma_t dma_vec_0(1, kCompute, kCompute);
+  vec_dma_t dma_vec_1(2, kCompute, kCompute + VEC_DMA_THREADS);
+  mat_dma_t dma_mat_0(3, kCompute, kCompute + 2 * VEC_DMA_THREADS, 4 * lda, 4 * ROWS);
+  mat_dma_t dma_mat_1(4, kCompute, kCompute + 2 * VEC_DMA_THREADS + MAT_DMA_THREADS, 4 * lda, 4 * ROWS);
+
+  const int panels = (m + COLS - 1) / COLS;
+  const int row0 = blockIdx.x * ROWS;
+  // first column of panel p
+  auto begin = [&](const int p) { const int c = p * COLS; return c < m - COLS ? c : m - COLS; };
+
+  if (threadIdx.x < kCompute) {
     dma_vec_0.start_async_dma();
     dma_mat_0.start_async_dma();
-    if (VEC_ELMTS < m) { dma_vec_1.start_async_dma(); dma_mat_1.start_async_dma(); }
+    if (panels > 1) { dma_vec_1.start_async_dma(); dma_mat_1.start_async_dma(); }
+    const int row = threadIdx.x % ROWS;
     float res = 0.0f;
-    for (int i = 0; i < m; i += 2 * VEC_ELMTS) {
+    for (int p = 0; p < panels; p += 2) {
       dma_vec_0.wait_for_dma_finish();
       dma_mat_0.wait_for_dma_finish();
-#pragma unroll
-      for (int j = 0; j < VEC_ELMTS; ++j)
-        res = __builtin_fmaf(mat0[j][threadIdx.x], buff0[j], res);
-      if (i + 2 * VEC_ELMTS < m) { dma_vec_0.start_async_dma(); dma_mat_0.start_async_dma(); }
-      if (i + VEC_ELMTS < m) {
+      res = sgemv_panel<ROWS, COLS>(mat0, buff0, row, p * COLS - begin(p), res);
+      if (p + 2 < panels) { dma_vec_0.start_async_dma(); dma_mat_0.start_async_dma(); }
+      if (p + 1 < panels) {
         dma_vec_1.wait_for_dma_finish();
         dma_mat_1.wait_for_dma_finish();
-#pragma unroll
-        for (int j = 0; j < VEC_ELMTS; ++j)
-          res = __builtin_fmaf(mat1[j][threadIdx.x], buff1[j], res);
-        if (i + 3 * VEC_ELMTS < m) { dma_vec_1.start_async_dma(); dma_mat_1.start_async_dma(); }
+        res = sgemv_panel<ROWS, COLS>(mat1, buff1, row, (p + 1) * COLS - begin(p + 1), res);
+        if (p + 3 < panels) { dma_vec_1.start_async_dma(); dma_mat_1.start_async_dma(); }
       }
     }
-    const int row = blockIdx.x * COMPUTE_THREADS + threadIdx.x;
-    if (row < n) y[row] = alpha * res;
+    if (threadIdx.x < ROWS && row0 + row < n) y[row0 + row] = alpha * res;
   } else if (dma_vec_0.owns_this_thread()) {
-    for (int i = 0; i < m; i += 2 * VEC_ELMTS) dma_vec_0.execute_dma(x + i, buff0);
+    for (int p = 0; p < panels; p += 2) dma_vec_0.execute_dma(x + begin(p), buff0);
   } else if (dma_vec_1.owns_this_thread()) {
-    for (int i = VEC_ELMTS; i < m; i += 2 * VEC_ELMTS) dma_vec_1.execute_dma(x + i, buff1);
+    for (int p = 1; p < panels; p += 2) dma_vec_1.execute_dma(x + begin(p), buff1);
   } else if (dma_mat_0.owns_this_thread()) {
-    const float* panel = A + (long long)blockIdx.x * COMPUTE_THREADS;
-    for (int i = 0; i < m; i += 2 * VEC_ELMTS)
-      dma_mat_0.execute_dma(panel + (long long)lda * i, mat0);
+    for (int p = 0; p < panels; p += 2) dma_mat_0.execute_dma(A + row0 + (long long)lda * begin(p), mat0);
   } else if (dma_mat_1.owns_this_thread()) {
-    const float* panel = A + (long long)blockIdx.x * COMPUTE_THREADS;
-    for (int i = VEC_ELMTS; i < m; i += 2 * VEC_ELMTS)
-      dma_mat_1.execute_dma(panel + (long long)lda * i, mat1);
+    for (int p = 1; p < panels; p += 2) dma_mat_1.execute_dma(A + row0 + (long long)lda * begin(p), mat1);
   }
 }
 

@@ -88,6 +88,25 @@ def test_sgemv_random(dev, variant, n, m, lda):
     assert np.all(got[n:] == 3.0)                          # rows beyond n are not written
 
 
+# the default variant's row tiles (16, 32 and 64 rows by the number of workgroups) and panels: n around the lines between the tiles, m
+# at one panel, between panels (the last one moves back) and below the smallest
+@pytest.mark.parametrize("n", [1, 17, 4096, 4097, 8192, 8209])
+@pytest.mark.parametrize("m", [32, 224, 256, 288, 480, 544, 768])
+def test_sgemv_panels(dev, n, m):
+    O = ol.load()
+    lda = (n + 127) // 128 * 128
+    a = ol.uniform(m * lda, 23).reshape(m, lda)
+    x = ol.uniform(m, 24)
+    want = np.empty(n, dtype=np.float32)
+    O.oracle_sgemv(n, m, -0.75, ptr(a), lda, ptr(x), ptr(want))
+    dy = torch.full((lda,), 3.0, dtype=torch.float32, device=dev)
+    ex.sgemv(-0.75, torch.from_numpy(a).to(dev), torch.from_numpy(x).to(dev), dy, n=n)
+    torch.cuda.synchronize()
+    got = dy.cpu().numpy()
+    assert np.array_equal(got[:n], want)
+    assert np.all(got[n:] == 3.0)
+
+
 def test_sgemv_argument_checks(dev):
     a = torch.zeros((96, 128), dtype=torch.float32, device=dev)
     x = torch.zeros(96, dtype=torch.float32, device=dev)
