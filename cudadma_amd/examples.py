@@ -1,23 +1,14 @@
 """Python face of the example consumers (saxpy, sgemv, 2-D stencil): the programs
 the reference ships under src/examples/, here as launchers in libcudadma_amd.so.
 Every function takes torch CUDA tensors and launches on torch's current stream."""
-import ctypes
-
 import torch
 
 from ._lib import check, lib
+from .workloads import _p, _stream
 
 SAXPY, SGEMV, STENCIL2D = range(3)
 STENCIL2D_RADIUS = 4
 STENCIL2D_TILE = (32, 4)
-
-
-def _stream():
-    return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
-
-
-def _p(t):
-    return ctypes.c_void_p(t.data_ptr())
 
 
 def _need(t, what):
