@@ -94,8 +94,12 @@ __device__ __forceinline__ TileWork tile_work(const float* in, float* out, const
     ty = (xcd / 2) * bh + slot / bw;
     b = 0;
   } else {
-    if ((zchunk_and_flags & kXcdFlag) && (gridDim.x % kXcds) == 0)
-      b = (b % kXcds) * (gridDim.x / kXcds) + b / kXcds;
+    if (zchunk_and_flags & kXcdFlag) {
+      // a contiguous run of tiles for each XCD; where eight does not divide the grid the first ones get a tile more
+      // (224 x 416 x 300, 273 workgroups: 71 us without the renumbering, 48 with it)
+      const int xcd = b % kXcds, each = (int)gridDim.x / kXcds, more = (int)gridDim.x % kXcds;
+      b = xcd * each + (xcd < more ? xcd : more) + b / kXcds;
+    }
     tx = b % tiles_x; b /= tiles_x;
     ty = b % tiles_y; b /= tiles_y;
   }
@@ -609,6 +613,36 @@ stencil_all_vec4(const float* __restrict__ in, float* __restrict__ out, const in
 // 32 x 32 tiles at 512^3 depending on the box (tiles of 128 x 8 cells were level with 32 x 32: their rings are twice
 // as large).
 constexpr int kWideTileVariants = 6;
+
+// How many planes a workgroup takes.  Every workgroup pays for about twelve planes before its first output (2 * radius planes of
+// the column plus the wait for them), whatever it then marches through.  A second workgroup on a compute unit slows both by 1.4
+// where the caches hold the grids from one sweep to the next and up to twice where they come from DRAM (512 x 512 x 64, 256 / 512
+// workgroups: 28.4 / 22.8 us, 512 x 512 x 256: 102 / 117; 384 x 320 x 200, 240 / 480: 41.5 / 31.3 from the caches, 43.6 / 53.5 from
+// DRAM); a third waits for its turn.  Of the numbers of chunks that just fill the compute units k times, the one with the least sum
+// of these is taken (192 x 256 x 130: 15.6 us with 288 workgroups of 22 planes, 13.2 with 480 of 13; 128^3: 9.4 -> 6.6;
+// 224 x 416 x 300, 273 / 455: 69 / 35 from the caches, 84 / 61 from DRAM).
+constexpr int kLeastZchunk = 4;
+static int best_zchunk(const long long tiles_xy, const long long bytes, const int nz, const bool dwordx4)
+{
+  const long long cus = workloads::device_cus();
+  // tenths of the time with one; the sweep kernels always want two
+  const long long two = bytes <= (128LL << 20) || !dwordx4 ? 14 : bytes <= (256LL << 20) ? 18 : 20;
+  const long long most = nz / kLeastZchunk > 1 ? nz / kLeastZchunk : 1;
+  int best = nz;
+  long long least = -1;
+  for (int k = 0; k <= 8; ++k) {
+    long long chunks = k == 0 ? 1 : k * cus / tiles_xy;
+    if (chunks < 1) continue;
+    if (chunks > most) chunks = most;
+    const int zchunk = (int)((nz + chunks - 1) / chunks);
+    const long long grid = tiles_xy * ((nz + zchunk - 1) / zchunk);
+    const long long rest = grid % (2 * cus);
+    const long long cost = (12 + zchunk) * (grid / (2 * cus) * two + (rest == 0 ? 0 : rest <= cus ? 10 : two));
+    if (least < 0 || cost < least) { least = cost; best = zchunk; }
+  }
+  return best;
+}
+
 #ifdef STENCIL_WIDE_TILES
 extern "C" int cudadma_halo_stencil_wide_tiles(const float* d_in, float* d_out, int nx, int ny, int nz, int variant, void* stream)
 {
@@ -632,15 +666,9 @@ extern "C" int cudadma_halo_stencil(const float* d_in, float* d_out, int nx, int
   CUDADMA_REQUIRE(cudadma_host::aligned_to(d_in, 16) && cudadma_host::aligned_to(d_out, 16), "pointers must be 16-byte aligned");
   const Coeffs k = {(float)(3.0 * (-205.0 / 72.0)), (float)(8.0 / 5.0), (float)(-1.0 / 5.0), (float)(8.0 / 315.0),
                     (float)(-1.0 / 560.0)};
-  // z is cut into as few chunks as still give every compute unit work: each chunk re-reads
-  // 2*radius + prefetch planes before it produces output.  The dwordx4 kernels run best with one workgroup
-  // per compute unit, with and without the handshake (512^3: 0.200 / 0.206 ms against 0.228 / 0.222 ms with two).
   const long long tiles_xy = (long long)(nx / kTX) * (ny / kTY);
-  const int per_cu = (variant <= 3) ? 1 : 2;
-  long long want_chunks = ((long long)per_cu * workloads::device_cus() + tiles_xy - 1) / tiles_xy;
-  if (want_chunks < 1) want_chunks = 1;
-  int zchunk = workloads::tuning("stencil_zchunk", (int)((nz + want_chunks - 1) / want_chunks));
-  if (zchunk < 16) zchunk = 16;
+  int zchunk = workloads::tuning("stencil_zchunk", best_zchunk(tiles_xy, 4LL * (2LL * nx * ny) * nz, nz, variant <= 3));
+  if (zchunk < kLeastZchunk) zchunk = kLeastZchunk;
   if (zchunk > nz) zchunk = nz;
   const int chunks = (nz + zchunk - 1) / zchunk;
   // knob "stencil_xcd_remap": 2 turns the XCD-aware numbering off, 4 asks for compact blocks instead of slabs

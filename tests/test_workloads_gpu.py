@@ -389,6 +389,19 @@ def test_halo_stencil_under_every_tuning(device, variant, ring, remap, shape):
     assert np.all(err <= STENCIL_RTOL * np.maximum(np.abs(want), 1.0)), float(err.max())
 
 
+# chunks of planes that do not divide the depth, grids that eight XCDs do not divide, fewer planes than a ring is deep
+@pytest.mark.parametrize("shape", [(32, 32, 1), (32, 32, 4), (32, 32, 41), (96, 160, 61), (224, 416, 13), (64, 32, 300), (512, 544, 9)])
+def test_halo_stencil_chunks(device, shape):
+    O = ol.load()
+    nx, ny, nz = shape
+    p = 2 * wl.STENCIL_RADIUS
+    g = ol.uniform((nx + p) * (ny + p) * (nz + p), 1014).reshape(nz + p, ny + p, nx + p)
+    want = np.empty((nz, ny, nx), dtype=np.float32)
+    O.oracle_stencil25(ptr(g), ptr(want), nx, ny, nz, wl.STENCIL_RADIUS)
+    got = wl.halo_stencil(torch.from_numpy(g).to(device), torch.full((nz, ny, nx), float("nan"), device=device)).cpu().numpy()
+    assert np.all(np.abs(got - want) <= 1e-5 * np.maximum(np.abs(want), 1.0))        # 29 fp32 terms below 3, as in the tests above
+
+
 @pytest.mark.parametrize("variant", [0, 1, 6])  # the kernel the benchmark reports, its form with the empty/full handshake, and wide tiles
 def test_halo_stencil_full_size(device, variant):
     n = 512
