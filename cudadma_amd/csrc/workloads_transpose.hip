@@ -776,6 +776,15 @@ extern "C" int cudadma_strided_transpose(const float* d_in, float* d_out, int n,
   CUDADMA_REQUIRE(cudadma_host::aligned_to(d_in, 16) && cudadma_host::aligned_to(d_out, 16), "pointers must be 16-byte aligned");
   const int tiles_per_side = n / kTile;
   const int tiles = tiles_per_side * tiles_per_side;
+  // Variant 0 is the library's choice.  Variant 10's shape, one 16 KB tile in flight per compute unit and streaming loads and stores,
+  // is for matrices from DRAM (16384: 358 us against 456 with variant 11, 4096: 26.2 / 29.8).  Small matrices come from the
+  // Infinity Cache or leave their result there, and its short queue only costs (2112: 9.5 us against 6.8 with variant 11 from the
+  // cache, 9.9 / 8.9 from DRAM; 2816, the last below the line: 14 / 10.6 and 14.1 / 15.2).  Up to two tiles per compute unit
+  // the tile is best moved by every wavefront, with no hand-off (variant 4; 512: 4.0 us against 3.1, 1280: 5.4 / 4.3).
+  if (variant == 0 && workloads::tuning("transpose_workgroups", 0) == 0) {
+    if (tiles <= 2 * workloads::device_cus()) variant = 4;
+    else if (8LL * n * n <= (64LL << 20)) variant = 11;
+  }
   // The kernels with one LDS tile (variants 1 and 4) run best with exactly one workgroup per compute unit, i.e. one
   // 16 KB tile of loads in flight per compute unit, and with the tiles walked down the columns (the workgroups that
   // run together then write whole output rows); the others with four workgroups and bands of 16 tile rows.
@@ -801,7 +810,7 @@ extern "C" int cudadma_strided_transpose(const float* d_in, float* d_out, int n,
     case 9: hipLaunchKernelGGL(transpose_pairs<true>, grid_for(4), dim3(128), 0, s, d_in, d_out, n, tiles, band); break;
     case 0:
     case 10: {
-      // variant 0 is the library's choice: the fastest split (three DMA wavefronts, one compute wavefront, one tile
+      // variant 0 beyond the caches: the fastest split (three DMA wavefronts, one compute wavefront, one tile
       // ahead).  Variant 10 takes the split from the knob "transpose_split" = 100 * DMA wavefronts + 10 * compute
       // wavefronts + tiles ahead (the same default).
       const int code = variant == 0 ? 311 : workloads::tuning("transpose_split", 311);

@@ -402,6 +402,15 @@ def test_halo_stencil_chunks(device, shape):
     assert np.all(np.abs(got - want) <= 1e-5 * np.maximum(np.abs(want), 1.0))        # 29 fp32 terms below 3, as in the tests above
 
 
+# the lines at which the default variants change kernels: one tile on either side
+@pytest.mark.parametrize("n", [1408, 1472, 2880, 2944])
+def test_default_transpose_around_its_lines(device, n):
+    src = wl.fill_uniform(torch.empty(n * n, dtype=torch.float32, device=device), 41).view(n, n)
+    dst = torch.full_like(src, float("nan"))
+    wl.strided_transpose(src, dst)
+    assert torch.equal(dst.view(torch.int32), src.t().contiguous().view(torch.int32))
+
+
 @pytest.mark.parametrize("variant", [0, 1, 6])  # the kernel the benchmark reports, its form with the empty/full handshake, and wide tiles
 def test_halo_stencil_full_size(device, variant):
     n = 512
