@@ -186,8 +186,12 @@ int launch_gather(const float* d_table, const int32_t* d_idx, float* d_out, size
   // 69.5 % on 1.875 GiB, against 74.0 / 68.2 with three).
   const int ahead_wgs = Consumer::kWritesEveryRecord ? 2 : n_records * (size_t)kRecBytes <= (1ull << 30) ? 3 : 4;
   auto grid = [&](const int per_cu) { return dim3((unsigned)workloads::persistent_grid(tiles, per_cu)); };
+  // The library's choice: a short list is over before three workgroups per compute unit with two tiles each have filled their
+  // queues; eight with one tile start sooner (row sums of 256 Ki records: 6.4 against 7.6 us from the caches, 8.7 / 8.9 from DRAM; 32 Ki:
+  // 3.2 / 3.7; copies of 32 Ki: 3.6 / 4.0).  Longer lists gain as much from the caches and lose twice that from DRAM (row sums of
+  // 1 Mi: 22.8 / 24.1 and 28.2 / 25.3).
+  if (variant == 0) variant = n_idx * (size_t)kRecBytes <= (32ull << 20) ? 1 : 6;
   switch (variant) {
-    case 0:
     case 6: hipLaunchKernelGGL((gather_manual<Consumer, 2, true>), grid(ahead_wgs), block, 0, s, d_table, d_idx, d_out, tiles); break;
     case 1: hipLaunchKernelGGL(gather_single<Consumer>, grid(8), block, 0, s, d_table, d_idx, d_out, tiles); break;
     case 2: hipLaunchKernelGGL((gather_manual<Consumer, 2>), grid(6), block, 0, s, d_table, d_idx, d_out, tiles); break;

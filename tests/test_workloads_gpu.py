@@ -411,6 +411,17 @@ def test_default_transpose_around_its_lines(device, n):
     assert torch.equal(dst.view(torch.int32), src.t().contiguous().view(torch.int32))
 
 
+@pytest.mark.parametrize("n_idx", [1 << 18, (1 << 18) + 32])
+def test_default_gather_around_its_line(device, n_idx):
+    recs = (2 << 20) + 64
+    table = wl.fill_uniform(torch.empty(recs * 32, dtype=torch.float32, device=device), 42).view(recs, 32)
+    idx = wl.fill_indices(torch.empty(n_idx, dtype=torch.int32, device=device), recs, 43)
+    out = wl.gather_copy(table, idx, torch.full((n_idx, 32), float("nan"), device=device))
+    assert torch.equal(out.view(torch.int32), table[idx.long()].view(torch.int32))
+    sums = [wl.gather_rowsum(table, idx, torch.full((n_idx // 32, 32), float("nan"), device=device), v) for v in (0, 1, 6)]
+    assert torch.equal(sums[0], sums[1]) and torch.equal(sums[0], sums[2])           # every variant adds in the same order
+
+
 @pytest.mark.parametrize("variant", [0, 1, 6])  # the kernel the benchmark reports, its form with the empty/full handshake, and wide tiles
 def test_halo_stencil_full_size(device, variant):
     n = 512
