@@ -127,8 +127,8 @@ static const VariantInfo kHalo[] = {
 };
 
 static const VariantInfo kGemm[] = {
-  {"the largest workgroup tile that divides the problem and gives every compute unit a tile: variant 9, 3 or 2, else "
-   "variant 1"},
+  {"the library's choice: of variants 1, 2, 3 and 9 that whose tile divides the problem and whose rounds over the compute units "
+   "take least time"},
   {"warp-specialised: two DMA wavefronts per operand with two CudaDMAStrided objects each (two LDS stages, tile two K "
    "steps ahead in flight), four compute wavefronts with v_mfma_f32_32x32x16_bf16, B fragments through "
    "ds_read_b64_tr_b16; 128 x 128 workgroup tile, 64 x 64 per compute wavefront, two workgroups per compute unit"},

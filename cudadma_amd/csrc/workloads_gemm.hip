@@ -1086,13 +1086,23 @@ extern "C" int cudadma_gemm_bf16(const uint16_t* d_a, const uint16_t* d_b, float
   CUDADMA_REQUIRE((long long)k * 2 <= 0x7fffffffLL && (long long)n * 2 <= 0x7fffffffLL, "row pitch must fit an int");
   hipStream_t s = (hipStream_t)stream;
   if (variant == 0) {
-    // the largest tile that divides the problem and still gives every compute unit a tile; the small one otherwise
+    // The tile whose rounds over the compute units cost least.  `full` is the time of a K step of 64 of a whole round in units of
+    // 10 ns, `part` that of a round of few workgroups: up to one per compute unit for the small tile, of which two share one, up to
+    // five eighths of them for the others (they get more of the clock and the memory); `once` is what a tile costs before its
+    // first and after its last K step.  Measured: 3072^3 61 us with 144 tiles of 256 x 256 against 96 with 256 x 128 and 79 with
+    // 128 x 128; 2048 x 3072 x 4096 77 / 63 / 72; 2048^3 41 / 35 / 25; 2816 x 2560 x 640 20 / 17.6 / 16.1.
     const long long cus = workloads::device_cus();
+    auto rounds = [&](const long long tiles, const long long slots, const long long few, const int full, const int part, const int once) {
+      const long long rest = tiles % slots;
+      return (k / kBK) * (tiles / slots * full + (rest == 0 ? 0 : rest <= few ? part : full)) + once;
+    };
     const bool m256 = (m % 256) == 0, n256 = (n % 256) == 0;
-    if (m256 && n256 && (long long)(m / 256) * (n / 256) >= cus) variant = 9;
-    else if (m256 && (long long)(m / 256) * (n / 128) >= cus) variant = 3;
-    else if (n256 && (long long)(m / 128) * (n / 256) >= cus) variant = 2;
-    else variant = 1;
+    long long least = rounds((long long)(m / 128) * (n / 128), 2 * cus, cus, 112, 60, 490);
+    variant = 1;
+    auto consider = [&](const bool fits, const int v, const long long cost) { if (fits && cost < least) { least = cost; variant = v; } };
+    consider(m256, 3, rounds((long long)(m / 256) * (n / 128), cus, cus * 5 / 8, 95, 85, 810));
+    consider(n256, 2, rounds((long long)(m / 128) * (n / 256), cus, cus * 5 / 8, 95, 85, 810));
+    consider(m256 && n256, 9, rounds((long long)(m / 256) * (n / 256), cus, cus * 5 / 8, 160, 110, 1000));
   }
   switch (variant) {
     case 1: return launch_gemm<2, 2>(d_a, d_b, d_c, m, n, k, s);
