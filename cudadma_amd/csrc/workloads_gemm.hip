@@ -44,18 +44,28 @@ struct GemmShape {
 
 // Workgroup -> tile.  Workgroup b runs on XCD b % 8; when the tile grid divides into eight
 // 2-D blocks (4 along m, 2 along n) every XCD gets one compact block, so its L2 holds few
-// distinct A and B panels; otherwise tiles are dealt row-major.
+// distinct A and B panels.  Other grids are walked in bands of up to eight tile rows, down the
+// columns of a band, and every XCD gets an eighth of that walk: the tiles in work on it
+// at one time are about as many rows as columns (tiles dealt row-major instead: 3712 x 4736 x 3712 with 128 x 128 tiles 188 us
+// against 139, 640 x 8064 x 2048 34 / 28).  Grids that do divide keep their blocks: the walk is level or slower there
+// (8192 x 8192 x 1024, 256 x 256 tiles: 140 us against 155).
 __device__ __forceinline__ void tile_of_workgroup(const int b, const int tiles_m, const int tiles_n, int& tile_m, int& tile_n)
 {
+  const int xcd = b & 7, idx = b >> 3;
   if ((tiles_m % 4) == 0 && (tiles_n % 2) == 0) {
-    const int xcd = b & 7, idx = b >> 3;
     const int bm = tiles_m / 4, bn = tiles_n / 2;       // block of one XCD
     tile_m = (xcd >> 1) * bm + idx / bn;
     tile_n = (xcd & 1) * bn + idx % bn;
-  } else {
-    tile_m = b / tiles_n;
-    tile_n = b % tiles_n;
+    return;
   }
+  const int tiles = tiles_m * tiles_n, each = tiles >> 3, more = tiles & 7;
+  const int at = xcd * each + (xcd < more ? xcd : more) + idx;
+  int rows = 1;
+  while (rows < 8 && rows * rows < each) ++rows;
+  const int band = at / (rows * tiles_n), in_band = at - band * rows * tiles_n;
+  const int height = tiles_m - band * rows < rows ? tiles_m - band * rows : rows;
+  tile_n = in_band / height;
+  tile_m = band * rows + in_band - tile_n * height;
 }
 
 // Order of one slice for the instruction scheduler: MFMAs matrix instructions with the READS
@@ -144,7 +154,7 @@ gemm_bf16_ws(const unsigned short* __restrict__ a, const unsigned short* __restr
     // With 128 accumulator registers a SIMD holds one compute wavefront, which has to hide its
     // own LDS latency: the order "request the next slice, then multiply the current one" is
     // pinned against the instruction scheduler.  With the small tile two workgroups share a
-    // compute unit and the scheduler's own order does better.
+    // compute unit and the scheduler's own order does better, and so it does with one (1408 x 2176 x 1920: 22 us against 24).
     constexpr bool kPinned = (WI * WJ >= 8) && (WM * WN == 4);
     // Fragments of one 16-deep slice of the K step: WI row blocks of A, WJ column blocks of B.
     auto load_frags = [&](bf16x8_t (&fa)[WI], bf16x8_t (&fb)[WJ], const char* sa, const char* sb, const int ks)
@@ -890,20 +900,24 @@ gemm_bf16_all_direct(const unsigned short* __restrict__ a, const unsigned short*
 // twice (TCP_TCC_READ_REQ: 12.8 M requests per 4096^3 launch instead of 8.4 M).  Here an A transfer is 256 rows x
 // 128 B for two K steps.  Three A buffers (96 KB) and the four B stages (64 KB) are all of the LDS: an A buffer is
 // free two K steps after its last read and its next transfer has to be complete a step before its first, so two
-// buffers would leave it one K step to land.  The A buffers form a ring indexed at run time (three does not divide
+// buffers would leave it one K step to land.  WI = 4 is that kernel.  With WI = 2 the tile is 128 x 128, all buffers are 80 KB and
+// two workgroups share a compute unit; LDS reads bound it (6 per 4 products; 16 KB a slice and workgroup), and against
+// the warp-specialised kernel of that tile it saves the ds_writes and the hand-offs: 2560 x 2560 x 1024 21.5 -> 18 us,
+// 1024^3 12.4 -> 10.3, 3072 x 2432 x 1408 29.6 -> 24.2 (both with the same order of tiles).  The A buffers form a ring indexed at run time (three does not divide
 // the K steps of every problem); a K step still issues eight loads, four of B and half an A transfer.
+template<int WI>
 __global__ void __launch_bounds__(256)
 gemm_bf16_all_direct_a64(const unsigned short* __restrict__ a, const unsigned short* __restrict__ b, float* __restrict__ c,
                          const int m, const int n, const int k)
 {
-  constexpr int WI = 4, WJ = 4, kBStages = 4, kABufs = 3, kBK4 = 32, kThreads = 256;
-  constexpr int kBM = 256, kBN = 256;
+  constexpr int WJ = WI, kBStages = 4, kABufs = 3, kBK4 = 32, kThreads = 256;
+  constexpr int kBM = 64 * WI, kBN = 64 * WJ;
   constexpr int kARow = 4 * kBK4, kBRow = kBN * 2;                 // 128 B (two K steps) and 512 B, unpadded
   constexpr int kABuf = kBM * kARow, kBStage = kBK4 * kBRow;       // 32 KB and 16 KB
   typedef CudaDMAStrided<false, 16, 16, kARow, kThreads, kBM> dma_a_t;
   typedef CudaDMAStrided<false, 16, 16, kBRow, kThreads, kBK4> dma_b_t;
-  static_assert(dma_a_t::loads_per_thread() == 8 && dma_b_t::loads_per_thread() == 4, "eight loads per thread and K step");
-  constexpr int kLoads = 8;
+  static_assert(dma_a_t::loads_per_thread() == 2 * WI && dma_b_t::loads_per_thread() == WI, "2 * WI loads per thread and K step");
+  constexpr int kLoads = 2 * WI;
   __shared__ __attribute__((aligned(1024))) char lds_a[kABufs * kABuf];
   __shared__ __attribute__((aligned(1024))) char lds_b[kBStages][kBStage];
   dma_a_t dma_a(k * 2, kARow);
@@ -954,7 +968,10 @@ gemm_bf16_all_direct_a64(const unsigned short* __restrict__ a, const unsigned sh
       b_hi[j] = (row + 4) * kBRow + hipdma::swizzled_chunk(row + 4, col_bytes >> 4, kBRow / 16) * 16 + (col_bytes & 15);
     }
   }
-  // Half a K step: sixteen products in four groups; under the first three the fragments of slice q of A buffer
+  // The group of products under which the B fragments are first requested, and reads behind each product: with four groups A, B and
+  // B take one each, with two everything goes under the first, to have landed after the second.
+  constexpr int kBFrom = WI == 4 ? 1 : 0, kReads = WI == 4 ? 1 : 3;
+  // Half a K step: WI * WI products in WI groups; under the first three (one) the fragments of slice q of A buffer
   // `abuf` and of slice ks of B stage `bbuf` are requested into (na, nb); `after_group(i)` places the loads.
   auto half_step = [&](const bf16x8_t (&fa)[WI], const bf16x8_t (&fb)[WJ], bf16x8_t (&na)[WI], bf16x8_t (&nb)[WJ],
                        const int abuf, const int q, const int bbuf, const int ks, auto after_group)
@@ -965,9 +982,10 @@ gemm_bf16_all_direct_a64(const unsigned short* __restrict__ a, const unsigned sh
       if (i == 0) {
 #pragma unroll
         for (int r = 0; r < WI; ++r) na[r] = *(const bf16x8_t*)(sa + r * 32 * kARow + a_lane[q]);
-      } else if (i < 3) {
+      }
+      if (i >= kBFrom && i < kBFrom + WJ / 2) {
 #pragma unroll
-        for (int j = 2 * (i - 1); j < 2 * i; ++j) {
+        for (int j = 2 * (i - kBFrom); j < 2 * (i - kBFrom) + 2; ++j) {
           const bf16x4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4bf16(
               (__attribute__((address_space(3))) bf16x4_t*)(sb + ks * 16 * kBRow + b_lo[j]));
           const bf16x4_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4bf16(
@@ -981,7 +999,7 @@ gemm_bf16_all_direct_a64(const unsigned short* __restrict__ a, const unsigned sh
 #pragma unroll
       for (int r = 0; r < WJ; ++r) {
         __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-        if (i < 3) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+        if (i < kBFrom + WJ / 2) __builtin_amdgcn_sched_group_barrier(0x100, kReads, 0);
       }
       __builtin_amdgcn_sched_barrier(0);
       after_group(i);
@@ -992,17 +1010,17 @@ gemm_bf16_all_direct_a64(const unsigned short* __restrict__ a, const unsigned sh
   // Before the loop, in the order the loop's wait counts assume: (A transfer 0, B stage 0), then what K steps -2
   // and -1 would have issued: (B stage 1, first half of A transfer 1), (B stage 2, second half of A transfer 1).
 #pragma unroll
-  for (int r = 0; r < 8; ++r) issue_a(0, 0, r);
+  for (int r = 0; r < 2 * WI; ++r) issue_a(0, 0, r);
 #pragma unroll
-  for (int r = 0; r < 4; ++r) issue_b(0, 0, r);
+  for (int r = 0; r < WI; ++r) issue_b(0, 0, r);
 #pragma unroll
-  for (int r = 0; r < 4; ++r) issue_b(1, 1, r);
+  for (int r = 0; r < WI; ++r) issue_b(1, 1, r);
 #pragma unroll
-  for (int r = 0; r < 4; ++r) issue_a(1, 1, r);
+  for (int r = 0; r < WI; ++r) issue_a(1, 1, r);
 #pragma unroll
-  for (int r = 0; r < 4; ++r) issue_b(2, 2, r);
+  for (int r = 0; r < WI; ++r) issue_b(2, 2, r);
 #pragma unroll
-  for (int r = 4; r < 8; ++r) issue_a(1, 1, r);
+  for (int r = WI; r < 2 * WI; ++r) issue_a(1, 1, r);
   hipdma::wait_direct_loads<2 * kLoads>();
   __builtin_amdgcn_s_barrier();
   // first slice of K step 0
@@ -1035,9 +1053,9 @@ gemm_bf16_all_direct_a64(const unsigned short* __restrict__ a, const unsigned sh
     const int ab2 = ab1 == 2 ? 0 : ab1 + 1;   // transfer kt / 2 + 2, requested during K steps kt and kt + 1
     const int d = kt >> 1;
     k_step(kt, 0, ab0, 0, ab0, 2, d + 2, ab2, 0);
-    k_step(kt + 1, 1, ab0, 1, ab1, 0, d + 2, ab2, 4);
+    k_step(kt + 1, 1, ab0, 1, ab1, 0, d + 2, ab2, WI);
     k_step(kt + 2, 2, ab1, 0, ab1, 2, d + 3, ab0, 0);     // transfer kt / 2 + 3 takes the buffer transfer kt / 2 has left
-    k_step(kt + 3, 3, ab1, 1, ab2, 0, d + 3, ab0, 4);
+    k_step(kt + 3, 3, ab1, 1, ab2, 0, d + 3, ab0, WI);
     ab0 = ab2;
   }
   hipdma::wait_direct_loads<0>();
@@ -1068,6 +1086,12 @@ int launch_gemm(const uint16_t* d_a, const uint16_t* d_b, float* d_c, int m, int
   return CUDADMA_OK;
 }
 
+// Whether the rows of one round of direct-to-LDS loads (32 of A, 16 of B) span less than the 4 GiB of a lane offset.
+bool direct_rows_fit(const long long n, const long long k)
+{
+  return 32 * (k * 2) + 128 <= 0xffffffffLL && 16 * (n * 2) + 256 <= 0xffffffffLL;
+}
+
 }  // namespace
 
 extern "C" int cudadma_gemm_bf16(const uint16_t* d_a, const uint16_t* d_b, float* d_c, int m, int n, int k,
@@ -1086,23 +1110,29 @@ extern "C" int cudadma_gemm_bf16(const uint16_t* d_a, const uint16_t* d_b, float
   CUDADMA_REQUIRE((long long)k * 2 <= 0x7fffffffLL && (long long)n * 2 <= 0x7fffffffLL, "row pitch must fit an int");
   hipStream_t s = (hipStream_t)stream;
   if (variant == 0) {
-    // The tile whose rounds over the compute units cost least.  `full` is the time of a K step of 64 of a whole round in units of
-    // 10 ns, `part` that of a round of few workgroups: up to one per compute unit for the small tile, of which two share one, up to
-    // five eighths of them for the others (they get more of the clock and the memory); `once` is what a tile costs before its
-    // first and after its last K step.  Measured: 3072^3 61 us with 144 tiles of 256 x 256 against 96 with 256 x 128 and 79 with
-    // 128 x 128; 2048 x 3072 x 4096 77 / 63 / 72; 2048^3 41 / 35 / 25; 2816 x 2560 x 640 20 / 17.6 / 16.1.
+    // Variant 9 with its tile of 256 x 256 or the same kernel with 128 x 128, whichever takes its rounds over the compute units in less time.
+    // `full` is the time of a K step of 64 of a whole round in units of 10 ns, `part` that of a round of few workgroups: up to one per
+    // compute unit for the small tile, of which two share one, up to five eighths of them for the large one (they get more of the
+    // clock and the memory); `once` is what a tile costs before its first and after its last K step.  Measured, 256 / 128:
+    // 3072^3 62 / 72 us, 2304 x 5888 x 2304 58 / 65, 2048^3 41 / 23, 2560 x 2560 x 1024 25 / 18.  The tiles of variants 2 and 3
+    // lie between and win nowhere.  Both load with 32-bit lane offsets, a round of 32 rows of A or 16 of B at a time; longer rows
+    // go through variant 1.
     const long long cus = workloads::device_cus();
     auto rounds = [&](const long long tiles, const long long slots, const long long few, const int full, const int part, const int once) {
       const long long rest = tiles % slots;
       return (k / kBK) * (tiles / slots * full + (rest == 0 ? 0 : rest <= few ? part : full)) + once;
     };
-    const bool m256 = (m % 256) == 0, n256 = (n % 256) == 0;
-    long long least = rounds((long long)(m / 128) * (n / 128), 2 * cus, cus, 112, 60, 490);
-    variant = 1;
-    auto consider = [&](const bool fits, const int v, const long long cost) { if (fits && cost < least) { least = cost; variant = v; } };
-    consider(m256, 3, rounds((long long)(m / 256) * (n / 128), cus, cus * 5 / 8, 95, 85, 810));
-    consider(n256, 2, rounds((long long)(m / 128) * (n / 256), cus, cus * 5 / 8, 95, 85, 810));
-    consider(m256 && n256, 9, rounds((long long)(m / 256) * (n / 256), cus, cus * 5 / 8, 160, 110, 1000));
+    const long long small = rounds((long long)(m / 128) * (n / 128), 2 * cus, cus, 92, 58, 400);
+    const bool even = (m % 256) == 0 && (n % 256) == 0;
+    if (!direct_rows_fit(n, k)) variant = 1;
+    else if (even && rounds((long long)(m / 256) * (n / 256), cus, cus * 5 / 8, 160, 110, 1000) < small) variant = 9;
+    else {
+      const long long grid = (long long)(m / 128) * (n / 128);
+      CUDADMA_REQUIRE(grid <= 0x7fffffffLL, "grid too large");
+      hipLaunchKernelGGL(gemm_bf16_all_direct_a64<2>, dim3((unsigned)grid), dim3(256), 0, s, d_a, d_b, d_c, m, n, k);
+      CUDADMA_HIP_CHECK(hipGetLastError());
+      return CUDADMA_OK;
+    }
   }
   switch (variant) {
     case 1: return launch_gemm<2, 2>(d_a, d_b, d_c, m, n, k, s);
@@ -1116,7 +1146,7 @@ extern "C" int cudadma_gemm_bf16(const uint16_t* d_a, const uint16_t* d_b, float
       const long long grid = (long long)(m / 256) * (n / 256);
       CUDADMA_REQUIRE(grid <= 0x7fffffffLL, "grid too large");
       if (variant == 7) hipLaunchKernelGGL(gemm_bf16_ws_direct4_a64, dim3((unsigned)grid), dim3(512 + 2 * kDirect4DmaThreads), 0, s, d_a, d_b, d_c, m, n, k);
-      else if (variant == 9) hipLaunchKernelGGL(gemm_bf16_all_direct_a64, dim3((unsigned)grid), dim3(256), 0, s, d_a, d_b, d_c, m, n, k);
+      else if (variant == 9) hipLaunchKernelGGL(gemm_bf16_all_direct_a64<4>, dim3((unsigned)grid), dim3(256), 0, s, d_a, d_b, d_c, m, n, k);
 #ifdef HIPDMA_SWEEP_VARIANTS
       else if (variant == 6) hipLaunchKernelGGL(gemm_bf16_ws_direct4, dim3((unsigned)grid), dim3(512 + 2 * kDirect4DmaThreads), 0, s, d_a, d_b, d_c, m, n, k);
       else hipLaunchKernelGGL(gemm_bf16_all_direct, dim3((unsigned)grid), dim3(256), 0, s, d_a, d_b, d_c, m, n, k);

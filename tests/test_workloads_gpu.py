@@ -556,6 +556,20 @@ def test_gemm_full_size(device, variant):
     assert float((d_c - ref).abs().max()) <= 1e-2 * 64.0
 
 
+# tile grids that divide into eight blocks and that do not (fewer tiles than XCDs, bands of tile rows with a remainder), both tiles of
+# the default variant, one and several rounds
+@pytest.mark.parametrize("shape", [(128, 128, 128), (128, 896, 256), (384, 1152, 128), (1152, 1408, 384), (2944, 2432, 128), (2816, 2816, 256),
+                                   (3072, 3072, 128), (3328, 3840, 128)])
+@pytest.mark.parametrize("variant", [0, 1])
+def test_gemm_tile_walks(device, shape, variant):
+    m, n, k = shape
+    a = wl.fill_normal_bf16(torch.empty((m, k), dtype=torch.bfloat16, device=device), 61)
+    b = wl.fill_normal_bf16(torch.empty((k, n), dtype=torch.bfloat16, device=device), 62)
+    got = wl.gemm_bf16(a, b, torch.full((m, n), float("nan"), device=device), variant)
+    want, size = a.double() @ b.double(), a.double().abs() @ b.double().abs()
+    assert bool(((got - want).abs() <= k * 2.0 ** -23 * size).all())      # k additions of 2^-24 each, the products exact in fp32, doubled
+
+
 def test_gemm_rejects_ragged_shapes(device):
     a = torch.zeros((100, 128), dtype=torch.bfloat16, device=device)
     b = torch.zeros((128, 128), dtype=torch.bfloat16, device=device)
