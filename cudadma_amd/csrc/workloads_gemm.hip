@@ -1114,7 +1114,7 @@ extern "C" int cudadma_gemm_bf16(const uint16_t* d_a, const uint16_t* d_b, float
     // `full` is the time of a K step of 64 of a whole round in units of 10 ns, `part` that of a round of few workgroups: up to one per
     // compute unit for the small tile, of which two share one, up to five eighths of them for the large one (they get more of the
     // clock and the memory); `once` is what a tile costs before its first and after its last K step.  Measured, 256 / 128:
-    // 3072^3 62 / 72 us, 2304 x 5888 x 2304 58 / 65, 2048^3 41 / 23, 2560 x 2560 x 1024 25 / 18.  The tiles of variants 2 and 3
+    // 1536 x 7680 x 1280 38 / 44 us, 2816 x 5888 x 1024 39 / 42, 7424 x 2304 x 2048 99 / 81, 2048^3 41 / 23, 2560 x 2560 x 1024 25 / 18.  The tiles of variants 2 and 3
     // lie between and win nowhere.  Both load with 32-bit lane offsets, a round of 32 rows of A or 16 of B at a time; longer rows
     // go through variant 1.
     const long long cus = workloads::device_cus();
@@ -1122,7 +1122,7 @@ extern "C" int cudadma_gemm_bf16(const uint16_t* d_a, const uint16_t* d_b, float
       const long long rest = tiles % slots;
       return (k / kBK) * (tiles / slots * full + (rest == 0 ? 0 : rest <= few ? part : full)) + once;
     };
-    const long long small = rounds((long long)(m / 128) * (n / 128), 2 * cus, cus, 92, 58, 400);
+    const long long small = rounds((long long)(m / 128) * (n / 128), 2 * cus, cus, 100, 58, 400);
     const bool even = (m % 256) == 0 && (n % 256) == 0;
     if (!direct_rows_fit(n, k)) variant = 1;
     else if (even && rounds((long long)(m / 256) * (n / 256), cus, cus * 5 / 8, 160, 110, 1000) < small) variant = 9;
