@@ -59,19 +59,20 @@ int replay_grid(const cudadma_plan_query_t& q, MapWriter& w, int* steps)
     hipdma::detail::GridCursor c = g.begin();
     for (int r = 0; r < g.steps * max_lds; ++r) {
       if (g.live(r, c)) {
+        using hipdma::detail::row_offset;
         if (c.row < 0 || c.row >= q.num_elmts || c.col < 0 || c.col >= g.LPE) return CUDADMA_ERANGE;
         long long so, dd;
         if (gather) {
           const int dense = q.dst_stride > e ? q.dst_stride : e;
           so = (long long)q.index[c.row] * e + c.col * a;
-          dd = (long long)c.row * dense + c.col * a;
+          dd = row_offset(c.row, dense) + c.col * a;
         } else if (scatter) {
           const int dense = q.src_stride > e ? q.src_stride : e;
-          so = (long long)c.row * dense + c.col * a;
+          so = row_offset(c.row, dense) + c.col * a;
           dd = (long long)q.index[c.row] * e + c.col * a;
         } else {
-          so = (long long)c.row * q.src_stride + c.col * a;
-          dd = (long long)c.row * q.dst_stride + c.col * a;
+          so = row_offset(c.row, q.src_stride) + c.col * a;
+          dd = row_offset(c.row, q.dst_stride) + c.col * a;
         }
         w.move(so, dd, g.chunk_bytes(a, c));
       }

@@ -49,6 +49,12 @@ struct GridPlan {
 
 namespace detail {
 
+// Byte offset of row `row` in a buffer whose rows lie `stride` bytes apart.  The product is formed in 64 bits: `stride` is an int,
+// but the rows of one transfer may span more than 2 GiB (256 columns of a column-major matrix with a leading dimension of
+// 2.2 M floats).
+__host__ __device__ constexpr long long row_offset(int row, int stride) { return (long long)row * stride; }
+static_assert(row_offset(255, 8800256) == 2244065280LL, "a product in 32 bits is no constant expression here");
+
 // Per-thread cursor over the slots of a GridPlan.
 struct GridCursor {
   int row, col;

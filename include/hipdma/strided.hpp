@@ -258,10 +258,10 @@ private:
       // part per thread that never changes (its row and column of round 0).  Written that way the thread keeps
       // one offset instead of a 64-bit address per load in flight, and the per-load part is scalar arithmetic.
       if (m_grid.dcol == 0) {
-        const long long lane_part = (long long)(m_grid.row0 * m_src_stride + m_grid.col0 * ALIGNMENT);
+        const long long lane_part = row_offset(m_grid.row0, m_src_stride) + m_grid.col0 * ALIGNMENT;
         // the same value in every lane (object parameters are); saying so keeps it in scalar registers
         auto rows_down = [&](const int round) __attribute__((always_inline)) {
-          const unsigned long long bytes = (unsigned long long)((long long)(round * m_grid.drow) * (long long)m_src_stride);
+          const unsigned long long bytes = (unsigned long long)row_offset(round * m_grid.drow, m_src_stride);
           return (long long)(((unsigned long long)scalar_u32((unsigned)(bytes >> 32)) << 32) | (unsigned long long)scalar_u32((unsigned)bytes));
         };
         if (padded_rows()) {
@@ -295,7 +295,7 @@ private:
     for (int k = 0; k < MAX_LDS; ++k) {
       if (m_grid.live(step * MAX_LDS + k, cur))
         load_chunk<ALIGNMENT, ALIGNMENT, GLOBAL_LOAD, LOAD_QUAL>(
-            m_buf[k], m_src + cur.row * m_src_stride + cur.col * ALIGNMENT, m_grid.chunk_bytes(ALIGNMENT, cur));
+            m_buf[k], m_src + row_offset(cur.row, m_src_stride) + cur.col * ALIGNMENT, m_grid.chunk_bytes(ALIGNMENT, cur));
       m_grid.advance(cur);
     }
   }
@@ -313,7 +313,7 @@ private:
         for (int k = 0; k < MAX_LDS; ++k) {
           if (step * MAX_LDS + k < m_grid.whole_rounds || cur.row < m_grid.N)
             store_chunk<ALIGNMENT, ALIGNMENT, STORE_QUAL>(
-                m_buf[k], dst + cur.row * m_dst_stride + lds_col<store_is_swizzled(STORE_QUAL)>(cur) * ALIGNMENT, bytes);
+                m_buf[k], dst + dst_row<STORE_QUAL>(cur.row) + lds_col<store_is_swizzled(STORE_QUAL)>(cur) * ALIGNMENT, bytes);
           cur.row += m_grid.drow;
         }
       } else {
@@ -325,10 +325,18 @@ private:
     for (int k = 0; k < MAX_LDS; ++k) {
       if (m_grid.live(step * MAX_LDS + k, cur))
         store_chunk<ALIGNMENT, ALIGNMENT, STORE_QUAL>(
-            m_buf[k], dst + cur.row * m_dst_stride + lds_col<store_is_swizzled(STORE_QUAL)>(cur) * ALIGNMENT,
+            m_buf[k], dst + dst_row<STORE_QUAL>(cur.row) + lds_col<store_is_swizzled(STORE_QUAL)>(cur) * ALIGNMENT,
             m_grid.chunk_bytes(ALIGNMENT, cur));
       m_grid.advance(cur);
     }
+  }
+
+  // Byte offset of destination row `row`; 32 bits do for a destination that is known to be LDS.
+  template<int STORE_QUAL>
+  __device__ __forceinline__ long long dst_row(const int row) const
+  {
+    if constexpr (hipdma::detail::store_is_lds(STORE_QUAL)) return row * m_dst_stride;
+    else return hipdma::detail::row_offset(row, m_dst_stride);
   }
 
   // Chunk position inside the LDS row for the chunk at cursor c.
@@ -363,7 +371,7 @@ private:
         ((long long)m_grid.drow * (long long)m_src_stride + (long long)m_grid.W * ALIGNMENT <= 0xffffffffLL);
     if constexpr (WHOLE_ROWS) HIPDMA_ASSERT(whole_rows);
     if (WHOLE_ROWS || whole_rows) {
-      const unsigned lane_row = (unsigned)(m_grid.row0 * m_src_stride);
+      const unsigned lane_row = (unsigned)m_grid.row0 * (unsigned)m_src_stride;     // below 4 GiB, see above
       // The pointers, strides and rows per round are the same in every lane by the contract of the call;
       // the compiler cannot always tell, so they are pinned to scalar registers once per transfer.
       const char* const base = scalar_ptr(m_src);
@@ -388,7 +396,7 @@ private:
       if (r >= first && r < end && m_grid.live(r, cur)) {
         const int lds_off = cur.row * m_dst_stride + cur.col * ALIGNMENT;
         if constexpr (ALIGNMENT == 16 || ALIGNMENT == 4)
-          load_to_lds<ALIGNMENT, LOAD_QUAL>(m_src + cur.row * m_src_stride + lds_col<SWIZZLE>(cur) * ALIGNMENT,
+          load_to_lds<ALIGNMENT, LOAD_QUAL>(m_src + row_offset(cur.row, m_src_stride) + lds_col<SWIZZLE>(cur) * ALIGNMENT,
                                  dst + (lds_off - lane * ALIGNMENT));
       }
       m_grid.advance(cur);

@@ -107,6 +107,25 @@ def test_sgemv_panels(dev, n, m):
     assert np.all(got[n:] == 3.0)
 
 
+# a leading dimension far beyond what n needs: the columns of one panel lie more than 2 GiB apart (256, 128 and 32 columns)
+@pytest.mark.parametrize("n,m,lda,variant", [(16, 256, 2_200_064, 3), (4160, 288, 2_200_064, 3), (8200, 288, 4_300_032, 3), (40, 32, 17_400_064, 3),
+                                             (40, 32, 17_400_064, 2), (40, 256, 17_400_064, 3)])
+def test_sgemv_columns_far_apart(dev, n, m, lda, variant):
+    O = ol.load()
+    pad = (n + 127) // 128 * 128
+    a = ol.uniform(m * pad, 25).reshape(m, pad)
+    x = ol.uniform(m, 26)
+    want = np.empty(n, dtype=np.float32)
+    O.oracle_sgemv(n, m, 1.5, ptr(a), pad, ptr(x), ptr(want))
+    da = torch.empty((m, lda), dtype=torch.float32, device=dev)        # only the rows that are read are filled
+    da[:, :pad] = torch.from_numpy(a).to(dev)
+    dy = torch.full((pad,), 3.0, dtype=torch.float32, device=dev)
+    ex.sgemv(1.5, da, torch.from_numpy(x).to(dev), dy, n=n, variant=variant)
+    torch.cuda.synchronize()
+    got = dy.cpu().numpy()
+    assert np.array_equal(got[:n], want) and np.all(got[n:] == 3.0)
+
+
 def test_sgemv_argument_checks(dev):
     a = torch.zeros((96, 128), dtype=torch.float32, device=dev)
     x = torch.zeros(96, dtype=torch.float32, device=dev)

@@ -349,6 +349,17 @@ def test_plan_extents_are_the_footprint_of_the_closed_form():
         assert (src_origin + ext[0], src_origin + ext[1]) == (src_bytes.min(), src_bytes.max() + 1), case
 
 
+@pytest.mark.parametrize("lda", [2_105_376, 2_105_380, 4_227_332, 17_318_420, (1 << 29) - 4])
+@pytest.mark.parametrize("rows,cols,threads", [(16, 256, 128), (32, 256, 128), (64, 128, 256), (128, 32, 128)])
+def test_row_offsets_beyond_two_gib(lda, rows, cols, threads):
+    """The panels of the sgemv example (`cols` columns of `rows` floats, a column every `lda` floats) with leading dimensions around
+    the ones at which the last column lies 2 GiB away, up to the largest whose bytes fit an int; once as source and once as destination."""
+    for src, dst in ((4 * lda, 4 * rows), (4 * rows, 4 * lda)):
+        ext = cd.plan.plan_extents(cd.PATTERN_STRIDED, alignment=16, bytes_per_thread=4 * rows * cols // threads, bytes_per_elmt=4 * rows,
+                                   dma_threads=threads, num_elmts=cols, src_stride=src, dst_stride=dst)
+        assert tuple(ext) == (0, (cols - 1) * src + 4 * rows, 0, (cols - 1) * dst + 4 * rows)
+
+
 def test_the_top_level_holds_only_what_belongs_there():
     """A stray file at the repository root (a shell redirect gone wrong, a result left behind) travels to every GPU run and
     into history: the tracked top-level entries are the ones named here and the records the round driver writes."""
