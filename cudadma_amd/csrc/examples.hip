@@ -44,15 +44,17 @@ void launch_sgemv_panels(hipStream_t s, int n, int m, float alpha, const float* 
 // The narrowest row tile that gives no compute unit a second workgroup: a row is one chain of multiply-adds whatever the tile, so
 // more and narrower workgroups share the bytes (4096 x 4096: 30 / 31 / 36 / 59 us with tiles of 16 / 32 / 64 / 128 rows); beyond one
 // workgroup per compute unit the memory counts, and with it the length of the pieces of a column (8192 x 8192: 100 / 60 / 70 us with
-// 16 / 32 / 64 rows, 16384 x 16384: 344 / 206 / 170).  A panel needs m >= its columns; what is shorter, and strides at which
-// the 31 rows a DMA thread may lie into a column group overflow 32 bits, go through the panel of 32 columns.
+// 16 / 32 / 64 rows, 16384 x 16384: 344 / 206 / 170).  The last panel moves back to end with the last column, so a matrix needs at
+// least the columns of one panel; narrower ones go through the panel of 32 columns.
 void launch_sgemv_double(hipStream_t s, int n, int m, float alpha, const float* a, int lda, const float* x, float* y)
 {
+  constexpr int kWide = 256, kTall = 128;
+  static_assert(kTall <= kWide, "the line below holds for both panels");
   const int cus = workloads::device_cus();
-  if (m < 256 || lda > (1 << 24)) launch_sgemv_panels<kGemvCompute, kGemvPanelCols, kGemvDmaPerLd, kGemvMatLds * kGemvDmaPerLd>(s, n, m, alpha, a, lda, x, y);
-  else if ((n + 15) / 16 <= cus) launch_sgemv_panels<16, 256, 64, 128>(s, n, m, alpha, a, lda, x, y);
-  else if ((n + 31) / 32 <= cus) launch_sgemv_panels<32, 256, 64, 128>(s, n, m, alpha, a, lda, x, y);
-  else launch_sgemv_panels<64, 128, 64, 256>(s, n, m, alpha, a, lda, x, y);
+  if (m < kWide) launch_sgemv_panels<kGemvCompute, kGemvPanelCols, kGemvDmaPerLd, kGemvMatLds * kGemvDmaPerLd>(s, n, m, alpha, a, lda, x, y);
+  else if ((n + 15) / 16 <= cus) launch_sgemv_panels<16, kWide, 64, 128>(s, n, m, alpha, a, lda, x, y);
+  else if ((n + 31) / 32 <= cus) launch_sgemv_panels<32, kWide, 64, 128>(s, n, m, alpha, a, lda, x, y);
+  else launch_sgemv_panels<64, kTall, 64, 256>(s, n, m, alpha, a, lda, x, y);
 }
 
 // ---- 2-D stencil ----
@@ -176,6 +178,8 @@ extern "C" int cudadma_example_sgemv(int variant, int n, int m, float alpha, con
   if (n == 0) return CUDADMA_OK;
   CUDADMA_REQUIRE(d_a != nullptr && d_x != nullptr && d_y != nullptr, "NULL pointer");
   CUDADMA_REQUIRE(cudadma_host::aligned_to(d_x, 16), "x must be 16-byte aligned");
+  // the objects that stage the matrix take the distance of two columns as an int
+  CUDADMA_REQUIRE(variant < 2 || lda <= 0x7fffffff / 4, "lda (%d) must not exceed %d when the matrix is staged", lda, 0x7fffffff / 4);
   const int grid = (n + kGemvCompute - 1) / kGemvCompute;
   const int cols = variant == 0 ? kGemvVecElmts : variant == 1 ? 2 * kGemvVecElmts : kGemvPanelCols;
   CUDADMA_REQUIRE(m > 0 && (m % cols) == 0, "m (%d) must be a positive multiple of %d for this variant", m, cols);

@@ -8,9 +8,10 @@
 // 0.0f, y[row] = alpha * res.  Written against the first-generation class names
 // (cudaDMASequential, cudaDMAStrided of include/cudaDMA.h).
 //
-// All kernels need m to be a multiple of the columns staged per hand-off and
-// lda*4 to be a multiple of 16 B when the matrix is staged; rows beyond n are
-// neither read from global memory by compute threads nor written.
+// The kernels need m to be a multiple of the columns staged per hand-off, except
+// sgemvn_both_double, which takes multiples of 32 from the columns of one panel on.
+// Where the matrix is staged, lda*4 has to be a multiple of 16 B and fit an int.
+// Rows beyond n are neither read from global memory by compute threads nor written.
 #pragma once
 
 #include "../../../include/cudaDMA.h"
@@ -212,6 +213,7 @@ void sgemvn_both_double(int n, int m, float alpha, const float* __restrict__ A, 
   __shared__ __attribute__((aligned(16))) float mat0[COLS * ROWS];
   __shared__ __attribute__((aligned(16))) float mat1[COLS * ROWS];
 
+  HIPDMA_ASSERT(m >= COLS && (m % 32) == 0);      // a shorter matrix would have the panel begin before its first column
   // a thread holds its share of a panel in registers: the next panel is on its way while this one is read
   constexpr int kMatBytes = 4 * ROWS * COLS / MAT_DMA_THREADS;
   typedef cudaDMASequential<true, 16, 4 * COLS, VEC_DMA_THREADS> vec_dma_t;

@@ -311,8 +311,8 @@ int cudadma_example_saxpy(int variant, float a, const float* d_x, float* d_y, lo
 /* y = alpha * A x, A column-major n x m with leading dimension lda, accumulated in
  * ascending column order with fused multiply-add (src/examples/sgemv/sgemv_dma.cu:140-175,
  * :262-325, :329-388, :392-470; host check :752-771).  m a multiple of 256 (variant 0),
- * 512 (variant 1) or 32 (variants 2, 3, which also need lda >= n rounded up to 128 and
- * 16-byte aligned columns). */
+ * 512 (variant 1) or 32 (variants 2, 3, which also need lda >= n rounded up to 128,
+ * lda * 4 within an int and 16-byte aligned columns). */
 int cudadma_example_sgemv(int variant, int n, int m, float alpha, const float* d_a, int lda, const float* d_x,
                           float* d_y, void* stream);
 

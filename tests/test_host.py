@@ -360,6 +360,15 @@ def test_row_offsets_beyond_two_gib(lda, rows, cols, threads):
         assert tuple(ext) == (0, (cols - 1) * src + 4 * rows, 0, (cols - 1) * dst + 4 * rows)
 
 
+@pytest.mark.parametrize("variant", [2, 3])
+@pytest.mark.parametrize("lda", [1 << 29, 1 << 30, 0x7ffffffc])
+def test_sgemv_refuses_columns_whose_distance_is_no_int(variant, lda):
+    """Pointers that are never dereferenced: the refusal comes before anything touches a device."""
+    at = ctypes.c_void_p(4096)
+    with pytest.raises(cd.CudaDMAError, match="must not exceed 536870911 when the matrix is staged"):
+        cd._lib.check(cd.lib().cudadma_example_sgemv(variant, 16, 256, 1.0, at, lda, at, at, None))
+
+
 def test_the_top_level_holds_only_what_belongs_there():
     """A stray file at the repository root (a shell redirect gone wrong, a result left behind) travels to every GPU run and
     into history: the tracked top-level entries are the ones named here and the records the round driver writes."""
