@@ -1116,7 +1116,7 @@ extern "C" int cudadma_gemm_bf16(const uint16_t* d_a, const uint16_t* d_b, float
     // clock and the memory); `once` is what a tile costs before its first and after its last K step.  Measured, 256 / 128:
     // 1536 x 7680 x 1280 38 / 44 us, 2816 x 5888 x 1024 39 / 42, 7424 x 2304 x 2048 99 / 81, 2048^3 41 / 23, 2560 x 2560 x 1024 25 / 18.  The tiles of variants 2 and 3
     // lie between and win nowhere.  Both load with 32-bit lane offsets, a round of 32 rows of A or 16 of B at a time; longer rows
-    // go through variant 1.
+    // go through variant 1, whose transfers take a 64-bit offset for every row.
     const long long cus = workloads::device_cus();
     auto rounds = [&](const long long tiles, const long long slots, const long long few, const int full, const int part, const int once) {
       const long long rest = tiles % slots;
@@ -1143,6 +1143,8 @@ extern "C" int cudadma_gemm_bf16(const uint16_t* d_a, const uint16_t* d_b, float
 #endif
     case 6: case 7: case 8: case 9: {
       CUDADMA_REQUIRE((m % 256) == 0 && (n % 256) == 0, "this variant needs m and n multiples of 256 (got %d x %d)", m, n);
+      // 6 and 7 go over to 64-bit row offsets by themselves (issue_direct), 8 and 9 are compiled for lane offsets alone
+      CUDADMA_REQUIRE(variant <= 7 || direct_rows_fit(n, k), "rows of %d x %d are too long for the lane offsets of this variant (0, 1 and 7 take them)", k, n);
       const long long grid = (long long)(m / 256) * (n / 256);
       CUDADMA_REQUIRE(grid <= 0x7fffffffLL, "grid too large");
       if (variant == 7) hipLaunchKernelGGL(gemm_bf16_ws_direct4_a64, dim3((unsigned)grid), dim3(512 + 2 * kDirect4DmaThreads), 0, s, d_a, d_b, d_c, m, n, k);

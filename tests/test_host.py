@@ -369,6 +369,14 @@ def test_sgemv_refuses_columns_whose_distance_is_no_int(variant, lda):
         cd._lib.check(cd.lib().cudadma_example_sgemv(variant, 16, 256, 1.0, at, lda, at, at, None))
 
 
+@pytest.mark.parametrize("n, k", [(256, 1 << 27), (1 << 28, 128)])
+def test_gemm_refuses_rows_beyond_its_lane_offsets(n, k):
+    """Variant 9 addresses 32 rows of A and 16 of B with 32-bit offsets: longer rows end before anything touches a device."""
+    at = ctypes.c_void_p(4096)
+    with pytest.raises(cd.CudaDMAError, match="too long for the lane offsets"):
+        cd._lib.check(cd.lib().cudadma_gemm_bf16(at, at, at, 256, n, k, 9, None))
+
+
 def test_the_top_level_holds_only_what_belongs_there():
     """A stray file at the repository root (a shell redirect gone wrong, a result left behind) travels to every GPU run and
     into history: the tracked top-level entries are the ones named here and the records the round driver writes."""

@@ -570,6 +570,22 @@ def test_gemm_tile_walks(device, shape, variant):
     assert bool(((got - want).abs() <= k * 2.0 ** -23 * size).all())      # k additions of 2^-24 each, the products exact in fp32, doubled
 
 
+def test_gemm_long_rows(device):
+    """Rows of A so long that those of one transfer lie more than 2 GiB apart, where the default variant leaves its 32-bit lane offsets;
+    a few columns hold small whole numbers, so the product is exact."""
+    mn, k = 128, 71_600_128
+    g = torch.Generator().manual_seed(71)
+    at = torch.tensor([0, 31, 64, k // 2 + 5, k - 129, k - 1], device=device)
+    some = torch.randint(-4, 5, (mn, at.numel()), generator=g).to(device, torch.bfloat16)
+    other = torch.randint(-4, 5, (at.numel(), mn), generator=g).to(device, torch.bfloat16)
+    a = torch.zeros((mn, k), dtype=torch.bfloat16, device=device)
+    b = torch.zeros((k, mn), dtype=torch.bfloat16, device=device)
+    a[:, at] = some
+    b[at] = other
+    got = wl.gemm_bf16(a, b, torch.full((mn, mn), float("nan"), device=device))
+    assert torch.equal(got, some.float() @ other.float())
+
+
 def test_gemm_rejects_ragged_shapes(device):
     a = torch.zeros((100, 128), dtype=torch.bfloat16, device=device)
     b = torch.zeros((128, 128), dtype=torch.bfloat16, device=device)
