@@ -616,28 +616,35 @@ constexpr int kWideTileVariants = 6;
 
 // How many planes a workgroup takes.  Every workgroup pays for about twelve planes before its first output (2 * radius planes of
 // the column plus the wait for them), whatever it then marches through.  A second workgroup on a compute unit slows both by 1.4
-// where the caches hold the grids from one sweep to the next and up to twice where they come from DRAM (512 x 512 x 64, 256 / 512
-// workgroups: 28.4 / 22.8 us, 512 x 512 x 256: 102 / 117; 384 x 320 x 200, 240 / 480: 41.5 / 31.3 from the caches, 43.6 / 53.5 from
-// DRAM); a third waits for its turn.  Of the numbers of chunks that just fill the compute units k times, the one with the least sum
-// of these is taken (192 x 256 x 130: 15.6 us with 288 workgroups of 22 planes, 13.2 with 480 of 13; 128^3: 9.4 -> 6.6;
-// 224 x 416 x 300, 273 / 455: 69 / 35 from the caches, 84 / 61 from DRAM).
+// where the caches hold the grids from one sweep to the next and up to twice where they come from DRAM; a third waits for its turn.
+// Of the numbers of chunks that just fill the compute units once, twice or three times, the one with the least sum of these is taken
+// (four were never the best).  Measured (us, resident / from DRAM, by workgroups; the first is one chunk per ceil(compute units / tiles)):
+//   192 x 256 x 130  288: 16.4 / 23.5  480: 13.4 / 19.8  240: 14.6 / 16.4      480 x 384 x 142  360: 41 / 65  720: 41 / 56  180: 54 / 56
+//   128^3            128:  9.9 / 10.8  256:  7.0 /  8.8                        384 x 320 x 200  360: 40 / 63  480: 36 / 53  240: 42 / 44
+//   256^3            256: 30.3 / 33.8  512: 25.2 / 37.8                        512 x 512 x 64   256: 29 / 31  512: 26 / 38
+// A shape is taken where it is faster both ways.  Where the chunks that it takes to occupy every compute unit, of 16 planes or more,
+// still make one workgroup each (the last pair), a second one gains 10 to 17 % from the caches and loses 12 to 24 from DRAM: it is
+// charged at the DRAM price there, as it is beyond what stays resident (448 x 512, 224 / 448 workgroups: 460 MiB 97 / 80 us, 500 MiB 112 / 125).
 constexpr int kLeastZchunk = 4;
 static int best_zchunk(const long long tiles_xy, const long long bytes, const int nz, const bool dwordx4)
 {
   const long long cus = workloads::device_cus();
-  // tenths of the time with one; the sweep kernels always want two
-  const long long two = bytes <= (128LL << 20) || !dwordx4 ? 14 : bytes <= (256LL << 20) ? 18 : 20;
   const long long most = nz / kLeastZchunk > 1 ? nz / kLeastZchunk : 1;
+  const long long cut = (cus + tiles_xy - 1) / tiles_xy, planes = (nz + cut - 1) / cut < 16 ? 16 : (nz + cut - 1) / cut;
+  const bool one_fills = tiles_xy * ((nz + planes - 1) / planes) <= cus;
+  // tenths of the time with one; the sweep kernels always want two
+  const long long two = dwordx4 && (one_fills || bytes > (480LL << 20)) ? 20 : 14;
   int best = nz;
   long long least = -1;
-  for (int k = 0; k <= 8; ++k) {
+  for (int k = 0; k <= 3; ++k) {
     long long chunks = k == 0 ? 1 : k * cus / tiles_xy;
     if (chunks < 1) continue;
     if (chunks > most) chunks = most;
     const int zchunk = (int)((nz + chunks - 1) / chunks);
     const long long grid = tiles_xy * ((nz + zchunk - 1) / zchunk);
     const long long rest = grid % (2 * cus);
-    const long long cost = (12 + zchunk) * (grid / (2 * cus) * two + (rest == 0 ? 0 : rest <= cus ? 10 : two));
+    const long long last = rest == 0 ? 0 : rest > cus ? two : grid <= cus ? 10 : 12;     // a third shares the caches with what is left of the two
+    const long long cost = (12 + zchunk) * (grid / (2 * cus) * two + last);
     if (least < 0 || cost < least) { least = cost; best = zchunk; }
   }
   return best;
