@@ -778,12 +778,14 @@ extern "C" int cudadma_strided_transpose(const float* d_in, float* d_out, int n,
   const int tiles = tiles_per_side * tiles_per_side;
   // Variant 0 is the library's choice.  Variant 10's shape, one 16 KB tile in flight per compute unit and streaming loads and stores,
   // is for matrices from DRAM (16384: 358 us against 456 with variant 11, 4096: 26.2 / 29.8).  Small matrices come from the
-  // Infinity Cache or leave their result there, and its short queue only costs (2112: 9.5 us against 6.8 with variant 11 from the
-  // cache, 9.9 / 8.9 from DRAM; 2816, the last below the line: 14 / 10.6 and 14.1 / 15.2).  Up to two tiles per compute unit
-  // the tile is best moved by every wavefront, with no hand-off (variant 4; 512: 4.0 us against 3.1, 1280: 5.4 / 4.3).
+  // Infinity Cache or leave their result there, and its short queue only costs (2112: 9.6 us against 6.8 with variant 11 from the
+  // cache, 10.2 / 8.9 from DRAM; 2496, the last below the line: 11.7 / 9.0 and 11.9 / 11.9).  Beyond it variant 11 still gains
+  // a quarter from the cache, but loses from DRAM (2560: 12.7 / 13.1, 2816: 14.5 / 16.1): the line lies where neither loses.  Up to
+  // two tiles per compute unit the tile is best moved by every wavefront, with no hand-off (variant 4; 512: 3.7 us against 2.7
+  // from DRAM, 1280: 5.6 / 4.4 and 5.6 / 5.4).
   if (variant == 0 && workloads::tuning("transpose_workgroups", 0) == 0) {
     if (tiles <= 2 * workloads::device_cus()) variant = 4;
-    else if (8LL * n * n <= (64LL << 20)) variant = 11;
+    else if (8LL * n * n <= (48LL << 20)) variant = 11;
   }
   // The kernels with one LDS tile (variants 1 and 4) run best with exactly one workgroup per compute unit, i.e. one
   // 16 KB tile of loads in flight per compute unit, and with the tiles walked down the columns (the workgroups that

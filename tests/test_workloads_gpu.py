@@ -403,7 +403,7 @@ def test_halo_stencil_chunks(device, shape):
 
 
 # the lines at which the default variants change kernels: one tile on either side
-@pytest.mark.parametrize("n", [1408, 1472, 2880, 2944])
+@pytest.mark.parametrize("n", [1408, 1472, 2496, 2560, 2880, 2944])
 def test_default_transpose_around_its_lines(device, n):
     src = wl.fill_uniform(torch.empty(n * n, dtype=torch.float32, device=device), 41).view(n, n)
     dst = torch.full_like(src, float("nan"))
