@@ -34,10 +34,10 @@ const char* const kGemvNames[] = {
   "vector by cudaDMASequential + panel of 32 to 256 columns by CudaDMAStrided, two buffers each",
 };
 
-template<int ROWS, int COLS, int VEC_DMA, int MAT_DMA>
+template<int ROWS, int COLS, int VEC_DMA, int MAT_DMA, int MAT_BYTES = 4 * ROWS * COLS / MAT_DMA>
 void launch_sgemv_panels(hipStream_t s, int n, int m, float alpha, const float* a, int lda, const float* x, float* y)
 {
-  hipLaunchKernelGGL((sgemvn_both_double<ROWS, COLS, VEC_DMA, MAT_DMA>), dim3((n + ROWS - 1) / ROWS),
+  hipLaunchKernelGGL((sgemvn_both_double<ROWS, COLS, VEC_DMA, MAT_DMA, MAT_BYTES>), dim3((n + ROWS - 1) / ROWS),
                      dim3((sgemv_both_double_threads<ROWS, VEC_DMA, MAT_DMA>())), 0, s, n, m, alpha, a, lda, x, y);
 }
 
@@ -45,15 +45,20 @@ void launch_sgemv_panels(hipStream_t s, int n, int m, float alpha, const float* 
 // more and narrower workgroups share the bytes (4096 x 4096: 30 / 31 / 36 / 59 us with tiles of 16 / 32 / 64 / 128 rows); beyond one
 // workgroup per compute unit the memory counts, and with it the length of the pieces of a column (8192 x 8192: 100 / 60 / 70 us with
 // 16 / 32 / 64 rows, 16384 x 16384: 344 / 206 / 170).  The last panel moves back to end with the last column, so a matrix needs at
-// least the columns of one panel; narrower ones go through the panel of 32 columns.
+// least the columns of one panel; narrower ones go through panels of 32 columns (16384 x 224: 5.1 us with 64 rows, 5.7 with 128).  So
+// do those with more rows than one tile of 64 per compute unit: several workgroups then share a compute unit and hide each
+// other's hand-offs, and small panels leave room for them (panels of 128 / 32 columns: 20480 x 4096 78 / 63 us, 28672 x 4096 91 / 78).
+// From about two such tiles per compute unit on, the longer pieces of 128 rows count again, in bursts of 64 bytes a thread (64 / 128
+// rows: 32768 x 2048 42 / 39 us, 98304 x 1024 76 / 72).
 void launch_sgemv_double(hipStream_t s, int n, int m, float alpha, const float* a, int lda, const float* x, float* y)
 {
   constexpr int kWide = 256, kTall = 128;
   static_assert(kTall <= kWide, "the line below holds for both panels");
   const int cus = workloads::device_cus();
-  if (m < kWide) launch_sgemv_panels<kGemvCompute, kGemvPanelCols, kGemvDmaPerLd, kGemvMatLds * kGemvDmaPerLd>(s, n, m, alpha, a, lda, x, y);
-  else if ((n + 15) / 16 <= cus) launch_sgemv_panels<16, kWide, 64, 128>(s, n, m, alpha, a, lda, x, y);
-  else if ((n + 31) / 32 <= cus) launch_sgemv_panels<32, kWide, 64, 128>(s, n, m, alpha, a, lda, x, y);
+  if (n > 112 * cus) launch_sgemv_panels<kGemvCompute, kGemvPanelCols, kGemvDmaPerLd, kGemvMatLds * kGemvDmaPerLd, 64>(s, n, m, alpha, a, lda, x, y);
+  else if (m < kWide || n > 64 * cus) launch_sgemv_panels<64, kGemvPanelCols, 64, 64>(s, n, m, alpha, a, lda, x, y);
+  else if (n <= 16 * cus) launch_sgemv_panels<16, kWide, 64, 128>(s, n, m, alpha, a, lda, x, y);
+  else if (n <= 32 * cus) launch_sgemv_panels<32, kWide, 64, 128>(s, n, m, alpha, a, lda, x, y);
   else launch_sgemv_panels<64, kTall, 64, 256>(s, n, m, alpha, a, lda, x, y);
 }
 

@@ -187,6 +187,12 @@ struct SgemvBlock {
 template<int ROWS, int COLS>
 __device__ __forceinline__ float sgemv_panel(const float* mat, const float* vec, const int row, const int first, float res)
 {
+  if constexpr (COLS == 32) {
+    // two blocks are over before a pipeline has filled: the compiler's own order is 5 % faster (16384 x 224: 5.4 -> 5.1 us)
+#pragma unroll
+    for (int j = 0; j < COLS; ++j) res = __builtin_fmaf(mat[j * ROWS + row], vec[j], res);
+    return res;
+  }
   SgemvBlock<ROWS> even, odd;
   even.load(mat, vec, row, first);
   for (int c = first; c < COLS; c += 32) {
@@ -202,7 +208,7 @@ __device__ __forceinline__ float sgemv_panel(const float* mat, const float* vec,
   return res;
 }
 
-template<int ROWS, int COLS, int VEC_DMA_THREADS, int MAT_DMA_THREADS>
+template<int ROWS, int COLS, int VEC_DMA_THREADS, int MAT_DMA_THREADS, int MAT_BYTES = 4 * ROWS * COLS / MAT_DMA_THREADS>
 __global__ __launch_bounds__((sgemv_both_double_threads<ROWS, VEC_DMA_THREADS, MAT_DMA_THREADS>()))
 void sgemvn_both_double(int n, int m, float alpha, const float* __restrict__ A, int lda, const float* __restrict__ x,
                         float* __restrict__ y)
@@ -214,10 +220,10 @@ void sgemvn_both_double(int n, int m, float alpha, const float* __restrict__ A, 
   __shared__ __attribute__((aligned(16))) float mat1[COLS * ROWS];
 
   HIPDMA_ASSERT(m >= COLS && (m % 32) == 0);      // a shorter matrix would have the panel begin before its first column
-  // a thread holds its share of a panel in registers: the next panel is on its way while this one is read
-  constexpr int kMatBytes = 4 * ROWS * COLS / MAT_DMA_THREADS;
+  // a thread holds its share of a panel in registers, all of it unless MAT_BYTES says less: the next panel is on its way while this
+  // one is read
   typedef cudaDMASequential<true, 16, 4 * COLS, VEC_DMA_THREADS> vec_dma_t;
-  typedef CudaDMAStrided<true, 16, kMatBytes, 4 * ROWS, MAT_DMA_THREADS, COLS> mat_dma_t;
+  typedef CudaDMAStrided<true, 16, MAT_BYTES, 4 * ROWS, MAT_DMA_THREADS, COLS> mat_dma_t;
   vec_dma_t dma_vec_0(1, kCompute, kCompute);
   vec_dma_t dma_vec_1(2, kCompute, kCompute + VEC_DMA_THREADS);
   mat_dma_t dma_mat_0(3, kCompute, kCompute + 2 * VEC_DMA_THREADS, 4 * lda, 4 * ROWS);

@@ -88,9 +88,9 @@ def test_sgemv_random(dev, variant, n, m, lda):
     assert np.all(got[n:] == 3.0)                          # rows beyond n are not written
 
 
-# the default variant's row tiles (16, 32 and 64 rows by the number of workgroups) and panels: n around the lines between the tiles, m
-# at one panel, between panels (the last one moves back) and below the smallest
-@pytest.mark.parametrize("n", [1, 17, 4096, 4097, 8192, 8209])
+# the default variant's row tiles (16, 32, 64 and 128 rows by the number of workgroups) and panels: n around the lines between the
+# tiles, m at one panel, between panels (the last one moves back) and below the smallest
+@pytest.mark.parametrize("n", [1, 17, 4096, 4097, 8192, 8209, 16390, 28690])
 @pytest.mark.parametrize("m", [32, 224, 256, 288, 480, 544, 768])
 def test_sgemv_panels(dev, n, m):
     O = ol.load()
