@@ -900,20 +900,31 @@ gemm_bf16_all_direct(const unsigned short* __restrict__ a, const unsigned short*
 // twice (TCP_TCC_READ_REQ: 12.8 M requests per 4096^3 launch instead of 8.4 M).  Here an A transfer is 256 rows x
 // 128 B for two K steps.  Three A buffers (96 KB) and the four B stages (64 KB) are all of the LDS: an A buffer is
 // free two K steps after its last read and its next transfer has to be complete a step before its first, so two
-// buffers would leave it one K step to land.  WI = 4 is that kernel.  With WI = 2 the tile is 128 x 128, all buffers are 80 KB and
-// two workgroups share a compute unit; LDS reads bound it (6 per 4 products; 16 KB a slice and workgroup), and against
-// the warp-specialised kernel of that tile it saves the ds_writes and the hand-offs: 2560 x 2560 x 1024 21.5 -> 18 us,
-// 1024^3 12.4 -> 10.3, 3072 x 2432 x 1408 29.6 -> 24.2 (both with the same order of tiles).  The A buffers form a ring indexed at run time (three does not divide
-// the K steps of every problem); a K step still issues eight loads, four of B and half an A transfer.
-template<int WI>
+// buffers would leave it one K step to land.  The A buffers form a ring indexed at run time (three does not divide the K steps of
+// every problem); a K step issues 2 * WI loads, WI of B and half an A transfer.  <4, 4> is that kernel.  With WI = 2 the tile is
+// 128 x 128; against the warp-specialised kernel of that tile it saves the ds_writes and the hand-offs (2560 x 2560 x 1024 21.5 -> 18 us,
+// 1024^3 12.4 -> 10.3, both with the same order of tiles).
+// STAGES is how far the loads run ahead: K step t requests B stage t + STAGES - 1, and A goes as far in STAGES / 2 + 1 buffers.  <2, 4>
+// takes 80 KB of LDS and two workgroups share a compute unit.  Where the grid gives a compute unit one, its two K steps in flight
+// do not cover the latency of DRAM: <2, 8>, 144 KB, has six (1408 x 1536 x 5248, 132 tiles: 44 us from the caches and 62 from DRAM with
+// <2, 4>, 36 and 48 with <2, 8>; the warp-specialised kernel 44 and 47).
+// With one wavefront per SIMD every instruction between two matrix instructions counts: the sources are pointers that move on with the
+// requests, kept in scalar registers (left alone the compiler forms them by vector additions and v_readfirstlane in <2, 8>: 128 x 128 x 1536
+// from the caches 13.5 us, 12.6 with the sources pinned, 12.2 with them moving; 4096^3 with <4, 4> 105.7 -> 104.7).
+// Counters (2048 x 1024 x 4096, one workgroup per compute unit, <2, 4> / <2, 8>): matrix cores busy 43 / 53 %, LDS busy 21 / 27 %, no
+// bank conflicts, wavefronts waiting for data 34 / 19 % of their cycles and for an issue slot 20 / 25 %; a K step takes a wavefront
+// 600 / 480 cycles for 256 of matrix instructions and about 60 others.  Nothing is saturated: with nothing else resident the waits at
+// the barrier of a K step and the issue of those 60 add up.
+template<int WI, int STAGES>
 __global__ void __launch_bounds__(256)
 gemm_bf16_all_direct_a64(const unsigned short* __restrict__ a, const unsigned short* __restrict__ b, float* __restrict__ c,
                          const int m, const int n, const int k)
 {
-  constexpr int WJ = WI, kBStages = 4, kABufs = 3, kBK4 = 32, kThreads = 256;
+  static_assert(STAGES == 4 || STAGES == 8, "the loop below takes four K steps at a time");
+  constexpr int WJ = WI, kBStages = STAGES, kAAhead = STAGES / 2, kABufs = kAAhead + 1, kBK4 = 32, kThreads = 256;
   constexpr int kBM = 64 * WI, kBN = 64 * WJ;
-  constexpr int kARow = 4 * kBK4, kBRow = kBN * 2;                 // 128 B (two K steps) and 512 B, unpadded
-  constexpr int kABuf = kBM * kARow, kBStage = kBK4 * kBRow;       // 32 KB and 16 KB
+  constexpr int kARow = 4 * kBK4, kBRow = kBN * 2;                 // 128 B (two K steps) and 128 * WI B, unpadded
+  constexpr int kABuf = kBM * kARow, kBStage = kBK4 * kBRow;       // 8 * WI and 4 * WI KB
   typedef CudaDMAStrided<false, 16, 16, kARow, kThreads, kBM> dma_a_t;
   typedef CudaDMAStrided<false, 16, 16, kBRow, kThreads, kBK4> dma_b_t;
   static_assert(dma_a_t::loads_per_thread() == 2 * WI && dma_b_t::loads_per_thread() == WI, "2 * WI loads per thread and K step");
@@ -926,18 +937,19 @@ gemm_bf16_all_direct_a64(const unsigned short* __restrict__ a, const unsigned sh
   tile_of_workgroup(blockIdx.x, m / kBM, n / kBN, tile_m, tile_n);
   const int ksteps = k / kBK4;            // a multiple of four
   const int klast = ksteps - 1, dlast = ksteps / 2 - 1;
-  const unsigned short* const src_a = a + (size_t)tile_m * kBM * k;
-  const unsigned short* const src_b = b + (size_t)tile_n * kBN;
+  const unsigned short* next_a = a + (size_t)tile_m * kBM * k;      // A transfer and B stage to request next; both go up one by one
+  const unsigned short* next_b = b + (size_t)tile_n * kBN;
   const size_t step_b = (size_t)kBK4 * n;
   // Round r of the B stage of K step t into B buffer `buf`; round r of A transfer d (K steps 2d, 2d+1) into A
-  // buffer `buf`.  Past the end the last one is requested again, into a buffer nobody reads any more.
+  // buffer `buf`.  Past the end the last one is requested again, into a buffer nobody reads any more.  The source moves on with
+  // the last round.
   auto issue_b = [&](const int t, const int buf, const int r) __attribute__((always_inline)) {
-    const int tt = t < klast ? t : klast;
-    dma_b.template issue_direct_part<STORE_LDS_DIRECT_SWIZZLE, true>(src_b + (size_t)tt * step_b, lds_b[buf], r, 1);
+    dma_b.template issue_direct_part<STORE_LDS_DIRECT_SWIZZLE, true>(next_b, lds_b[buf], r, 1);
+    if (r == WI - 1) { next_b += t < klast ? step_b : 0; asm("" : "+s"(next_b)); }
   };
   auto issue_a = [&](const int d, const int buf, const int r) __attribute__((always_inline)) {
-    const int dd = d < dlast ? d : dlast;
-    dma_a.template issue_direct_part<STORE_LDS_DIRECT_SWIZZLE, true>(src_a + (size_t)dd * (2 * kBK4), lds_a + buf * kABuf, r, 1);
+    dma_a.template issue_direct_part<STORE_LDS_DIRECT_SWIZZLE, true>(next_a, lds_a + buf * kABuf, r, 1);
+    if (r == 2 * WI - 1) { next_a += d < dlast ? 2 * kBK4 : 0; asm("" : "+s"(next_a)); }
   };
   const int lane = threadIdx.x & 63;
   const int wave = threadIdx.x >> 6;
@@ -1007,21 +1019,20 @@ gemm_bf16_all_direct_a64(const unsigned short* __restrict__ a, const unsigned sh
     }
   };
   bf16x8_t fa0[WI], fb0[WJ], fa1[WI], fb1[WJ];
-  // Before the loop, in the order the loop's wait counts assume: (A transfer 0, B stage 0), then what K steps -2
-  // and -1 would have issued: (B stage 1, first half of A transfer 1), (B stage 2, second half of A transfer 1).
+  // Before the loop, in the order the loop's wait counts assume: (A transfer 0, B stage 0), then what the STAGES - 2 K steps before
+  // step 0 would have issued: (B stage 1, first half of A transfer 1), (B stage 2, second half of A transfer 1) and so on.
 #pragma unroll
   for (int r = 0; r < 2 * WI; ++r) issue_a(0, 0, r);
 #pragma unroll
   for (int r = 0; r < WI; ++r) issue_b(0, 0, r);
 #pragma unroll
-  for (int r = 0; r < WI; ++r) issue_b(1, 1, r);
+  for (int t = 1; t < kBStages - 1; ++t) {
 #pragma unroll
-  for (int r = 0; r < WI; ++r) issue_a(1, 1, r);
+    for (int r = 0; r < WI; ++r) issue_b(t, t, r);
 #pragma unroll
-  for (int r = 0; r < WI; ++r) issue_b(2, 2, r);
-#pragma unroll
-  for (int r = WI; r < 2 * WI; ++r) issue_a(1, 1, r);
-  hipdma::wait_direct_loads<2 * kLoads>();
+    for (int r = 0; r < WI; ++r) issue_a((t + 1) / 2, (t + 1) / 2, (t % 2 == 1 ? 0 : WI) + r);
+  }
+  hipdma::wait_direct_loads<(kBStages - 2) * kLoads>();
   __builtin_amdgcn_s_barrier();
   // first slice of K step 0
   {
@@ -1034,29 +1045,40 @@ gemm_bf16_all_direct_a64(const unsigned short* __restrict__ a, const unsigned sh
       fb0[j] = bf16x8_t{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
     }
   }
-  // One K step t on B buffer bbuf and slices (2*h, 2*h+1) of A buffer abuf; the next step starts in A buffer nabuf
-  // at slice nq.  It issues B stage t + 3 and rounds [ar, ar + 4) of A transfer ad into A buffer aibuf.
+  // One K step t on B buffer bbuf and slices (2*h, 2*h+1) of A buffer abuf; the next step starts in A buffer nabuf at slice nq.  It
+  // issues B stage t + STAGES - 1 into the buffer that step t - 1 has left and rounds [ar, ar + WI) of A transfer ad into A buffer aibuf.
   auto k_step = [&](const int t, const int bbuf, const int abuf, const int h, const int nabuf, const int nq,
                     const int ad, const int aibuf, const int ar) __attribute__((always_inline)) {
-    hipdma::wait_direct_loads<kLoads>();          // everything up to K step t - 2; what step t - 1 issued stays in flight
+    // everything up to K step t + 2 - STAGES, which issued what step t + 1 reads; what the steps since then issued stays in flight
+    hipdma::wait_direct_loads<(kBStages - 3) * kLoads>();
     __builtin_amdgcn_s_barrier();
     half_step(fa0, fb0, fa1, fb1, abuf, 2 * h + 1, bbuf, 1, [&](const int i) __attribute__((always_inline)) {
-      issue_b(t + 3, (bbuf + 3) % kBStages, i);
+      issue_b(t + kBStages - 1, (bbuf + kBStages - 1) % kBStages, i);
     });
     half_step(fa1, fb1, fa0, fb0, nabuf, nq, (bbuf + 1) % kBStages, 0, [&](const int i) __attribute__((always_inline)) {
       issue_a(ad, aibuf, ar + i);
     });
   };
+  auto ring = [](const int i) __attribute__((always_inline)) { return i < kABufs ? i : i - kABufs; };
   int ab0 = 0;                                // A buffer of transfer kt / 2
-  for (int kt = 0; kt < ksteps; kt += 4) {
-    const int ab1 = ab0 == 2 ? 0 : ab0 + 1;   // transfer kt / 2 + 1
-    const int ab2 = ab1 == 2 ? 0 : ab1 + 1;   // transfer kt / 2 + 2, requested during K steps kt and kt + 1
-    const int d = kt >> 1;
-    k_step(kt, 0, ab0, 0, ab0, 2, d + 2, ab2, 0);
-    k_step(kt + 1, 1, ab0, 1, ab1, 0, d + 2, ab2, WI);
-    k_step(kt + 2, 2, ab1, 0, ab1, 2, d + 3, ab0, 0);     // transfer kt / 2 + 3 takes the buffer transfer kt / 2 has left
-    k_step(kt + 3, 3, ab1, 1, ab2, 0, d + 3, ab0, WI);
+  // K steps kt to kt + 3, the first in B buffer B0
+  auto four_steps = [&](const int kt, auto first) __attribute__((always_inline)) {
+    constexpr int B0 = decltype(first)::value;
+    const int ab1 = ring(ab0 + 1), ab2 = ring(ab0 + 2);       // transfers kt / 2 + 1 and kt / 2 + 2
+    const int abn = ring(ab0 + kAAhead);      // transfer kt / 2 + kAAhead, requested during K steps kt and kt + 1
+    const int d = (kt >> 1) + kAAhead;
+    k_step(kt, B0, ab0, 0, ab0, 2, d, abn, 0);
+    k_step(kt + 1, B0 + 1, ab0, 1, ab1, 0, d, abn, WI);
+    k_step(kt + 2, B0 + 2, ab1, 0, ab1, 2, d + 1, ab0, 0);    // the next transfer takes the buffer transfer kt / 2 has left
+    k_step(kt + 3, B0 + 3, ab1, 1, ab2, 0, d + 1, ab0, WI);
     ab0 = ab2;
+  };
+  // the B buffers are named by constants: one turn of the loop goes through all of them
+  for (int kt = 0; kt < ksteps; kt += kBStages) {
+    four_steps(kt, std::integral_constant<int, 0>());
+    if constexpr (kBStages == 8) {
+      if (kt + 4 < ksteps) four_steps(kt + 4, std::integral_constant<int, 4>());
+    }
   }
   hipdma::wait_direct_loads<0>();
   float* cbase = c + (size_t)(tile_m * kBM + wm) * n + (size_t)tile_n * kBN + wn;
@@ -1129,7 +1151,10 @@ extern "C" int cudadma_gemm_bf16(const uint16_t* d_a, const uint16_t* d_b, float
     else {
       const long long grid = (long long)(m / 128) * (n / 128);
       CUDADMA_REQUIRE(grid <= 0x7fffffffLL, "grid too large");
-      hipLaunchKernelGGL(gemm_bf16_all_direct_a64<2>, dim3((unsigned)grid), dim3(256), 0, s, d_a, d_b, d_c, m, n, k);
+      // one tile or none for a compute unit: requests that run further ahead, from the K steps on that pay for as many before the first
+      // product (<2, 4> / <2, 8>, caches and DRAM: 1152 x 256 x 512 6.3 / 6.8 and 6.9 / 6.9 us, 768 x 2048 x 4736 40 / 33 and 56 / 45)
+      if (grid <= cus && k >= 512) hipLaunchKernelGGL((gemm_bf16_all_direct_a64<2, 8>), dim3((unsigned)grid), dim3(256), 0, s, d_a, d_b, d_c, m, n, k);
+      else hipLaunchKernelGGL((gemm_bf16_all_direct_a64<2, 4>), dim3((unsigned)grid), dim3(256), 0, s, d_a, d_b, d_c, m, n, k);
       CUDADMA_HIP_CHECK(hipGetLastError());
       return CUDADMA_OK;
     }
@@ -1148,7 +1173,7 @@ extern "C" int cudadma_gemm_bf16(const uint16_t* d_a, const uint16_t* d_b, float
       const long long grid = (long long)(m / 256) * (n / 256);
       CUDADMA_REQUIRE(grid <= 0x7fffffffLL, "grid too large");
       if (variant == 7) hipLaunchKernelGGL(gemm_bf16_ws_direct4_a64, dim3((unsigned)grid), dim3(512 + 2 * kDirect4DmaThreads), 0, s, d_a, d_b, d_c, m, n, k);
-      else if (variant == 9) hipLaunchKernelGGL(gemm_bf16_all_direct_a64<4>, dim3((unsigned)grid), dim3(256), 0, s, d_a, d_b, d_c, m, n, k);
+      else if (variant == 9) hipLaunchKernelGGL((gemm_bf16_all_direct_a64<4, 4>), dim3((unsigned)grid), dim3(256), 0, s, d_a, d_b, d_c, m, n, k);
 #ifdef HIPDMA_SWEEP_VARIANTS
       else if (variant == 6) hipLaunchKernelGGL(gemm_bf16_ws_direct4, dim3((unsigned)grid), dim3(512 + 2 * kDirect4DmaThreads), 0, s, d_a, d_b, d_c, m, n, k);
       else hipLaunchKernelGGL(gemm_bf16_all_direct, dim3((unsigned)grid), dim3(256), 0, s, d_a, d_b, d_c, m, n, k);
