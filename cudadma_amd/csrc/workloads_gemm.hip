@@ -38,34 +38,58 @@ struct GemmShape {
   static constexpr int kBPitch = kBN * 2 + 64;      // B row in LDS: the four rows a transposing read touches land 64 B apart modulo 256
   static constexpr int kAStage = kBM * kAPitch;
   static constexpr int kBStage = kBK * kBPitch;
+  static constexpr int kPerCu = 2 * (kAStage + kBStage) <= (80 << 10) ? 2 : 1;      // workgroups that share a compute unit's LDS
   typedef CudaDMAStrided<false, 16, kBM * kBK * 2 / kDmaWave, kBK * 2, kDmaWave, kBM> dma_a_t;   // kBM rows x 128 B
   typedef CudaDMAStrided<false, 16, kBK * kBN * 2 / kDmaWave, kBN * 2, kDmaWave, kBK> dma_b_t;   // 64 rows x 2*kBN B
 };
 
-// Workgroup -> tile.  Workgroup b runs on XCD b % 8; when the tile grid divides into eight
-// 2-D blocks (4 along m, 2 along n) every XCD gets one compact block, so its L2 holds few
-// distinct A and B panels.  Other grids are walked in bands of up to eight tile rows, down the
-// columns of a band, and every XCD gets an eighth of that walk: the tiles in work on it
-// at one time are about as many rows as columns (tiles dealt row-major instead: 3712 x 4736 x 3712 with 128 x 128 tiles 188 us
-// against 139, 640 x 8064 x 2048 34 / 28).  Grids that do divide keep their blocks: the walk is level or slower there
-// (8192 x 8192 x 1024, 256 x 256 tiles: 140 us against 155).
-__device__ __forceinline__ void tile_of_workgroup(const int b, const int tiles_m, const int tiles_n, int& tile_m, int& tile_n)
+// Workgroup -> tile.  Workgroup b runs on XCD b % 8.  `walk` is what tile_walk() chose: blocks, row-major, or the rows of a band.
+constexpr int kWalkBlocks = 0, kWalkRowMajor = -1;
+__device__ __forceinline__ void tile_of_workgroup(const int b, const int tiles_m, const int tiles_n, const int walk, int& tile_m, int& tile_n)
 {
   const int xcd = b & 7, idx = b >> 3;
-  if ((tiles_m % 4) == 0 && (tiles_n % 2) == 0) {
+  if (walk == kWalkBlocks) {
     const int bm = tiles_m / 4, bn = tiles_n / 2;       // block of one XCD
     tile_m = (xcd >> 1) * bm + idx / bn;
     tile_n = (xcd & 1) * bn + idx % bn;
-    return;
+  } else if (walk == kWalkRowMajor) {
+    tile_m = b / tiles_n;
+    tile_n = b % tiles_n;
+  } else {
+    const int rows = walk, tiles = tiles_m * tiles_n, each = tiles >> 3, more = tiles & 7;
+    const int at = xcd * each + (xcd < more ? xcd : more) + idx;
+    const int band = at / (rows * tiles_n), in_band = at - band * rows * tiles_n;
+    const int height = tiles_m - band * rows < rows ? tiles_m - band * rows : rows;
+    tile_n = in_band / height;
+    tile_m = band * rows + in_band - tile_n * height;
   }
-  const int tiles = tiles_m * tiles_n, each = tiles >> 3, more = tiles & 7;
-  const int at = xcd * each + (xcd < more ? xcd : more) + idx;
+}
+
+// The order in which the workgroups take the tiles; `per_cu` of them share a compute unit.  Every XCD has an L2 of its own, so the panels
+// of A and B behind the tiles that are in work on one XCD at a time should be few.
+//   blocks     grids that divide into 4 x 2: every XCD gets one compact block.
+//   bands      up to eight tile rows, down the columns of a band, an eighth of that walk for every XCD (dealt row-major instead:
+//              3712 x 4736 x 3712 with 128 x 128 tiles 188 us against 139, 640 x 8064 x 2048 34 / 28).  In grids that divide level or slower than
+//              blocks (8192 x 8192 x 1024, 256 x 256 tiles: 155 us against 140).
+//   row-major  where eight divides the tiles of a row, so that every XCD has columns of its own, and its rows and columns are then no more
+//              than with bands (7680 x 8192 x 384, 256 x 256 tiles: 79 us, bands 87; 640 x 8192 x 1024, 128 x 128: 15.5 / 16.8.  But
+//              16 rows and 4 columns against 8 and 8: 3712 x 4096 x 640 33.5 / 28.8 from DRAM; 15 and 2 against 6 and 5: 1920 x 2048 x 2048
+//              26.6 / 23.0); where one round of tiles is over in a few K steps and finding the place in a band counts (0.2 us: 640 x 4096 x 256
+//              5.4 / 5.6); and with two K steps of 64, when a tile is mostly its block of C and the bands scatter the writes of a large C, as long as
+//              an L2 holds B (from DRAM: 8064 x 8064 x 128 49 / 55, 4224 x 5760 x 128 20.7 / 22.9; 6528 x 896 x 128, a small C, 8.0 / 7.5;
+//              2176 x 7808 x 256 24.4 / 21.9).
+int tile_walk(const int m, const int n, const int k, const int tile_rows, const int tile_cols, const int per_cu)
+{
+  const int tiles_m = m / tile_rows, tiles_n = n / tile_cols;
+  if ((tiles_m % 4) == 0 && (tiles_n % 2) == 0) return kWalkBlocks;
+  const int cus = workloads::device_cus();
+  const long long tiles = (long long)tiles_m * tiles_n, each = tiles / 8;
   int rows = 1;
   while (rows < 8 && rows * rows < each) ++rows;
-  const int band = at / (rows * tiles_n), in_band = at - band * rows * tiles_n;
-  const int height = tiles_m - band * rows < rows ? tiles_m - band * rows : rows;
-  tile_n = in_band / height;
-  tile_m = band * rows + in_band - tile_n * height;
+  const double in_work = (double)(each < per_cu * cus / 8 ? each : per_cu * cus / 8), columns = tiles_n / 8;
+  const bool own_columns = (tiles_n % 8) == 0 && in_work / columns + columns <= rows + in_work / rows + 1;
+  const bool mostly_c = k < 256 && (long long)n * k < (3 << 19) && (long long)m * n >= (16 << 20);
+  return own_columns || mostly_c || (tiles <= cus && k < 512) ? kWalkRowMajor : rows;
 }
 
 // Order of one slice for the instruction scheduler: MFMAs matrix instructions with the READS
@@ -86,7 +110,7 @@ __device__ __forceinline__ void pin_slice()
 template<int WI, int WJ, int WM = 2, int WN = 2>
 __global__ void __launch_bounds__(64 * WM * WN + 2 * kDmaWave)
 gemm_bf16_ws(const unsigned short* __restrict__ a, const unsigned short* __restrict__ b, float* __restrict__ c,
-             const int m, const int n, const int k)
+             const int m, const int n, const int k, const int walk)
 {
   typedef GemmShape<WI, WJ, WM, WN> shape;
   constexpr int kComputeThreads = shape::kCompute;
@@ -105,7 +129,7 @@ gemm_bf16_ws(const unsigned short* __restrict__ a, const unsigned short* __restr
   cudaDMACustom stage0(0, 2 * kDmaWave, kComputeThreads, kComputeThreads);
   cudaDMACustom stage1(1, 2 * kDmaWave, kComputeThreads, kComputeThreads);
   int tile_m, tile_n;
-  tile_of_workgroup(blockIdx.x, m / shape::kBM, n / shape::kBN, tile_m, tile_n);
+  tile_of_workgroup(blockIdx.x, m / shape::kBM, n / shape::kBN, walk, tile_m, tile_n);
   const int ksteps = k / kBK;            // even: k is a multiple of 2 * kBK
   const int klast = ksteps - 1;
 
@@ -263,7 +287,7 @@ struct Three {
 #ifdef HIPDMA_SWEEP_VARIANTS
 __global__ void __launch_bounds__(kComputeThreads + 2 * kDmaWave)
 gemm_bf16_ws_direct(const unsigned short* __restrict__ a, const unsigned short* __restrict__ b, float* __restrict__ c,
-                    const int m, const int n, const int k)
+                    const int m, const int n, const int k, const int walk)
 {
   constexpr int WI = 4, WJ = 2, kStages = 3;
   constexpr int kBM = 64 * WI, kBN = 64 * WJ;
@@ -279,7 +303,7 @@ gemm_bf16_ws_direct(const unsigned short* __restrict__ a, const unsigned short* 
                              cudaDMACustom(1, 2 * kDmaWave, kComputeThreads, kComputeThreads),
                              cudaDMACustom(2, 2 * kDmaWave, kComputeThreads, kComputeThreads)};
   int tile_m, tile_n;
-  tile_of_workgroup(blockIdx.x, m / kBM, n / kBN, tile_m, tile_n);
+  tile_of_workgroup(blockIdx.x, m / kBM, n / kBN, walk, tile_m, tile_n);
   const int ksteps = k / kBK;
 
   // One DMA wavefront: tile t lands in stage t % 3.  Tiles t+1 and t+2 are in flight while the
@@ -426,7 +450,7 @@ constexpr int kDirect4Ahead = 3;           // transfers in flight per DMA wavefr
 #ifdef HIPDMA_SWEEP_VARIANTS
 __global__ void __launch_bounds__(512 + 2 * kDirect4DmaThreads)
 gemm_bf16_ws_direct4(const unsigned short* __restrict__ a, const unsigned short* __restrict__ b, float* __restrict__ c,
-                     const int m, const int n, const int k)
+                     const int m, const int n, const int k, const int walk)
 {
   constexpr int WI = 4, WJ = 2, WN = 4, kStages = 4, kBK4 = 32, kCompute = 512, kDmaWave = kDirect4DmaThreads;
   constexpr int kBM = 256, kBN = 256;
@@ -441,7 +465,7 @@ gemm_bf16_ws_direct4(const unsigned short* __restrict__ a, const unsigned short*
   Four4<cudaDMACustom> stage{cudaDMACustom(0, 2 * kDmaWave, kCompute, kCompute), cudaDMACustom(1, 2 * kDmaWave, kCompute, kCompute),
                              cudaDMACustom(2, 2 * kDmaWave, kCompute, kCompute), cudaDMACustom(3, 2 * kDmaWave, kCompute, kCompute)};
   int tile_m, tile_n;
-  tile_of_workgroup(blockIdx.x, m / kBM, n / kBN, tile_m, tile_n);
+  tile_of_workgroup(blockIdx.x, m / kBM, n / kBN, walk, tile_m, tile_n);
   const int ksteps = k / kBK4;            // a multiple of four: k is a multiple of 128
 
   // One DMA wavefront: tile t lands in stage t % 4; tiles t+1 .. t+3 are in flight while the compute
@@ -578,7 +602,7 @@ gemm_bf16_ws_direct4(const unsigned short* __restrict__ a, const unsigned short*
 // an A buffer every other step.
 __global__ void __launch_bounds__(512 + 2 * kDirect4DmaThreads)
 gemm_bf16_ws_direct4_a64(const unsigned short* __restrict__ a, const unsigned short* __restrict__ b, float* __restrict__ c,
-                         const int m, const int n, const int k)
+                         const int m, const int n, const int k, const int walk)
 {
   constexpr int WI = 4, WJ = 2, WN = 4, kBStages = 4, kBK4 = 32, kCompute = 512, kDmaWave = kDirect4DmaThreads;
   constexpr int kBM = 256, kBN = 256;
@@ -595,7 +619,7 @@ gemm_bf16_ws_direct4_a64(const unsigned short* __restrict__ a, const unsigned sh
   cudaDMACustom ga0(4, kDmaWave, kCompute, kCompute);
   cudaDMACustom ga1(5, kDmaWave, kCompute, kCompute);
   int tile_m, tile_n;
-  tile_of_workgroup(blockIdx.x, m / kBM, n / kBN, tile_m, tile_n);
+  tile_of_workgroup(blockIdx.x, m / kBM, n / kBN, walk, tile_m, tile_n);
   const int ksteps = k / kBK4;            // a multiple of four: k is a multiple of 128
 
   if (dma_a.owns_this_thread()) {
@@ -750,7 +774,7 @@ gemm_bf16_ws_direct4_a64(const unsigned short* __restrict__ a, const unsigned sh
 #ifdef HIPDMA_SWEEP_VARIANTS
 __global__ void __launch_bounds__(256)
 gemm_bf16_all_direct(const unsigned short* __restrict__ a, const unsigned short* __restrict__ b, float* __restrict__ c,
-                     const int m, const int n, const int k)
+                     const int m, const int n, const int k, const int walk)
 {
   constexpr int WI = 4, WJ = 4, kStages = 4, kBK4 = 32, kThreads = 256;
   constexpr int kBM = 256, kBN = 256;
@@ -764,7 +788,7 @@ gemm_bf16_all_direct(const unsigned short* __restrict__ a, const unsigned short*
   dma_a_t dma_a(k * 2, kARow);
   dma_b_t dma_b(n * 2, kBRow);
   int tile_m, tile_n;
-  tile_of_workgroup(blockIdx.x, m / kBM, n / kBN, tile_m, tile_n);
+  tile_of_workgroup(blockIdx.x, m / kBM, n / kBN, walk, tile_m, tile_n);
   const int ksteps = k / kBK4;            // a multiple of four
   const int klast = ksteps - 1;
   const unsigned short* const src_a = a + (size_t)tile_m * kBM * k;
@@ -918,7 +942,7 @@ gemm_bf16_all_direct(const unsigned short* __restrict__ a, const unsigned short*
 template<int WI, int STAGES>
 __global__ void __launch_bounds__(256)
 gemm_bf16_all_direct_a64(const unsigned short* __restrict__ a, const unsigned short* __restrict__ b, float* __restrict__ c,
-                         const int m, const int n, const int k)
+                         const int m, const int n, const int k, const int walk)
 {
   static_assert(STAGES == 4 || STAGES == 8, "the loop below takes four K steps at a time");
   constexpr int WJ = WI, kBStages = STAGES, kAAhead = STAGES / 2, kABufs = kAAhead + 1, kBK4 = 32, kThreads = 256;
@@ -934,7 +958,7 @@ gemm_bf16_all_direct_a64(const unsigned short* __restrict__ a, const unsigned sh
   dma_a_t dma_a(k * 2, kARow);
   dma_b_t dma_b(n * 2, kBRow);
   int tile_m, tile_n;
-  tile_of_workgroup(blockIdx.x, m / kBM, n / kBN, tile_m, tile_n);
+  tile_of_workgroup(blockIdx.x, m / kBM, n / kBN, walk, tile_m, tile_n);
   const int ksteps = k / kBK4;            // a multiple of four
   const int klast = ksteps - 1, dlast = ksteps / 2 - 1;
   const unsigned short* next_a = a + (size_t)tile_m * kBM * k;      // A transfer and B stage to request next; both go up one by one
@@ -1103,7 +1127,7 @@ int launch_gemm(const uint16_t* d_a, const uint16_t* d_b, float* d_c, int m, int
   const long long grid = (long long)(m / shape::kBM) * (n / shape::kBN);
   CUDADMA_REQUIRE(grid <= 0x7fffffffLL, "grid too large");
   hipLaunchKernelGGL((gemm_bf16_ws<WI, WJ, WM, WN>), dim3((unsigned)grid), dim3(shape::kCompute + 2 * kDmaWave), 0, stream,
-                     d_a, d_b, d_c, m, n, k);
+                     d_a, d_b, d_c, m, n, k, tile_walk(m, n, k, shape::kBM, shape::kBN, shape::kPerCu));
   CUDADMA_HIP_CHECK(hipGetLastError());
   return CUDADMA_OK;
 }
@@ -1153,8 +1177,8 @@ extern "C" int cudadma_gemm_bf16(const uint16_t* d_a, const uint16_t* d_b, float
       CUDADMA_REQUIRE(grid <= 0x7fffffffLL, "grid too large");
       // one tile or none for a compute unit: requests that run further ahead, from the K steps on that pay for as many before the first
       // product (<2, 4> / <2, 8>, caches and DRAM: 1152 x 256 x 512 6.3 / 6.8 and 6.9 / 6.9 us, 768 x 2048 x 4736 40 / 33 and 56 / 45)
-      if (grid <= cus && k >= 512) hipLaunchKernelGGL((gemm_bf16_all_direct_a64<2, 8>), dim3((unsigned)grid), dim3(256), 0, s, d_a, d_b, d_c, m, n, k);
-      else hipLaunchKernelGGL((gemm_bf16_all_direct_a64<2, 4>), dim3((unsigned)grid), dim3(256), 0, s, d_a, d_b, d_c, m, n, k);
+      if (grid <= cus && k >= 512) hipLaunchKernelGGL((gemm_bf16_all_direct_a64<2, 8>), dim3((unsigned)grid), dim3(256), 0, s, d_a, d_b, d_c, m, n, k, tile_walk(m, n, k, 128, 128, 1));
+      else hipLaunchKernelGGL((gemm_bf16_all_direct_a64<2, 4>), dim3((unsigned)grid), dim3(256), 0, s, d_a, d_b, d_c, m, n, k, tile_walk(m, n, k, 128, 128, 2));
       CUDADMA_HIP_CHECK(hipGetLastError());
       return CUDADMA_OK;
     }
@@ -1172,11 +1196,12 @@ extern "C" int cudadma_gemm_bf16(const uint16_t* d_a, const uint16_t* d_b, float
       CUDADMA_REQUIRE(variant <= 7 || direct_rows_fit(n, k), "rows of %d x %d are too long for the lane offsets of this variant (0, 1 and 7 take them)", k, n);
       const long long grid = (long long)(m / 256) * (n / 256);
       CUDADMA_REQUIRE(grid <= 0x7fffffffLL, "grid too large");
-      if (variant == 7) hipLaunchKernelGGL(gemm_bf16_ws_direct4_a64, dim3((unsigned)grid), dim3(512 + 2 * kDirect4DmaThreads), 0, s, d_a, d_b, d_c, m, n, k);
-      else if (variant == 9) hipLaunchKernelGGL((gemm_bf16_all_direct_a64<4, 4>), dim3((unsigned)grid), dim3(256), 0, s, d_a, d_b, d_c, m, n, k);
+      const int walk = tile_walk(m, n, k, 256, 256, 1);
+      if (variant == 7) hipLaunchKernelGGL(gemm_bf16_ws_direct4_a64, dim3((unsigned)grid), dim3(512 + 2 * kDirect4DmaThreads), 0, s, d_a, d_b, d_c, m, n, k, walk);
+      else if (variant == 9) hipLaunchKernelGGL((gemm_bf16_all_direct_a64<4, 4>), dim3((unsigned)grid), dim3(256), 0, s, d_a, d_b, d_c, m, n, k, walk);
 #ifdef HIPDMA_SWEEP_VARIANTS
-      else if (variant == 6) hipLaunchKernelGGL(gemm_bf16_ws_direct4, dim3((unsigned)grid), dim3(512 + 2 * kDirect4DmaThreads), 0, s, d_a, d_b, d_c, m, n, k);
-      else hipLaunchKernelGGL(gemm_bf16_all_direct, dim3((unsigned)grid), dim3(256), 0, s, d_a, d_b, d_c, m, n, k);
+      else if (variant == 6) hipLaunchKernelGGL(gemm_bf16_ws_direct4, dim3((unsigned)grid), dim3(512 + 2 * kDirect4DmaThreads), 0, s, d_a, d_b, d_c, m, n, k, walk);
+      else hipLaunchKernelGGL(gemm_bf16_all_direct, dim3((unsigned)grid), dim3(256), 0, s, d_a, d_b, d_c, m, n, k, walk);
 #else
       else CUDADMA_REQUIRE(false, "gemm variant %d is a sweep kernel: build the library with make EXTRA=-DHIPDMA_SWEEP_VARIANTS", variant);
 #endif
@@ -1188,7 +1213,7 @@ extern "C" int cudadma_gemm_bf16(const uint16_t* d_a, const uint16_t* d_b, float
       CUDADMA_REQUIRE((m % 256) == 0, "this variant needs m a multiple of 256 (got %d)", m);
       const long long grid = (long long)(m / 256) * (n / 128);
       CUDADMA_REQUIRE(grid <= 0x7fffffffLL, "grid too large");
-      hipLaunchKernelGGL(gemm_bf16_ws_direct, dim3((unsigned)grid), dim3(kComputeThreads + 2 * kDmaWave), 0, s, d_a, d_b, d_c, m, n, k);
+      hipLaunchKernelGGL(gemm_bf16_ws_direct, dim3((unsigned)grid), dim3(kComputeThreads + 2 * kDmaWave), 0, s, d_a, d_b, d_c, m, n, k, tile_walk(m, n, k, 256, 128, 1));
       CUDADMA_HIP_CHECK(hipGetLastError());
       return CUDADMA_OK;
 #else

@@ -556,10 +556,11 @@ def test_gemm_full_size(device, variant):
     assert float((d_c - ref).abs().max()) <= 1e-2 * 64.0
 
 
-# tile grids that divide into eight blocks and that do not (fewer tiles than XCDs, bands of tile rows with a remainder), both tiles of
-# the default variant, one and several rounds
+# tile grids that divide into eight blocks and that do not (fewer tiles than XCDs, bands of tile rows with a remainder, rows of tiles
+# that eight divides, a large C of few K steps), both tiles of the default variant, one and several rounds
 @pytest.mark.parametrize("shape", [(128, 128, 128), (128, 896, 256), (384, 1152, 128), (1152, 1408, 384), (2944, 2432, 128), (2816, 2816, 256),
-                                   (3072, 3072, 128), (3328, 3840, 128)])
+                                   (3072, 3072, 128), (3328, 3840, 128), (2176, 3072, 256), (4224, 4224, 128), (1280, 4096, 256), (640, 2048, 1024),
+                                   (768, 4096, 128)])
 @pytest.mark.parametrize("variant", [0, 1])
 def test_gemm_tile_walks(device, shape, variant):
     m, n, k = shape
