@@ -1043,20 +1043,24 @@ gemm_bf16_all_direct_a64(const unsigned short* __restrict__ a, const unsigned sh
     }
   };
   bf16x8_t fa0[WI], fb0[WJ], fa1[WI], fb1[WJ];
-  // Before the loop, in the order the loop's wait counts assume: (A transfer 0, B stage 0), then what the STAGES - 2 K steps before
-  // step 0 would have issued: (B stage 1, first half of A transfer 1), (B stage 2, second half of A transfer 1) and so on.
+  // Group g of the requests, in the order that all wait counts assume: B stage g and the half of A transfer (g + 1) / 2 that goes with it
+  // (the first half with odd g); group 0 is B stage 0 and all of A transfer 0.  K step t reads groups up to t + 1 and issues group
+  // t + STAGES - 1.
+  auto issue_of_group = [&](const int g, const int i) __attribute__((always_inline)) {
+    issue_b(g, g % kBStages, i);
+    issue_a((g + 1) / 2, (g + 1) / 2 % kABufs, (g % 2 == 1 ? 0 : WI) + i);
+  };
+  constexpr int kFirstGroups = 2;             // behind group 0, before the first product
 #pragma unroll
   for (int r = 0; r < 2 * WI; ++r) issue_a(0, 0, r);
 #pragma unroll
   for (int r = 0; r < WI; ++r) issue_b(0, 0, r);
 #pragma unroll
-  for (int t = 1; t < kBStages - 1; ++t) {
+  for (int g = 1; g <= kFirstGroups; ++g) {
 #pragma unroll
-    for (int r = 0; r < WI; ++r) issue_b(t, t, r);
-#pragma unroll
-    for (int r = 0; r < WI; ++r) issue_a((t + 1) / 2, (t + 1) / 2, (t % 2 == 1 ? 0 : WI) + r);
+    for (int r = 0; r < WI; ++r) issue_of_group(g, r);
   }
-  hipdma::wait_direct_loads<(kBStages - 2) * kLoads>();
+  hipdma::wait_direct_loads<kFirstGroups * kLoads>();
   __builtin_amdgcn_s_barrier();
   // first slice of K step 0
   {
@@ -1097,12 +1101,28 @@ gemm_bf16_all_direct_a64(const unsigned short* __restrict__ a, const unsigned sh
     k_step(kt + 3, B0 + 3, ab1, 1, ab2, 0, d + 1, ab0, WI);
     ab0 = ab2;
   };
+  // With eight stages the first four K steps issue two groups each, 3 to 10, and so reach the distance that the others keep.  (All six
+  // groups before the first product held it up: 128 x 128 x 768 from the caches 7.9 us, 7.6 so, 7.4 with <2, 4>.)  Groups 8 to 10 go where K steps 0 to 2 have been.
+  auto ramp_step = [&](auto step) __attribute__((always_inline)) {
+    constexpr int t = decltype(step)::value, issued = kFirstGroups + 2 * t;
+    hipdma::wait_direct_loads<(issued - (t + 1)) * kLoads>();
+    __builtin_amdgcn_s_barrier();
+    half_step(fa0, fb0, fa1, fb1, t / 2, 2 * (t % 2) + 1, t, 1, [&](const int i) __attribute__((always_inline)) { issue_of_group(issued + 1, i); });
+    half_step(fa1, fb1, fa0, fb0, (t + 1) / 2, t % 2 == 0 ? 2 : 0, t + 1, 0, [&](const int i) __attribute__((always_inline)) { issue_of_group(issued + 2, i); });
+  };
   // the B buffers are named by constants: one turn of the loop goes through all of them
-  for (int kt = 0; kt < ksteps; kt += kBStages) {
-    four_steps(kt, std::integral_constant<int, 0>());
-    if constexpr (kBStages == 8) {
-      if (kt + 4 < ksteps) four_steps(kt + 4, std::integral_constant<int, 4>());
+  if constexpr (kBStages == 8) {
+    ramp_step(std::integral_constant<int, 0>());
+    ramp_step(std::integral_constant<int, 1>());
+    ramp_step(std::integral_constant<int, 2>());
+    ramp_step(std::integral_constant<int, 3>());
+    ab0 = 2;
+    for (int kt = 4; kt < ksteps; kt += 8) {
+      four_steps(kt, std::integral_constant<int, 4>());
+      if (kt + 4 < ksteps) four_steps(kt + 4, std::integral_constant<int, 0>());
     }
+  } else {
+    for (int kt = 0; kt < ksteps; kt += 4) four_steps(kt, std::integral_constant<int, 0>());
   }
   hipdma::wait_direct_loads<0>();
   float* cbase = c + (size_t)(tile_m * kBM + wm) * n + (size_t)tile_n * kBN + wn;
@@ -1175,9 +1195,11 @@ extern "C" int cudadma_gemm_bf16(const uint16_t* d_a, const uint16_t* d_b, float
     else {
       const long long grid = (long long)(m / 128) * (n / 128);
       CUDADMA_REQUIRE(grid <= 0x7fffffffLL, "grid too large");
-      // one tile or none for a compute unit: requests that run further ahead, from the K steps on that pay for as many before the first
-      // product (<2, 4> / <2, 8>, caches and DRAM: 1152 x 256 x 512 6.3 / 6.8 and 6.9 / 6.9 us, 768 x 2048 x 4736 40 / 33 and 56 / 45)
-      if (grid <= cus && k >= 512) hipLaunchKernelGGL((gemm_bf16_all_direct_a64<2, 8>), dim3((unsigned)grid), dim3(256), 0, s, d_a, d_b, d_c, m, n, k, tile_walk(m, n, k, 128, 128, 1));
+      // One tile or none for a compute unit: requests that run further ahead, from the k on at which <2, 4> loses from DRAM what it gained
+      // over the warp-specialised kernel (us, <2, 4> / <2, 8> from the caches, <2, 4> / <2, 8> / variant 1 from DRAM): 2048 x 2048 x 640
+      // 9.4 / 9.9, 10.2 / 10.3 / 10.6; x 768 10.3 / 10.5, 13.4 / 12.3 / 12.3; x 1280 15.1 / 15.2, 19.2 / 17.1 / 16.9; x 2048 23.3 / 20.9,
+      // 28.7 / 24.2 / 24.6; 768 x 2048 x 4736 40 / 33, 56 / 45.
+      if (grid <= cus && k >= 768) hipLaunchKernelGGL((gemm_bf16_all_direct_a64<2, 8>), dim3((unsigned)grid), dim3(256), 0, s, d_a, d_b, d_c, m, n, k, tile_walk(m, n, k, 128, 128, 1));
       else hipLaunchKernelGGL((gemm_bf16_all_direct_a64<2, 4>), dim3((unsigned)grid), dim3(256), 0, s, d_a, d_b, d_c, m, n, k, tile_walk(m, n, k, 128, 128, 2));
       CUDADMA_HIP_CHECK(hipGetLastError());
       return CUDADMA_OK;
