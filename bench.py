@@ -53,7 +53,7 @@ PATTERN_KERNELS = {
     "halo": "stencil_ws_vec4<2, 8>",
     "halo_handshake": "stencil_ws_vec4<0, 8>",
     "halo_wide_tiles": "stencil_ws_vec4<2, 8>",          # the same template in the translation unit compiled for 64 x 16 tiles
-    "gemm": "gemm_bf16_all_direct_a64",
+    "gemm": "gemm_bf16_all_direct_a64<4, 4>",
     "gemm_warp_specialised": "gemm_bf16_ws_direct4_a64",
 }
 

@@ -294,7 +294,7 @@ long long cudadma_probe_pattern(int mode, const void* d_in, const int32_t* d_idx
  * The kernels behind these are written against the DMA classes alone (the first-
  * generation names of include/cudaDMA.h for saxpy and sgemv, the current ones for the
  * stencil); the reference has them as stand-alone programs with compile-time sizes,
- * here sizes are arguments and the launch geometry is fixed per example. */
+ * here sizes are arguments, and the tiles of sgemv and the grid of the stencil follow from them. */
 enum {
   CUDADMA_EXAMPLE_SAXPY     = 0,
   CUDADMA_EXAMPLE_SGEMV     = 1,
