@@ -31,35 +31,45 @@ const char* const kGemvNames[] = {
   "vector staged by cudaDMASequential, one buffer",
   "vector staged by two cudaDMASequential on shared DMA threads",
   "vector by cudaDMASequential + 32-column panel by cudaDMAStrided, one buffer each",
-  "vector by cudaDMASequential + panel of 32 to 256 columns by CudaDMAStrided, two buffers each",
+  "vector and matrix in a ring of four stages of 128 columns by direct-to-LDS CudaDMAStrided; 32-column panels, two buffers each, for narrow matrices and for many rows",
 };
 
-template<int ROWS, int COLS, int VEC_DMA, int MAT_DMA, int MAT_BYTES = 4 * ROWS * COLS / MAT_DMA>
-void launch_sgemv_panels(hipStream_t s, int n, int m, float alpha, const float* a, int lda, const float* x, float* y)
+template<int ROWS, int MAT_DMA, int MAT_BYTES = 4 * ROWS * kGemvPanelCols / MAT_DMA>
+void launch_sgemv_small_panels(hipStream_t s, int n, int m, float alpha, const float* a, int lda, const float* x, float* y)
 {
-  hipLaunchKernelGGL((sgemvn_both_double<ROWS, COLS, VEC_DMA, MAT_DMA, MAT_BYTES>), dim3((n + ROWS - 1) / ROWS),
-                     dim3((sgemv_both_double_threads<ROWS, VEC_DMA, MAT_DMA>())), 0, s, n, m, alpha, a, lda, x, y);
+  hipLaunchKernelGGL((sgemvn_both_double<ROWS, kGemvPanelCols, kGemvDmaPerLd, MAT_DMA, MAT_BYTES>), dim3((n + ROWS - 1) / ROWS),
+                     dim3((sgemv_both_double_threads<ROWS, kGemvDmaPerLd, MAT_DMA>())), 0, s, n, m, alpha, a, lda, x, y);
 }
 
-// The narrowest row tile that gives no compute unit a second workgroup: a row is one chain of multiply-adds whatever the tile, so
-// more and narrower workgroups share the bytes (4096 x 4096: 30 / 31 / 36 / 59 us with tiles of 16 / 32 / 64 / 128 rows); beyond one
-// workgroup per compute unit the memory counts, and with it the length of the pieces of a column (8192 x 8192: 100 / 60 / 70 us with
-// 16 / 32 / 64 rows, 16384 x 16384: 344 / 206 / 170).  The last panel moves back to end with the last column, so a matrix needs at
-// least the columns of one panel; narrower ones go through panels of 32 columns (16384 x 224: 5.1 us with 64 rows, 5.7 with 128).  So
-// do those with more rows than one tile of 64 per compute unit: several workgroups then share a compute unit and hide each
-// other's hand-offs, and small panels leave room for them (panels of 128 / 32 columns: 20480 x 4096 78 / 63 us, 28672 x 4096 91 / 78).
-// From about two such tiles per compute unit on, the longer pieces of 128 rows count again, in bursts of 64 bytes a thread (64 / 128
-// rows: 32768 x 2048 42 / 39 us, 98304 x 1024 76 / 72).
+template<int ROWS, int DMA_WAVES>
+void launch_sgemv_ring(hipStream_t s, int n, int m, float alpha, const float* a, int lda, const float* x, float* y)
+{
+  hipLaunchKernelGGL((sgemvn_ring<ROWS, DMA_WAVES>), dim3((n + ROWS - 1) / ROWS), dim3((sgemv_ring_threads<ROWS, DMA_WAVES>())), 0, s,
+                     n, m, alpha, a, lda, x, y);
+}
+
+// A row is one chain of multiply-adds whatever the tile, and sixteen rows per compute wavefront are what gives every chain a SIMD of its
+// own; what the rows of a workgroup decide is how long the pieces of a column are that come from memory.  us, ring of 16 / 32 / 64 rows,
+// from the caches and from DRAM:
+//   4096 x 4096   17.2 / 18.4 / 22.5 and 19.5 / 19.9 / 26.9   (one workgroup of 16 rows per compute unit)
+//   6000 x 2048   12.0 / 10.4 / 12.3 and 17.0 / 12.0 / 15.2   8192 x 8192   48 / 44 / 40 and 68 / 50 / 58
+//   9000 x 512    5.4 / 6.0 / 5.8 and 8.5 / 7.8 / 7.1         16384 x 1024  15.3 / 14.7 / 13.7 and 19.3 / 16.4 / 14.3
+// Two stages are over before a wide workgroup has started up: with fewer than 256 columns sixteen rows go further (8209 x 128 3.0 / 3.6 /
+// 3.7 and 3.6 / 3.9 / 4.1).  The ring needs the columns of one stage, and its loads reach sixteen columns by 32-bit lane offsets.
+// Narrower matrices and longer leading dimensions go through small panels, and so do those with more rows than 64 per compute
+// unit: several workgroups then share a compute unit and hide each other's hand-offs (20480 x 4096 64 us, ring of 64 rows 72; 32768 x 4096 85 and
+// 95), and narrow ones from 40 on (12288 x 224 from DRAM 5.7, ring of 16 rows 6.3).
+// From 112 rows on the longer pieces of 128 rows count, in bursts of 64 bytes a thread (64 / 128 rows: 32768 x 2048 42 / 39 us, 98304 x 1024
+// 76 / 72).
 void launch_sgemv_double(hipStream_t s, int n, int m, float alpha, const float* a, int lda, const float* x, float* y)
 {
-  constexpr int kWide = 256, kTall = 128;
-  static_assert(kTall <= kWide, "the line below holds for both panels");
   const int cus = workloads::device_cus();
-  if (n > 112 * cus) launch_sgemv_panels<kGemvCompute, kGemvPanelCols, kGemvDmaPerLd, kGemvMatLds * kGemvDmaPerLd, 64>(s, n, m, alpha, a, lda, x, y);
-  else if (m < kWide || n > 64 * cus) launch_sgemv_panels<64, kGemvPanelCols, 64, 64>(s, n, m, alpha, a, lda, x, y);
-  else if (n <= 16 * cus) launch_sgemv_panels<16, kWide, 64, 128>(s, n, m, alpha, a, lda, x, y);
-  else if (n <= 32 * cus) launch_sgemv_panels<32, kWide, 64, 128>(s, n, m, alpha, a, lda, x, y);
-  else launch_sgemv_panels<64, kTall, 64, 256>(s, n, m, alpha, a, lda, x, y);
+  const bool ring = m >= kSgemvCols && lda <= (0xffffffffLL - 4 * kSgemvRows) / (4 * kSgemvRows) && n <= (m < 2 * kSgemvCols ? 40 : 64) * cus;
+  if (n > 112 * cus) launch_sgemv_small_panels<kGemvCompute, kGemvMatLds * kGemvDmaPerLd, 64>(s, n, m, alpha, a, lda, x, y);
+  else if (!ring) launch_sgemv_small_panels<64, 64>(s, n, m, alpha, a, lda, x, y);
+  else if (n <= 16 * cus || m < 2 * kSgemvCols) launch_sgemv_ring<16, 2>(s, n, m, alpha, a, lda, x, y);
+  else if (n <= 32 * cus) launch_sgemv_ring<32, 2>(s, n, m, alpha, a, lda, x, y);
+  else launch_sgemv_ring<64, 4>(s, n, m, alpha, a, lda, x, y);
 }
 
 // ---- 2-D stencil ----

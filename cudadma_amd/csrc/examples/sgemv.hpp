@@ -9,10 +9,12 @@
 // (cudaDMASequential, cudaDMAStrided of include/cudaDMA.h).
 //
 // The kernels need m to be a multiple of the columns staged per hand-off, except
-// sgemvn_both_double, which takes multiples of 32 from the columns of one panel on.
+// sgemvn_ring, which takes multiples of 32 from 128 on.
 // Where the matrix is staged, lda*4 has to be a multiple of 16 B and fit an int.
 // Rows beyond n are neither read from global memory by compute threads nor written.
 #pragma once
+
+#include <utility>
 
 #include "../../../include/cudaDMA.h"
 
@@ -142,125 +144,239 @@ __global__ void sgemvn_both_single(int n, int m, float alpha, const float* __res
 }
 
 // Vector and matrix panel staged through two buffers each, four objects on
-// disjoint DMA wavefronts.  A workgroup owns ROWS rows; the panels hold COLS columns,
-// and the last one is moved back to end with column m - 1, its columns that were
-// summed before are skipped (m >= COLS, m and COLS multiples of 32).
-//
-// What bounds it: a row's sum is one chain of multiply-adds in ascending column order, 8 cycles each (4096 columns:
-// 14 us), and the wavefront that runs it also issues 12 LDS reads per 16 columns (160 cycles per 16 columns with the LDS to
-// itself, 230 next to the DMA wavefronts).  4096 x 4096: 59 us with panels of 128 rows x 32 columns (32 workgroups,
-// 128 hand-offs), 30 with 16 x 256.  Fewer DMA wavefronts leave too few bytes in flight (one per panel: 40 us).
+// disjoint DMA wavefronts; a compute thread per row.  A workgroup owns ROWS rows, the panels hold COLS columns (m a multiple of
+// COLS).  For narrow matrices and for many rows, where several workgroups share a compute unit and hide each other's hand-offs.
 // Launch with sgemv_both_double_threads<ROWS, VEC_DMA, MAT_DMA>() threads.
-template<int ROWS, int VEC_DMA_THREADS, int MAT_DMA_THREADS>
-constexpr int sgemv_both_double_threads() { return (ROWS < 64 ? 64 : ROWS) + 2 * (VEC_DMA_THREADS + MAT_DMA_THREADS); }
-
-// 16 columns of a panel on their way from LDS to the chain of a compute thread.
-template<int ROWS>
-struct SgemvBlock {
-  float a[16];
-  f32x4_t x[4];
-  __device__ __forceinline__ void load(const float* mat, const float* vec, const int row, const int col)
-  {
-    // one base address per group of columns that the offsets of ds_read2_b32 or ds_read2st64_b32 reach
-    constexpr int kReach = ROWS == 32 ? 8 : 16;
-#pragma unroll
-    for (int g = 0; g < 16; g += kReach) {
-      int base = (col + g) * ROWS + row;
-      asm("" : "+v"(base));
-#pragma unroll
-      for (int j = 0; j < kReach; ++j) a[g + j] = mat[base + j * ROWS];
-    }
-#pragma unroll
-    for (int j = 0; j < 4; ++j) x[j] = *(const f32x4_t*)(vec + col + 4 * j);
-  }
-  __device__ __forceinline__ float chain(float res) const
-  {
-#pragma unroll
-    for (int j = 0; j < 16; ++j) res = __builtin_fmaf(a[j], x[j / 4][j % 4], res);
-    return res;
-  }
-};
-
-// Sums the columns [first, COLS) of a panel; both are multiples of 32.
-// The reads of one block go out back to back under the sums of the other: read and multiply-add in turn issue at
-// half the speed (266 against 160 cycles per 16 columns), and left alone the scheduler reads a block right before it is needed.
-template<int ROWS, int COLS>
-__device__ __forceinline__ float sgemv_panel(const float* mat, const float* vec, const int row, const int first, float res)
-{
-  if constexpr (COLS == 32) {
-    // two blocks are over before a pipeline has filled: the compiler's own order is 5 % faster (16384 x 224: 5.4 -> 5.1 us)
-#pragma unroll
-    for (int j = 0; j < COLS; ++j) res = __builtin_fmaf(mat[j * ROWS + row], vec[j], res);
-    return res;
-  }
-  SgemvBlock<ROWS> even, odd;
-  even.load(mat, vec, row, first);
-  for (int c = first; c < COLS; c += 32) {
-    odd.load(mat, vec, row, c + 16);
-    __builtin_amdgcn_sched_barrier(0);
-    res = even.chain(res);
-    __builtin_amdgcn_sched_barrier(0);
-    even.load(mat, vec, row, c + 32 < COLS ? c + 32 : 0);
-    __builtin_amdgcn_sched_barrier(0);
-    res = odd.chain(res);
-    __builtin_amdgcn_sched_barrier(0);
-  }
-  return res;
-}
+template<int COMPUTE_THREADS, int VEC_DMA_THREADS, int MAT_DMA_THREADS>
+constexpr int sgemv_both_double_threads() { return COMPUTE_THREADS + 2 * (VEC_DMA_THREADS + MAT_DMA_THREADS); }
 
 template<int ROWS, int COLS, int VEC_DMA_THREADS, int MAT_DMA_THREADS, int MAT_BYTES = 4 * ROWS * COLS / MAT_DMA_THREADS>
 __global__ __launch_bounds__((sgemv_both_double_threads<ROWS, VEC_DMA_THREADS, MAT_DMA_THREADS>()))
 void sgemvn_both_double(int n, int m, float alpha, const float* __restrict__ A, int lda, const float* __restrict__ x,
                         float* __restrict__ y)
 {
-  constexpr int kCompute = ROWS < 64 ? 64 : ROWS;       // with fewer rows the rest of the wavefront doubles them
   __shared__ __attribute__((aligned(16))) float buff0[COLS];
   __shared__ __attribute__((aligned(16))) float buff1[COLS];
   __shared__ __attribute__((aligned(16))) float mat0[COLS * ROWS];
   __shared__ __attribute__((aligned(16))) float mat1[COLS * ROWS];
 
-  HIPDMA_ASSERT(m >= COLS && (m % 32) == 0);      // a shorter matrix would have the panel begin before its first column
+  HIPDMA_ASSERT(m >= COLS && (m % COLS) == 0);
   // a thread holds its share of a panel in registers, all of it unless MAT_BYTES says less: the next panel is on its way while this
   // one is read
   typedef cudaDMASequential<true, 16, 4 * COLS, VEC_DMA_THREADS> vec_dma_t;
   typedef CudaDMAStrided<true, 16, MAT_BYTES, 4 * ROWS, MAT_DMA_THREADS, COLS> mat_dma_t;
-  vec_dma_t dma_vec_0(1, kCompute, kCompute);
-  vec_dma_t dma_vec_1(2, kCompute, kCompute + VEC_DMA_THREADS);
-  mat_dma_t dma_mat_0(3, kCompute, kCompute + 2 * VEC_DMA_THREADS, 4 * lda, 4 * ROWS);
-  mat_dma_t dma_mat_1(4, kCompute, kCompute + 2 * VEC_DMA_THREADS + MAT_DMA_THREADS, 4 * lda, 4 * ROWS);
+  vec_dma_t dma_vec_0(1, ROWS, ROWS);
+  vec_dma_t dma_vec_1(2, ROWS, ROWS + VEC_DMA_THREADS);
+  mat_dma_t dma_mat_0(3, ROWS, ROWS + 2 * VEC_DMA_THREADS, 4 * lda, 4 * ROWS);
+  mat_dma_t dma_mat_1(4, ROWS, ROWS + 2 * VEC_DMA_THREADS + MAT_DMA_THREADS, 4 * lda, 4 * ROWS);
 
-  const int panels = (m + COLS - 1) / COLS;
+  const int panels = m / COLS;
   const int row0 = blockIdx.x * ROWS;
-  // first column of panel p
-  auto begin = [&](const int p) { const int c = p * COLS; return c < m - COLS ? c : m - COLS; };
-
-  if (threadIdx.x < kCompute) {
+  auto sum = [&](const float* mat, const float* vec, float res) __attribute__((always_inline)) {
+#pragma unroll
+    for (int j = 0; j < COLS; ++j) res = __builtin_fmaf(mat[j * ROWS + threadIdx.x], vec[j], res);
+    return res;
+  };
+  if (threadIdx.x < ROWS) {
     dma_vec_0.start_async_dma();
     dma_mat_0.start_async_dma();
     if (panels > 1) { dma_vec_1.start_async_dma(); dma_mat_1.start_async_dma(); }
-    const int row = threadIdx.x % ROWS;
     float res = 0.0f;
     for (int p = 0; p < panels; p += 2) {
       dma_vec_0.wait_for_dma_finish();
       dma_mat_0.wait_for_dma_finish();
-      res = sgemv_panel<ROWS, COLS>(mat0, buff0, row, p * COLS - begin(p), res);
+      res = sum(mat0, buff0, res);
       if (p + 2 < panels) { dma_vec_0.start_async_dma(); dma_mat_0.start_async_dma(); }
       if (p + 1 < panels) {
         dma_vec_1.wait_for_dma_finish();
         dma_mat_1.wait_for_dma_finish();
-        res = sgemv_panel<ROWS, COLS>(mat1, buff1, row, (p + 1) * COLS - begin(p + 1), res);
+        res = sum(mat1, buff1, res);
         if (p + 3 < panels) { dma_vec_1.start_async_dma(); dma_mat_1.start_async_dma(); }
       }
     }
-    if (threadIdx.x < ROWS && row0 + row < n) y[row0 + row] = alpha * res;
+    if (row0 + threadIdx.x < n) y[row0 + threadIdx.x] = alpha * res;
   } else if (dma_vec_0.owns_this_thread()) {
-    for (int p = 0; p < panels; p += 2) dma_vec_0.execute_dma(x + begin(p), buff0);
+    for (int p = 0; p < panels; p += 2) dma_vec_0.execute_dma(x + p * COLS, buff0);
   } else if (dma_vec_1.owns_this_thread()) {
-    for (int p = 1; p < panels; p += 2) dma_vec_1.execute_dma(x + begin(p), buff1);
+    for (int p = 1; p < panels; p += 2) dma_vec_1.execute_dma(x + p * COLS, buff1);
   } else if (dma_mat_0.owns_this_thread()) {
-    for (int p = 0; p < panels; p += 2) dma_mat_0.execute_dma(A + row0 + (long long)lda * begin(p), mat0);
+    for (int p = 0; p < panels; p += 2) dma_mat_0.execute_dma(A + row0 + (long long)lda * p * COLS, mat0);
   } else if (dma_mat_1.owns_this_thread()) {
-    for (int p = 1; p < panels; p += 2) dma_mat_1.execute_dma(A + row0 + (long long)lda * begin(p), mat1);
+    for (int p = 1; p < panels; p += 2) dma_mat_1.execute_dma(A + row0 + (long long)lda * p * COLS, mat1);
+  }
+}
+
+// ---- sixteen rows per compute wavefront, a ring of stages of 128 columns ----
+// A row's sum is one chain of multiply-adds in ascending column order, 4.6 cycles each with the operands in registers (4096 columns:
+// 7.9 us), and every LDS request of the wavefront that runs the chain holds it up by about 7.  So the wavefront asks for four columns at a
+// time: its four rows of sixteen lanes hold the same sixteen matrix rows, each a quarter of a stage's columns.  (With a lane per matrix
+// row a request fetches one column, and the chain takes 17 cycles per column with the hand-offs; now 8.)  The quarters are summed
+// one after the other: the lanes of one quarter run their 32 multiply-adds and hand the sums on to the lanes of the next one; what the
+// other lanes compute meanwhile is not used.  The hand-over is one v_permlane16_swap or v_permlane32_swap, for which the quarters lie in the
+// lane rows 0, 1, 3, 2.  The columns are swizzled in LDS: of four that follow each other, a wavefront's sixteen rows lie in four different
+// quarters of the 64 banks.  Lane row h takes columns 4q .. 4q+3 of its quarter in the order that begins with 4q + h, so the four lane
+// rows read four different ones.
+//
+// 4096 x 4096: 31.5 us with a lane per row and two register-staged panels of 256 columns, 17.2 now (19.5 from DRAM); 8192 x 8192 62 and 44;
+// 512 x 16384, whose chain is all there is, 103 and 55.  Matrix instructions would run the same chain (v_mfma_f32_16x16x4_f32 adds its four
+// products in order), at 8.1 cycles a column: no faster than this, hand-offs included.
+constexpr int kSgemvRows = 16, kSgemvQuarter = 32, kSgemvCols = 4 * kSgemvQuarter;
+constexpr int sgemv_lane_row(const int quarter) { return quarter < 2 ? quarter : 5 - quarter; }
+
+template<int ROWS>
+struct SgemvStage {
+  float mat[kSgemvCols * ROWS];
+  float vec[kSgemvCols];
+};
+
+// A stage on its way from LDS to the chain.
+template<int ROWS>
+struct SgemvBlock {
+  float a[kSgemvQuarter];                   // a[4q + i]: column 4q + (i + lane row) % 4 of the quarter
+  f32x4_t x[kSgemvQuarter / 4];
+
+  // where a lane finds its row of column 4q + (i + lane row) % 4 of its quarter, q < 4; sixteen columns on the keys repeat
+  struct Places {
+    int at[4][4], vec;
+    __device__ __forceinline__ Places(const int wave, const int lane)
+    {
+      const int h = lane >> 4, first = (h < 2 ? h : 5 - h) * kSgemvQuarter;
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const int col = 4 * q + ((i + h) & 3), chunk = (wave * kSgemvRows + (lane & 15)) / 4;
+          at[q][i] = (first + col) * ROWS + hipdma::swizzled_chunk(col, chunk, ROWS / 4) * 4 + (lane & 3);
+        }
+      vec = first;
+    }
+  };
+  __device__ __forceinline__ void load(const SgemvStage<ROWS>& stage, const Places& places)
+  {
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const float* p = stage.mat + places.at[q][i];
+        a[4 * q + i] = p[0];
+        a[4 * (q + 4) + i] = p[16 * ROWS];
+      }
+#pragma unroll
+    for (int q = 0; q < kSgemvQuarter / 4; ++q) x[q] = *(const f32x4_t*)(stage.vec + places.vec + 4 * q);
+  }
+  // The quarters from `first` on; on entry and exit the sums are in lane row 0.
+  __device__ __forceinline__ float chain(float res, const int first) const
+  {
+#pragma unroll
+    for (int p = 0; p < 4; ++p) {
+      if (p >= first) {
+#pragma unroll
+        for (int c = 0; c < kSgemvQuarter; ++c)
+          res = __builtin_fmaf(a[(c & ~3) + ((c - sgemv_lane_row(p)) & 3)], x[c / 4][c % 4], res);
+      }
+      const unsigned bits = __float_as_uint(res);
+      // first of the pair: odd lane rows (upper half) take the even ones' (lower half's) values; second: the other way round
+      if (p == 0) res = __uint_as_float(__builtin_amdgcn_permlane16_swap(bits, bits, false, false)[0]);        // lane row 0 -> 1
+      else if (p == 1) res = __uint_as_float(__builtin_amdgcn_permlane32_swap(bits, bits, false, false)[0]);   // 1 -> 3
+      else if (p == 2) res = __uint_as_float(__builtin_amdgcn_permlane16_swap(bits, bits, false, false)[1]);   // 3 -> 2
+      else res = __uint_as_float(__builtin_amdgcn_permlane32_swap(bits, bits, false, false)[1]);               // 2 -> 0
+    }
+    return res;
+  }
+};
+
+template<typename IDS> struct SgemvGuards;
+template<int... ID>
+struct SgemvGuards<std::integer_sequence<int, ID...>> {
+  cudaDMACustom of[sizeof...(ID)];
+  __device__ __forceinline__ SgemvGuards(const int dma_threads, const int compute_threads)
+    : of{cudaDMACustom(ID, dma_threads, compute_threads, compute_threads)...} {}
+};
+
+// ROWS rows per workgroup, one compute wavefront for sixteen of them; DMA wavefronts that share the columns of a stage.  Two of the four
+// stages are on their way, by direct-to-LDS loads, which hold no registers; the third is read, the fourth waits to be: with three on their way a
+// DMA wavefront waits for a stage to be given back before it reports the next one (2048 x 8192 30.0 -> 38 us), and more stages gain
+// nothing (six, three on their way: 31).  A DMA wavefront gets rid of a 1 KB load every 50 ns, so one of them alone holds the chain up (32
+// rows: 2048 x 8192 61 us, two 31).
+// The last stage is moved back to end with column m - 1; its columns that were summed before are skipped (m >= 128, a multiple of 32).
+template<int ROWS, int DMA_WAVES> constexpr int sgemv_ring_threads() { return 64 * (ROWS / kSgemvRows + DMA_WAVES); }
+template<int ROWS, int DMA_WAVES>
+__global__ __launch_bounds__((sgemv_ring_threads<ROWS, DMA_WAVES>()))
+void sgemvn_ring(int n, int m, float alpha, const float* __restrict__ A, int lda, const float* __restrict__ x, float* __restrict__ y)
+{
+  constexpr int kStages = 4, kAhead = 2, kCompute = 64 * (ROWS / kSgemvRows), kCols = kSgemvCols / DMA_WAVES;
+  static_assert(kAhead < kStages, "a stage is requested when the one before it in its place has long been read");
+  __shared__ __attribute__((aligned(1024))) SgemvStage<ROWS> ring[kStages];
+  typedef CudaDMAStrided<false, 16, 16, 4 * ROWS, 64, kCols> mat_dma_t;
+  typedef CudaDMAStrided<false, 16, 16, 4 * kCols, 64, 1> vec_dma_t;
+  constexpr int kLoads = mat_dma_t::loads_per_thread() + vec_dma_t::loads_per_thread();
+  static_assert(kLoads * kAhead <= 63, "loads in flight that a wavefront can count");
+  HIPDMA_ASSERT(m >= kSgemvCols && (m % kSgemvQuarter) == 0);      // a shorter matrix would have the stage begin before its first column
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int dma = wave < kCompute / 64 ? 0 : wave - kCompute / 64;           // number among the DMA wavefronts
+  mat_dma_t dma_mat(4 * lda, 4 * ROWS, kCompute + 64 * dma);
+  vec_dma_t dma_vec(4 * kCols, 4 * kCols, kCompute + 64 * dma);
+  SgemvGuards<std::make_integer_sequence<int, kStages>> guards(64 * DMA_WAVES, kCompute);
+  auto& guard = guards.of;
+
+  const int blocks = (m + kSgemvCols - 1) / kSgemvCols;
+  // workgroup b runs on XCD b % 8: every XCD gets a run of row tiles, whose pieces of a column share cache lines and pages with their
+  // neighbours; pieces of 256 B are left dealt out (16384 x 16384 184 us, in runs 192)
+  const int xcd = blockIdx.x & 7, each = gridDim.x >> 3, more = gridDim.x & 7;
+  const int row0 = (ROWS >= 64 ? (int)blockIdx.x : xcd * each + (xcd < more ? xcd : more) + (int)(blockIdx.x >> 3)) * ROWS;
+  auto begin = [&](const int b) { const int c = b * kSgemvCols; return c < m - kSgemvCols ? c : m - kSgemvCols; };
+
+  if (wave >= kCompute / 64) {
+    auto issue = [&](const int b, const int at) __attribute__((always_inline)) {
+      const int col = begin(b) + dma * kCols;
+      if (b >= kStages) guard[at].wait_for_dma_start_direct();       // the stages are empty to begin with
+      dma_vec.template issue_direct_part<STORE_LDS_DIRECT, true>(x + col, ring[at].vec + dma * kCols, 0, 1);
+      dma_mat.template issue_direct_part<STORE_LDS_DIRECT_SWIZZLE, true>(A + row0 + (long long)lda * col, ring[at].mat + dma * kCols * ROWS, 0, kLoads - 1);
+    };
+#pragma unroll
+    for (int b = 0; b < kAhead; ++b)
+      if (b < blocks) issue(b, b);
+    auto land = [&](const int b, const int at) __attribute__((always_inline)) {
+      if (b >= blocks) return;
+      if (b + kAhead <= blocks) hipdma::wait_direct_loads<(kAhead - 1) * kLoads>();
+      else hipdma::wait_direct_loads<0>();
+      guard[at].finish_async_dma_direct();
+      if (b + kAhead < blocks) issue(b + kAhead, (at + kAhead) % kStages);
+    };
+    for (int b = 0; b < blocks; b += kStages) {
+#pragma unroll
+      for (int i = 0; i < kStages; ++i) land(b + i, i);
+    }
+  } else {
+    const typename SgemvBlock<ROWS>::Places places(wave, lane);
+    SgemvBlock<ROWS> even, odd;
+    float res = 0.0f;
+    guard[0].wait_for_dma_finish();
+    even.load(ring[0], places);
+    unsigned seen = guard[1].peek_dma_finish();
+    // Block b, in `cur`.  The requests of the next one go out back to back before the chain: in turn with its multiply-adds they
+    // take half as long again.
+    auto step = [&](const int b, const int at, SgemvBlock<ROWS>& cur, SgemvBlock<ROWS>& next) __attribute__((always_inline)) {
+      if (b >= blocks) return;
+      guard[at].start_async_dma();        // waits for the requests of `cur`: their stage may be filled again
+      if (b + 1 < blocks) {
+        guard[(at + 1) % kStages].wait_for_dma_finish(seen);
+        next.load(ring[(at + 1) % kStages], places);
+        seen = guard[(at + 2) % kStages].peek_dma_finish();
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      res = cur.chain(res, (b * kSgemvCols - begin(b)) / kSgemvQuarter);
+      __builtin_amdgcn_sched_barrier(0);
+    };
+    for (int b = 0; b < blocks; b += kStages) {
+#pragma unroll
+      for (int i = 0; i < kStages; i += 2) {
+        step(b + i, i, even, odd);
+        step(b + i + 1, i + 1, odd, even);
+      }
+    }
+    const int row = row0 + wave * kSgemvRows + lane;
+    if (lane < kSgemvRows && row < n) y[row] = alpha * res;
   }
 }
 

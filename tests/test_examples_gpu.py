@@ -107,9 +107,50 @@ def test_sgemv_panels(dev, n, m):
     assert np.all(got[n:] == 3.0)
 
 
+# the ring of stages: rows around the lines between its workgroups of 16, 32 and 64 rows, with and without a last stage that moves
+# back, by one to three quarters, and one to six stages of the four; and what leaves it (fewer columns, more rows)
+@pytest.mark.parametrize("n", [16, 4096, 4112, 8192, 8193, 10240, 10241, 16384, 16385])
+@pytest.mark.parametrize("m", [96, 128, 160, 192, 352, 512, 640, 736])
+def test_sgemv_ring(dev, n, m):
+    O = ol.load()
+    lda = (n + 127) // 128 * 128
+    a = ol.uniform(m * lda, 27).reshape(m, lda)
+    x = ol.uniform(m, 28)
+    want = np.empty(n, dtype=np.float32)
+    O.oracle_sgemv(n, m, 0.5, ptr(a), lda, ptr(x), ptr(want))
+    dy = torch.full((lda,), 3.0, dtype=torch.float32, device=dev)
+    ex.sgemv(0.5, torch.from_numpy(a).to(dev), torch.from_numpy(x).to(dev), dy, n=n)
+    torch.cuda.synchronize()
+    got = dy.cpu().numpy()
+    assert np.array_equal(got[:n], want)
+    assert np.all(got[n:] == 3.0)
+
+
+def test_sgemv_special_values(dev):
+    """Infinities and NaN stay in their rows (lanes that sum other columns of the same rows meanwhile see them too), zeros keep
+    their sign through alpha, and denormal products count."""
+    n, m = 48, 416
+    O = ol.load()
+    a = ol.uniform(m * 128, 29).reshape(m, 128)
+    x = ol.uniform(m, 30)
+    a[[0, 33, 70, 127, 128, 300, 415], [1, 2, 3, 4, 5, 6, 7]] = [np.inf, -np.inf, np.nan, np.inf, np.nan, -np.inf, np.inf]
+    a[40, 1] = -np.sign(x[40] * x[0]) * np.inf              # inf - inf
+    a[:, 8] = 0.0
+    a[:, 9] *= np.float32(2.0 ** -126)
+    a[:, 10] = -0.0
+    want = np.empty(n, dtype=np.float32)
+    O.oracle_sgemv(n, m, -1.0, ptr(a), 128, ptr(x), ptr(want))
+    dy = torch.zeros(128, dtype=torch.float32, device=dev)
+    ex.sgemv(-1.0, torch.from_numpy(a).to(dev), torch.from_numpy(x).to(dev), dy, n=n)
+    got = dy.cpu().numpy()[:n]
+    nan = np.isnan(want)
+    assert nan.sum() >= 3 and np.array_equal(np.isnan(got), nan)
+    assert np.array_equal(got[~nan].view(np.uint32), want[~nan].view(np.uint32))
+
+
 # a leading dimension far beyond what n needs: the columns of one panel lie more than 2 GiB apart (256, 128 and 32 columns)
 @pytest.mark.parametrize("n,m,lda,variant", [(16, 256, 2_200_064, 3), (4160, 288, 2_200_064, 3), (8200, 288, 4_300_032, 3), (40, 32, 17_400_064, 3),
-                                             (40, 32, 17_400_064, 2), (40, 256, 17_400_064, 3)])
+                                             (40, 32, 17_400_064, 2), (40, 256, 17_400_064, 3), (40, 128, 67_108_860, 3), (40, 128, 67_108_864, 3)])
 def test_sgemv_columns_far_apart(dev, n, m, lda, variant):
     O = ol.load()
     pad = (n + 127) // 128 * 128
