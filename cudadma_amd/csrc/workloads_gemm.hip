@@ -67,7 +67,10 @@ __device__ __forceinline__ void tile_of_workgroup(const int b, const int tiles_m
 
 // The order in which the workgroups take the tiles; `per_cu` of them share a compute unit.  Every XCD has an L2 of its own, so the panels
 // of A and B behind the tiles that are in work on one XCD at a time should be few.
-//   blocks     grids that divide into 4 x 2: every XCD gets one compact block.
+//   blocks     grids that divide into 4 x 2: every XCD gets one compact block.  Not where the blocks are narrow strips with half as many panels
+//              again as a band's share (128 x 128 tiles, us in blocks and in bands, from the caches and from DRAM: 512 x 16384 x 1024 28.2 / 22.3 and
+//              32.6 / 27.4; 1024 x 6144 x 2048 32.1 / 28.7 and 41.6 / 34.8; 512 x 8192 x 4096 43.5 / 41.0 and 46.2 / 44.3); with few K steps it is the writes of C
+//              that count (1024 x 16384 x 256, variant 1: 22.1 / 24.3).
 //   bands      up to eight tile rows, down the columns of a band, an eighth of that walk for every XCD (dealt row-major instead:
 //              3712 x 4736 x 3712 with 128 x 128 tiles 188 us against 139, 640 x 8064 x 2048 34 / 28).  In grids that divide level or slower than
 //              blocks (8192 x 8192 x 1024, 256 x 256 tiles: 155 us against 140).
@@ -81,11 +84,13 @@ __device__ __forceinline__ void tile_of_workgroup(const int b, const int tiles_m
 int tile_walk(const int m, const int n, const int k, const int tile_rows, const int tile_cols, const int per_cu)
 {
   const int tiles_m = m / tile_rows, tiles_n = n / tile_cols;
-  if ((tiles_m % 4) == 0 && (tiles_n % 2) == 0) return kWalkBlocks;
   const int cus = workloads::device_cus();
   const long long tiles = (long long)tiles_m * tiles_n, each = tiles / 8;
   int rows = 1;
   while (rows < 8 && rows * rows < each) ++rows;
+  const int high = tiles_m < rows ? tiles_m : rows;
+  const bool narrow = k >= 512 && tiles_m / 4 + tiles_n / 2 > 3 * (high + each / high) / 2;      // panels behind a block and behind a band's share
+  if ((tiles_m % 4) == 0 && (tiles_n % 2) == 0 && !narrow) return kWalkBlocks;
   const double in_work = (double)(each < per_cu * cus / 8 ? each : per_cu * cus / 8), columns = tiles_n / 8;
   const bool own_columns = (tiles_n % 8) == 0 && in_work / columns + columns <= rows + in_work / rows + 1;
   const bool mostly_c = k < 256 && (long long)n * k < (3 << 19) && (long long)m * n >= (16 << 20);
