@@ -22,6 +22,7 @@ namespace {
 
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x4_t __attribute__((ext_vector_type(4)));
+typedef float f32x4_t __attribute__((ext_vector_type(4)));
 typedef float f32x16_t __attribute__((ext_vector_type(16)));
 
 constexpr int kBK = 64;
@@ -70,7 +71,7 @@ __device__ __forceinline__ void tile_of_workgroup(const int b, const int tiles_m
 //   blocks     grids that divide into 4 x 2: every XCD gets one compact block.  Not where the blocks are narrow strips with half as many panels
 //              again as a band's share (128 x 128 tiles, us in blocks and in bands, from the caches and from DRAM: 512 x 16384 x 1024 28.2 / 22.3 and
 //              32.6 / 27.4; 1024 x 6144 x 2048 32.1 / 28.7 and 41.6 / 34.8; 512 x 8192 x 4096 43.5 / 41.0 and 46.2 / 44.3); with few K steps it is the writes of C
-//              that count (1024 x 16384 x 256, variant 1: 22.1 / 24.3).
+//              that count (1024 x 16384 x 256, variant 1: 22.1 / 24.3), though not with tiles below 128 x 128 (256 x 5376 x 256 from DRAM 6.3 / 5.7).
 //   bands      up to eight tile rows, down the columns of a band, an eighth of that walk for every XCD (dealt row-major instead:
 //              3712 x 4736 x 3712 with 128 x 128 tiles 188 us against 139, 640 x 8064 x 2048 34 / 28).  In grids that divide level or slower than
 //              blocks (8192 x 8192 x 1024, 256 x 256 tiles: 155 us against 140).
@@ -89,7 +90,7 @@ int tile_walk(const int m, const int n, const int k, const int tile_rows, const 
   int rows = 1;
   while (rows < 8 && rows * rows < each) ++rows;
   const int high = tiles_m < rows ? tiles_m : rows;
-  const bool narrow = k >= 512 && tiles_m / 4 + tiles_n / 2 > 3 * (high + each / high) / 2;      // panels behind a block and behind a band's share
+  const bool narrow = (k >= 512 || tile_rows < 128) && tiles_m / 4 + tiles_n / 2 > 3 * (high + each / high) / 2;      // panels behind a block and behind a band's share
   if ((tiles_m % 4) == 0 && (tiles_n % 2) == 0 && !narrow) return kWalkBlocks;
   const double in_work = (double)(each < per_cu * cus / 8 ? each : per_cu * cus / 8), columns = tiles_n / 8;
   const bool own_columns = (tiles_n % 8) == 0 && in_work / columns + columns <= rows + in_work / rows + 1;
@@ -1143,6 +1144,169 @@ gemm_bf16_all_direct_a64(const unsigned short* __restrict__ a, const unsigned sh
       }
 }
 
+// ---- small grids: the K steps dealt out to the wavefronts of a workgroup ----
+// A grid of few tiles leaves compute units idle, and a product of few rows and columns is one long chain of K steps per tile.  Here the tile
+// is 32 * WI x 32 * WJ, every one of the WAVES wavefronts holds all of it, and wavefront w takes the K steps (of 64) w, w + WAVES, ...  A
+// wavefront brings its own operands with direct-to-LDS loads into a stage of its own and is the only one to read them, so nothing in the loop
+// waits for another wavefront: no barrier, no hand-off, s_waitcnt alone.  It takes a whole stage into registers, and while it multiplies
+// it the next one is on its way into the same place.  At the end the partial tiles are added through LDS.
+// What bounds the loop is the LDS: direct loads land at about 100 B a cycle, fragments are read at 128, and the two share it.  32 x 32 takes 70
+// cycles per K = 32, 64 x 64 takes 126 to 144, against 434 of a 128 x 128 tile with four wavefronts, which is 4 to 16 times the work.
+// Measured (us, former choice -> this, from the caches and from DRAM): 512^3 6.0 -> 3.5 and 7.2 -> 4.0; 128 x 128 x 8192 48.7 -> 9.9 and 48.9 ->
+// 16.6; 1024^3 9.2 -> 6.2 and 10.1 -> 7.3; 2560 x 384 x 6528 40.7 -> 22.4 and 60 -> 28.
+// Stages of K = 32, two per wavefront, read A in pieces of 64 B, half a cache line: 1024 x 1024 x 4096 18.5 us, 16.4 so.  Four wavefronts with four
+// such stages 18.9.  Tiles of 64 x 128 the same way start and end too slowly (1408^3 11.8 against 11.3 with 64 x 64).
+template<int WI, int WJ, int WAVES>
+__global__ void __launch_bounds__(64 * WAVES)
+gemm_bf16_dealt_steps(const unsigned short* __restrict__ a, const unsigned short* __restrict__ b, float* __restrict__ c,
+                      const int m, const int n, const int k, const int walk)
+{
+  constexpr int kSlices = 4, kStepK = 16 * kSlices, kBM = 32 * WI, kBN = 32 * WJ;
+  constexpr int kARow = 2 * kStepK, kBRow = 2 * kBN;
+  constexpr int kAStage = kBM * kARow, kStage = kAStage + kStepK * kBRow;
+  typedef CudaDMAStrided<false, 16, 16, kARow, 64, kBM> dma_a_t;
+  typedef CudaDMAStrided<false, 16, 16, kBRow, 64, kStepK> dma_b_t;
+  constexpr int kALoads = dma_a_t::loads_per_thread(), kLoads = kALoads + dma_b_t::loads_per_thread();
+  constexpr int kProducts = WI * WJ;                               // per slice of 16
+  constexpr int kShare = 16 * kProducts / WAVES;                   // accumulators that a wavefront adds up and stores in the end
+  __shared__ __attribute__((aligned(1024))) char lds[WAVES * kStage];
+  static_assert(kProducts * 4096 <= kStage, "a partial tile takes the place of a stage");
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  dma_a_t dma_a(k * 2, kARow, 64 * wave);
+  dma_b_t dma_b(n * 2, kBRow, 64 * wave);
+  int tile_m, tile_n;
+  tile_of_workgroup(blockIdx.x, m / kBM, n / kBN, walk, tile_m, tile_n);
+  const int all_steps = k / kStepK;
+  const int steps = (all_steps - wave + WAVES - 1) / WAVES;        // of this wavefront
+  const unsigned short* next_a = a + (size_t)tile_m * kBM * k + wave * kStepK;      // the stage to request next
+  const unsigned short* next_b = b + (size_t)tile_n * kBN + (size_t)wave * kStepK * n;
+  const size_t step_b = (size_t)WAVES * kStepK * n;
+  // as an LDS address: a generic one would be compared with null at every load
+  char* const stage = (char*)((HIPDMA_LDS_AS char*)lds + wave * kStage);
+  auto issue = [&](const int g) __attribute__((always_inline)) {
+    if (g < kALoads) dma_a.template issue_direct_part<STORE_LDS_DIRECT_SWIZZLE, true>(next_a, stage, g, 1);
+    else dma_b.template issue_direct_part<STORE_LDS_DIRECT_SWIZZLE, true>(next_b, stage + kAStage, g - kALoads, 1);
+    if (g == kLoads - 1) {
+      next_a += WAVES * kStepK; next_b += step_b;
+      asm("" : "+s"(next_a));               // kept in scalar registers
+      asm("" : "+s"(next_b));
+    }
+  };
+  f32x16_t acc[WI][WJ];
+#pragma unroll
+  for (int i = 0; i < WI; ++i)
+#pragma unroll
+    for (int j = 0; j < WJ; ++j)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.0f;
+  int a_lane[kSlices], b_lo[WJ], b_hi[WJ];
+  {
+    const int row = lane & 31;
+#pragma unroll
+    for (int ks = 0; ks < kSlices; ++ks) a_lane[ks] = row * kARow + hipdma::swizzled_chunk(row, 2 * ks + (lane >> 5), kARow / 16) * 16;
+  }
+  {
+    const int j16 = lane & 15;
+    const int row = (lane >> 5) * 8 + (j16 >> 2);
+#pragma unroll
+    for (int j = 0; j < WJ; ++j) {
+      const int col_bytes = (j * 32 + ((lane >> 4) & 1) * 16 + (j16 & 3) * 4) * 2;
+      b_lo[j] = kAStage + row * kBRow + hipdma::swizzled_chunk(row, col_bytes >> 4, kBRow / 16) * 16 + (col_bytes & 15);
+      b_hi[j] = kAStage + (row + 4) * kBRow + hipdma::swizzled_chunk(row + 4, col_bytes >> 4, kBRow / 16) * 16 + (col_bytes & 15);
+    }
+  }
+  bf16x8_t fa[kSlices][WI], fb[kSlices][WJ];
+  auto load_frags = [&]() __attribute__((always_inline)) {
+#pragma unroll
+    for (int ks = 0; ks < kSlices; ++ks) {
+#pragma unroll
+      for (int i = 0; i < WI; ++i) fa[ks][i] = *(const bf16x8_t*)(stage + i * 32 * kARow + a_lane[ks]);
+#pragma unroll
+      for (int j = 0; j < WJ; ++j) {
+        const bf16x4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((__attribute__((address_space(3))) bf16x4_t*)(stage + ks * 16 * kBRow + b_lo[j]));
+        const bf16x4_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((__attribute__((address_space(3))) bf16x4_t*)(stage + ks * 16 * kBRow + b_hi[j]));
+        fb[ks][j] = bf16x8_t{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+      }
+    }
+  };
+  // The products of a stage, with `more` the loads of the next one spread behind them.
+  auto multiply = [&](auto more) __attribute__((always_inline)) {
+    constexpr int kAll = kSlices * kProducts, kEach = (kLoads + kAll - 1) / kAll;      // loads behind a product
+#pragma unroll
+    for (int p = 0; p < kAll; ++p) {
+      const int ks = p / kProducts, i = p % kProducts / WJ, j = p % WJ;
+      acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[ks][i], fb[ks][j], acc[i][j], 0, 0, 0);
+      __builtin_amdgcn_sched_barrier(0);
+      if constexpr (decltype(more)::value) {
+#pragma unroll
+        for (int g = p * kEach; g < (p + 1) * kEach && g < kLoads; ++g) issue(g);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  };
+  if (steps > 0) {
+#pragma unroll
+    for (int g = 0; g < kLoads; ++g) issue(g);
+    hipdma::wait_direct_loads<0>();
+    load_frags();
+    for (int t = 1; t < steps; ++t) {
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");           // the stage has been read: the next one may land
+      multiply(std::true_type());
+      hipdma::wait_direct_loads<0>();
+      load_frags();
+    }
+    multiply(std::false_type());
+  }
+  // The accumulators go to LDS as they lie in the registers; every wavefront then adds up kShare of them, in the order of the wavefronts,
+  // and stores those.  Wavefronts beyond the K steps have nothing to add.
+  const int active = all_steps < WAVES ? all_steps : WAVES;
+  constexpr int kPiece = kShare % 4 == 0 ? 4 : 2;                  // accumulators of one LDS access
+  typedef float piece_t __attribute__((ext_vector_type(kPiece)));
+  constexpr int kPieces = 16 * kProducts / kPiece;
+  auto piece_of = [&](const int partial, const int q) __attribute__((always_inline)) {
+    return (piece_t*)(lds + ((partial * kPieces + q) * 64 + lane) * sizeof(piece_t));
+  };
+  __syncthreads();                          // the stages are no longer read
+  if (wave < active) {
+#pragma unroll
+    for (int q = 0; q < kPieces; ++q) {
+      piece_t v;
+#pragma unroll
+      for (int e = 0; e < kPiece; ++e) v[e] = acc[q * kPiece / 16 / WJ][q * kPiece / 16 % WJ][q * kPiece % 16 + e];
+      *piece_of(wave, q) = v;
+    }
+  }
+  __syncthreads();
+  piece_t sum[kShare / kPiece];
+#pragma unroll
+  for (int q = 0; q < kShare / kPiece; ++q) sum[q] = *piece_of(0, wave * (kShare / kPiece) + q);
+#pragma unroll
+  for (int w = 1; w < WAVES; ++w)
+    if (w < active) {
+#pragma unroll
+      for (int q = 0; q < kShare / kPiece; ++q) sum[q] += *piece_of(w, wave * (kShare / kPiece) + q);
+    }
+  float* const cbase = c + (size_t)tile_m * kBM * n + (size_t)tile_n * kBN;
+#pragma unroll
+  for (int q = 0; q < kShare / kPiece; ++q)
+#pragma unroll
+    for (int e = 0; e < kPiece; ++e) {
+      const int at = wave * kShare + q * kPiece + e, block = at / 16, reg = at % 16;
+      const int row = block / WJ * 32 + 8 * (reg / 4) + 4 * (lane >> 5) + reg % 4, col = block % WJ * 32 + (lane & 31);
+      __builtin_nontemporal_store(sum[q][e], &cbase[(size_t)row * n + col]);
+    }
+}
+
+template<int WI, int WJ, int WAVES>
+int launch_dealt_steps(const uint16_t* d_a, const uint16_t* d_b, float* d_c, int m, int n, int k, hipStream_t stream)
+{
+  constexpr int kPerCu = 2 * WAVES * (WI + WJ) * 4096 <= (160 << 10) ? 2 : 1;
+  hipLaunchKernelGGL((gemm_bf16_dealt_steps<WI, WJ, WAVES>), dim3((unsigned)((m / (32 * WI)) * (n / (32 * WJ)))), dim3(64 * WAVES), 0, stream,
+                     d_a, d_b, d_c, m, n, k, tile_walk(m, n, k, 32 * WI, 32 * WJ, kPerCu));
+  CUDADMA_HIP_CHECK(hipGetLastError());
+  return CUDADMA_OK;
+}
+
 template<int WI, int WJ, int WM = 2, int WN = 2>
 int launch_gemm(const uint16_t* d_a, const uint16_t* d_b, float* d_c, int m, int n, int k, hipStream_t stream)
 {
@@ -1195,7 +1359,16 @@ extern "C" int cudadma_gemm_bf16(const uint16_t* d_a, const uint16_t* d_b, float
     };
     const long long small = rounds((long long)(m / 128) * (n / 128), 2 * cus, cus, 100, 58, 400);
     const bool even = (m % 256) == 0 && (n % 256) == 0;
+    // Grids of few tiles take the smallest tile that still gives every compute unit at most one (32 x 32, 32 x 64, 64 x 64) or, with half as
+    // many wavefronts, two workgroups (64 x 64).  us with those four and with 128 x 128, from the caches: 512 x 512 x 512 3.5 / 3.7 / 4.6 / 4.6 / 6.0;
+    // 640 x 512 x 1152 6.0 / 4.8 / 6.0 / 6.4 / 9.8; 768^3 6.7 / 7.0 / 5.3 / 5.5 / 7.8; 1024 x 1152 x 1920 - / - / 15.2 / 12.6 / 14.8 and from DRAM
+    // 17.0 / 14.8 / 20.4.  The last one gains 4 % from the caches (30 shapes; least 0.95, 384 x 4864 x 256 5.0 -> 5.3) and 15 % from DRAM.
+    const long long t32 = (long long)(m / 32) * (n / 32);
     if (!direct_rows_fit(n, k)) variant = 1;
+    else if (t32 <= cus) return launch_dealt_steps<1, 1, 8>(d_a, d_b, d_c, m, n, k, s);
+    else if (t32 <= 2 * cus) return launch_dealt_steps<1, 2, 8>(d_a, d_b, d_c, m, n, k, s);
+    else if (t32 <= 4 * cus) return launch_dealt_steps<2, 2, 8>(d_a, d_b, d_c, m, n, k, s);
+    else if (t32 <= 8 * cus) return launch_dealt_steps<2, 2, 4>(d_a, d_b, d_c, m, n, k, s);
     else if (even && rounds((long long)(m / 256) * (n / 256), cus, cus * 5 / 8, 160, 110, 1000) < small) variant = 9;
     else {
       const long long grid = (long long)(m / 128) * (n / 128);

@@ -178,7 +178,8 @@ int cudadma_halo_stencil(const float* d_in, float* d_out, int nx, int ny, int nz
  * float, fp32 accumulation on the matrix cores.  m, n and k multiples of 128.
  * In the warp-specialised variants four DMA wavefronts stage the A and B tiles of one K step
  * through CudaDMAStrided and four or eight compute wavefronts multiply.  variant 0 picks variant 9 or its
- * kernel with a tile of 128 x 128, whichever takes less time for the problem's tiles; 1: 128 x 128; 2: 128 x 256 (n a multiple of
+ * kernel with a tile of 128 x 128, whichever takes less time for the problem's tiles, and for few tiles smaller ones whose
+ * wavefronts share the K steps and add their partial sums; 1: 128 x 128; 2: 128 x 256 (n a multiple of
  * 256); 3: 256 x 128 (m a multiple of 256); 4: 256 x 128 with the tiles brought in by
  * global_load_lds into swizzled LDS rows; 5: 256 x 256 with eight compute wavefronts (m and n
  * multiples of 256); 6: the same tile with K steps of 32 brought into four swizzled LDS stages by

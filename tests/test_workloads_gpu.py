@@ -583,6 +583,21 @@ def test_gemm_stages(device, m, n, k):
     assert bool(((got - want).abs() <= k * 2.0 ** -23 * size).all())      # k additions of 2^-24 each, the products exact in fp32, doubled
 
 
+# small grids of the default variant, whose wavefronts take K steps of 64 in turn: both sides of the lines between its tiles (32 x 32, 32 x 64,
+# 64 x 64 with eight and with four wavefronts, then 128 x 128) on 256 compute units, fewer K steps than wavefronts, as many, and a remainder
+@pytest.mark.parametrize("m, n", [(128, 128), (512, 512), (640, 512), (512, 1024), (1152, 512), (1024, 1024), (128, 8320), (2048, 1024), (2176, 1024)])
+@pytest.mark.parametrize("k", [128, 256, 384, 512, 640, 1152])
+def test_gemm_dealt_steps(device, m, n, k):
+    a = wl.fill_normal_bf16(torch.empty((m, k), dtype=torch.bfloat16, device=device), 65)
+    b = wl.fill_normal_bf16(torch.empty((k, n), dtype=torch.bfloat16, device=device), 66)
+    buf = torch.full((m * n + 256,), float("nan"), device=device)
+    buf[m * n:] = 7.0
+    got = wl.gemm_bf16(a, b, buf[:m * n].view(m, n))
+    want, size = a.double() @ b.double(), a.double().abs() @ b.double().abs()
+    assert bool(((got - want).abs() <= k * 2.0 ** -23 * size).all())      # k additions of 2^-24 each, the products exact in fp32, doubled
+    assert bool((buf[m * n:] == 7.0).all())
+
+
 def test_gemm_long_rows(device):
     """Rows of A so long that those of one transfer lie more than 2 GiB apart, where the default variant leaves its 32-bit lane offsets;
     a few columns hold small whole numbers, so the product is exact."""
