@@ -94,8 +94,8 @@ static const VariantInfo kStrided[] = {
    "workgroup per compute unit"},
 };
 static const VariantInfo kGather[] = {
-  {"the library's choice: variant 1 for up to 32 MiB of records, else variant 6 (two objects, "
-   "index words requested one transfer ahead)"},
+  {"the library's choice: copies variant 1 for up to 32 MiB of records, else variant 6 (two objects, index words requested one "
+   "transfer ahead); row sums variant 1 for up to 14 MiB, else one object with four tiles in a transfer, index words ahead"},
   {"single buffer: one object, execute_dma"},
   {"manual double buffer: one DMA group of 2 wavefronts, two CudaDMAIndirect objects, each transfer fetches its own index words"},
   {"manual 4-stage buffering: four objects, each transfer fetches its own index words"},

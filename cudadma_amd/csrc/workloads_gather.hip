@@ -16,57 +16,68 @@ constexpr int kRecsPerTile = 32;
 constexpr int kTileBytes = kRecBytes * kRecsPerTile;     // 4 KiB
 constexpr int kDmaThreads = 128;
 constexpr int kComputeThreads = 128;
-constexpr int kBytesPerThread = kTileBytes / kDmaThreads;   // 32: two dwordx4 per DMA thread, one step
 
-typedef CudaDMAIndirect<true, true, 16, kBytesPerThread, kRecBytes, kDmaThreads, kRecsPerTile> dma_t;
+// TILES tiles in one transfer: 32 B per DMA thread for each, all in one step
+template<int TILES>
+using dma_of = CudaDMAIndirect<true, true, 16, TILES * kTileBytes / kDmaThreads, kRecBytes, kDmaThreads, TILES * kRecsPerTile>;
+typedef dma_of<1> dma_t;
 
 struct CopyConsumer {
   static constexpr bool kWritesEveryRecord = true;
-  static __device__ __forceinline__ void run(const char* lds_tile, float* __restrict__ out, const long long tile,
-                                             const dma_t& dma)
+  template<int TILES>
+  static __device__ __forceinline__ void run(const char* lds_tiles, float* __restrict__ out, const long long tile, const dma_of<TILES>& dma)
   {
-    vec4_t v[2];
-    const vec4_t* src = (const vec4_t*)lds_tile;
-    v[0] = src[threadIdx.x];
-    v[1] = src[threadIdx.x + kComputeThreads];
+    constexpr int kEach = TILES * kTileBytes / 16 / kComputeThreads;
+    vec4_t v[kEach];
+    const vec4_t* src = (const vec4_t*)lds_tiles;
+#pragma unroll
+    for (int i = 0; i < kEach; ++i) v[i] = src[threadIdx.x + i * kComputeThreads];
     dma.start_async_dma();
     // Non-temporal: the records written are not read again, and lines of them would push those of the table out of the L2 (us, plain /
     // non-temporal: 6 Mi records from a table of 24000 248 / 136, 24000 x 512 Ki from DRAM 23 / 15; 8 Mi from one of 4 Mi 367 / 319).
     vec4_t* dst = (vec4_t*)(out + tile * (kTileBytes / 4));
-    __builtin_nontemporal_store(v[0], &dst[threadIdx.x]);
-    __builtin_nontemporal_store(v[1], &dst[threadIdx.x + kComputeThreads]);
+#pragma unroll
+    for (int i = 0; i < kEach; ++i) {
+      __builtin_nontemporal_store(v[i], &dst[threadIdx.x + i * kComputeThreads]);
+    }
   }
 };
 
 struct RowsumConsumer {
   static constexpr bool kWritesEveryRecord = false;
-  static __device__ __forceinline__ void run(const char* lds_tile, float* __restrict__ out, const long long tile,
-                                             const dma_t& dma)
+  template<int TILES>
+  static __device__ __forceinline__ void run(const char* lds_tiles, float* __restrict__ out, const long long tile, const dma_of<TILES>& dma)
   {
-    // 32 sums per tile: the first 32 compute threads each add one word of every record, record 0 first
-    const float* t = (const float*)lds_tile;
+    static_assert(TILES * kRecFloats <= kComputeThreads, "a sum per compute thread");
+    // 32 sums per tile: the first 32 compute threads each add one word of every record, record 0 first; the next 32 those of the next tile
+    const float* t = (const float*)lds_tiles + threadIdx.x / kRecFloats * (kTileBytes / 4) + threadIdx.x % kRecFloats;
     float acc = 0.0f;
-    if (threadIdx.x < kRecFloats) {
-      acc = t[threadIdx.x];
+    if (threadIdx.x < TILES * kRecFloats) {
+      acc = t[0];
 #pragma unroll
-      for (int r = 1; r < kRecsPerTile; ++r) acc = acc + t[r * kRecFloats + threadIdx.x];
+      for (int r = 1; r < kRecsPerTile; ++r) acc = acc + t[r * kRecFloats];
     }
     dma.start_async_dma();
-    if (threadIdx.x < kRecFloats) out[tile * kRecFloats + threadIdx.x] = acc;
+    if (threadIdx.x < TILES * kRecFloats) out[tile * kRecFloats + threadIdx.x] = acc;
   }
 };
 
-// STAGES objects share the DMA threads; each has its own 4 KiB buffer.  With PREFETCH the index words of an
+// STAGES objects share the DMA threads; each has its own buffer of TILES tiles.  With PREFETCH the index words of an
 // object's next tile are requested right after its current tile (prefetch_index), one turn of the ring before
 // they are used: the transfer that uses them then waits only for loads older than they are, and the elements of
 // the other STAGES - 1 objects stay in flight across it.  Without it every start_xfer_async fetches its own index
 // words and, a wavefront's loads returning in order, waits until nothing of the thread is in flight any more.
-template<typename Consumer, int STAGES, bool PREFETCH = false>
+template<typename Consumer, int STAGES, bool PREFETCH = false, int TILES = 1>
 __global__ void __launch_bounds__(kDmaThreads + kComputeThreads)
 gather_manual(const float* __restrict__ table, const int* __restrict__ idx, float* __restrict__ out,
-              const long long num_tiles)
+              const long long all_tiles)
 {
-  __shared__ __attribute__((aligned(16))) char buf[STAGES][kTileBytes];
+  typedef dma_of<TILES> dma_t;
+  // transfers, the last of them moved back to end with the last tile
+  const long long num_tiles = (all_tiles + TILES - 1) / TILES;
+  auto tile_of = [&](const long long t) __attribute__((always_inline)) { return TILES == 1 || t * TILES < all_tiles - TILES ? t * TILES : all_tiles - TILES; };
+  auto words = [&](const long long t) __attribute__((always_inline)) { return idx + tile_of(t) * kRecsPerTile; };
+  __shared__ __attribute__((aligned(16))) char buf[STAGES][TILES * kTileBytes];
   dma_t dma0(0, kComputeThreads, kComputeThreads);
   dma_t dma1(1, kComputeThreads, kComputeThreads);
   dma_t dma2(2, kComputeThreads, kComputeThreads);
@@ -86,28 +97,28 @@ gather_manual(const float* __restrict__ table, const int* __restrict__ idx, floa
       if constexpr (PREFETCH) {
         // a prefetch beyond the last tile reads the last tile's words instead (never used): no branch
         const long long last = num_tiles - 1;
-        HIPDMA_FOR_STAGES({ d.template prefetch_index<true>(idx + (t + s * stride) * kRecsPerTile); })
+        HIPDMA_FOR_STAGES({ d.template prefetch_index<true>(words(t + s * stride)); })
         HIPDMA_FOR_STAGES({
-          d.template start_xfer_async_prefetched<true, LOAD_CACHE_ALL, STORE_LDS>(idx + (t + s * stride) * kRecsPerTile, table);
-          d.template prefetch_index<true>(idx + (t + (s + STAGES) * stride) * kRecsPerTile);
+          d.template start_xfer_async_prefetched<true, LOAD_CACHE_ALL, STORE_LDS>(words(t + s * stride), table);
+          d.template prefetch_index<true>(words(t + (s + STAGES) * stride));
         })
         do {
           HIPDMA_FOR_STAGES({
             d.template wait_xfer_finish<true, LOAD_CACHE_ALL, STORE_LDS>(buf[s]);
-            d.template start_xfer_async_prefetched<true, LOAD_CACHE_ALL, STORE_LDS>(idx + (t + (s + STAGES) * stride) * kRecsPerTile, table);
+            d.template start_xfer_async_prefetched<true, LOAD_CACHE_ALL, STORE_LDS>(words(t + (s + STAGES) * stride), table);
             const long long ahead = t + (s + 2 * STAGES) * stride;
-            d.template prefetch_index<true>(idx + (ahead < last ? ahead : last) * kRecsPerTile);
+            d.template prefetch_index<true>(words(ahead < last ? ahead : last));
           })
           t += STAGES * stride;
         } while (t + (2 * STAGES - 1) * stride < num_tiles);
       } else {
         HIPDMA_FOR_STAGES({
-          d.template start_xfer_async<true, LOAD_CACHE_ALL, STORE_LDS>(idx + (t + s * stride) * kRecsPerTile, table);
+          d.template start_xfer_async<true, LOAD_CACHE_ALL, STORE_LDS>(words(t + s * stride), table);
         })
         do {
           HIPDMA_FOR_STAGES({
             d.template wait_xfer_finish<true, LOAD_CACHE_ALL, STORE_LDS>(buf[s]);
-            d.template start_xfer_async<true, LOAD_CACHE_ALL, STORE_LDS>(idx + (t + (s + STAGES) * stride) * kRecsPerTile, table);
+            d.template start_xfer_async<true, LOAD_CACHE_ALL, STORE_LDS>(words(t + (s + STAGES) * stride), table);
           })
           t += STAGES * stride;
         } while (t + (2 * STAGES - 1) * stride < num_tiles);
@@ -115,7 +126,7 @@ gather_manual(const float* __restrict__ table, const int* __restrict__ idx, floa
     } else {
       HIPDMA_FOR_STAGES({
         const long long tt = t + s * stride;
-        if (tt < num_tiles) d.template start_xfer_async<true, LOAD_CACHE_ALL, STORE_LDS>(idx + tt * kRecsPerTile, table);
+        if (tt < num_tiles) d.template start_xfer_async<true, LOAD_CACHE_ALL, STORE_LDS>(words(tt), table);
       })
     }
     // the last tiles of this workgroup
@@ -125,7 +136,7 @@ gather_manual(const float* __restrict__ table, const int* __restrict__ idx, floa
         if (tt < num_tiles) {
           d.template wait_xfer_finish<true, LOAD_CACHE_ALL, STORE_LDS>(buf[s]);
           const long long nx = tt + STAGES * stride;
-          if (nx < num_tiles) d.template start_xfer_async<true, LOAD_CACHE_ALL, STORE_LDS>(idx + nx * kRecsPerTile, table);
+          if (nx < num_tiles) d.template start_xfer_async<true, LOAD_CACHE_ALL, STORE_LDS>(words(nx), table);
         }
       })
     }
@@ -136,7 +147,7 @@ gather_manual(const float* __restrict__ table, const int* __restrict__ idx, floa
         const long long tt = t + s * stride;
         if (tt < num_tiles) {
           d.wait_for_dma_finish();
-          Consumer::run(buf[s], out, tt, d);
+          Consumer::template run<TILES>(buf[s], out, tile_of(tt), d);
         }
       })
     }
@@ -158,7 +169,7 @@ gather_single(const float* __restrict__ table, const int* __restrict__ idx, floa
     dma.start_async_dma();
     for (long long t = blockIdx.x; t < num_tiles; t += gridDim.x) {
       dma.wait_for_dma_finish();
-      Consumer::run(buf, out, t, dma);
+      Consumer::template run<1>(buf, out, t, dma);
     }
   }
 }
@@ -179,7 +190,7 @@ int launch_gather(const float* d_table, const int32_t* d_idx, float* d_out, size
   const long long tiles = (long long)(n_idx / kRecsPerTile);
   hipStream_t s = (hipStream_t)stream;
   const dim3 block(kDmaThreads + kComputeThreads);
-  // Workgroups per compute unit.  Objects that fetch their own index words drain the DMA wavefronts at every
+  // Workgroups per compute unit of the numbered variants.  Objects that fetch their own index words drain the DMA wavefronts at every
   // transfer and need many workgroups to cover that (six with several objects, eight with one).  With the index
   // words requested ahead two objects and three workgroups are enough (0.634 ms on the configuration's 512 MiB
   // table, which the caches help to serve); a table several times the Infinity Cache wants four (0.724 ms against
@@ -187,19 +198,35 @@ int launch_gather(const float* d_table, const int32_t* d_idx, float* d_out, size
   // The copy consumer writes as much as it reads and wants a shorter queue still: two (74.6 % on the 512 MiB table,
   // 69.5 % on 1.875 GiB, against 74.0 / 68.2 with three).
   const int ahead_wgs = Consumer::kWritesEveryRecord ? 2 : n_records * (size_t)kRecBytes <= (1ull << 30) ? 3 : 4;
-  auto grid = [&](const int per_cu) { return dim3((unsigned)workloads::persistent_grid(tiles, per_cu)); };
-  // The library's choice: a short list is over before three workgroups per compute unit with two tiles each have filled their
-  // queues; eight with one tile start sooner (row sums of 256 Ki records: 6.4 against 7.6 us from the caches, 8.7 / 8.9 from DRAM; 32 Ki:
-  // 3.2 / 3.7; copies of 32 Ki: 3.6 / 4.0).  Longer lists gain as much from the caches and lose twice that from DRAM (row sums of
-  // 1 Mi: 22.8 / 24.1 and 28.2 / 25.3).
-  if (variant == 0) variant = n_idx * (size_t)kRecBytes <= (32ull << 20) ? 1 : 6;
+  auto grid = [&](const int per_cu, const long long n) { return dim3((unsigned)workloads::persistent_grid(n, per_cu)); };
+  if constexpr (Consumer::kWritesEveryRecord) {
+    // The library's choice: a short list is over before two workgroups per compute unit with two tiles each have filled their queues; eight
+    // with one tile start sooner (copies of 32 Ki records from the caches 3.6 us against 4.0).
+    if (variant == 0) variant = n_idx * (size_t)kRecBytes <= (32ull << 20) ? 1 : 6;
+  } else if (variant == 0) {
+    // The library's choice: short lists as above.  Longer ones take four tiles in one transfer, whose sums occupy all compute threads (with one
+    // tile in turn a quarter of one of the two wavefronts adds while the DMA wavefronts wait for the buffer): 16 KiB in flight per
+    // workgroup instead of 8, a quarter of the hand-offs.  It counts where an L2 holds the table (us, variant 6 / this: 6 Mi indices of 24000
+    // records 104 / 51, of 60000 106 / 66, 1 Mi of 24000 21 / 13); elsewhere what is in flight does, and four workgroups per compute unit become
+    // two or three where the table exceeds the Infinity Cache (4 Mi records, 32 Mi indices 632 / 619; two 617, three 639, four 646; 32 Mi records,
+    // 16 Mi indices 378, two 382, three 376, four 384).  Between 64 and 112 Ki indices the short form is 0.3 us ahead from the caches, beyond
+    // the long one (2 Mi records, 176 Ki indices 4.6 / 4.6 and from DRAM 7.8 / 7.4; 24000, 256 Ki 5.2 / 4.6 and 6.3 / 6.0).
+    if (n_idx <= (112u << 10)) variant = 1;
+    else {
+      const size_t table = n_records * (size_t)kRecBytes;
+      const int wgs = table <= (256ull << 20) || n_idx <= (1u << 20) ? 4 : table <= (1ull << 30) ? 2 : 3;
+      hipLaunchKernelGGL((gather_manual<Consumer, 1, true, 4>), grid(wgs, (tiles + 3) / 4), block, 0, s, d_table, d_idx, d_out, tiles);
+      CUDADMA_HIP_CHECK(hipGetLastError());
+      return CUDADMA_OK;
+    }
+  }
   switch (variant) {
-    case 6: hipLaunchKernelGGL((gather_manual<Consumer, 2, true>), grid(ahead_wgs), block, 0, s, d_table, d_idx, d_out, tiles); break;
-    case 1: hipLaunchKernelGGL(gather_single<Consumer>, grid(8), block, 0, s, d_table, d_idx, d_out, tiles); break;
-    case 2: hipLaunchKernelGGL((gather_manual<Consumer, 2>), grid(6), block, 0, s, d_table, d_idx, d_out, tiles); break;
-    case 3: hipLaunchKernelGGL((gather_manual<Consumer, 4>), grid(6), block, 0, s, d_table, d_idx, d_out, tiles); break;
-    case 4: hipLaunchKernelGGL((gather_manual<Consumer, 4, true>), grid(ahead_wgs), block, 0, s, d_table, d_idx, d_out, tiles); break;
-    default: hipLaunchKernelGGL((gather_manual<Consumer, 3, true>), grid(ahead_wgs), block, 0, s, d_table, d_idx, d_out, tiles); break;
+    case 6: hipLaunchKernelGGL((gather_manual<Consumer, 2, true>), grid(ahead_wgs, tiles), block, 0, s, d_table, d_idx, d_out, tiles); break;
+    case 1: hipLaunchKernelGGL(gather_single<Consumer>, grid(8, tiles), block, 0, s, d_table, d_idx, d_out, tiles); break;
+    case 2: hipLaunchKernelGGL((gather_manual<Consumer, 2>), grid(6, tiles), block, 0, s, d_table, d_idx, d_out, tiles); break;
+    case 3: hipLaunchKernelGGL((gather_manual<Consumer, 4>), grid(6, tiles), block, 0, s, d_table, d_idx, d_out, tiles); break;
+    case 4: hipLaunchKernelGGL((gather_manual<Consumer, 4, true>), grid(ahead_wgs, tiles), block, 0, s, d_table, d_idx, d_out, tiles); break;
+    default: hipLaunchKernelGGL((gather_manual<Consumer, 3, true>), grid(ahead_wgs, tiles), block, 0, s, d_table, d_idx, d_out, tiles); break;
   }
   CUDADMA_HIP_CHECK(hipGetLastError());
   return CUDADMA_OK;

@@ -411,6 +411,23 @@ def test_default_transpose_around_its_lines(device, n):
     assert torch.equal(dst.view(torch.int32), src.t().contiguous().view(torch.int32))
 
 
+# the default row sums beyond 112 Ki indices: four tiles in one transfer, the last one moved back where four does not divide the tiles; one
+# transfer and several for a workgroup, and the tables at which the number of workgroups changes (256 MiB, 1 GiB; beyond 1 Mi indices)
+@pytest.mark.parametrize("n_idx", [112 << 10, (112 << 10) + 32, (112 << 10) + 64, (112 << 10) + 96, 4 * 32 * 1024 + 128, (1 << 20) + 32, 3 * (1 << 20) - 32])
+@pytest.mark.parametrize("recs", [1, 3000, (2 << 20) + 1, (8 << 20) + 1])
+def test_default_gather_rowsum_transfers(device, n_idx, recs):
+    table = wl.fill_uniform(torch.empty((recs, 32), device=device), 51)
+    idx = wl.fill_indices(torch.empty(n_idx, dtype=torch.int32, device=device), recs, 52)
+    buf = torch.full((n_idx // 32 + 4, 32), float("nan"), device=device)
+    got = wl.gather_rowsum(table, idx, buf[:n_idx // 32])
+    rows = table[idx.long()].view(-1, 32, 32)
+    want = rows[:, 0].clone()
+    for r in range(1, 32):
+        want += rows[:, r]
+    assert torch.equal(got, want)
+    assert bool(torch.isnan(buf[n_idx // 32:]).all())
+
+
 @pytest.mark.parametrize("n_idx", [1 << 18, (1 << 18) + 32])
 def test_default_gather_around_its_line(device, n_idx):
     recs = (2 << 20) + 64
