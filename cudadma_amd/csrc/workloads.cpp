@@ -56,7 +56,7 @@ static const VariantInfo kSequential[] = {
   {"variant 5 with a contiguous run of tiles per workgroup instead of every n-th tile"},
 };
 static const VariantInfo kStrided[] = {
-  {"the library's choice: variant 4 for up to two tiles per compute unit, variant 11 up to 48 MiB of both matrices, beyond "
+  {"the library's choice: variant 4 for up to three tiles per compute unit, variant 11 up to 108 MiB of both matrices, beyond "
    "that variant 10 at its default split (three DMA wavefronts, one compute wavefront, one LDS tile, "
    "the next tile in the DMA wavefronts' registers)"},
   {"single buffer: one object and one LDS tile, execute_dma (the next tile waits in the DMA wavefronts' registers); one "

@@ -159,11 +159,11 @@ transpose_manual_double(const float* __restrict__ in, float* __restrict__ out, c
       int ty, tx;
       tile_coords(t, tiles_per_side, band, ty, tx);
       dma0.wait_for_dma_finish();
-      write_tile_transposed<LDS_ROW_BYTES, false, QUAD>(buf0, out, n, ty, tx, dma0);
+      write_tile_transposed<LDS_ROW_BYTES, false, QUAD, true>(buf0, out, n, ty, tx, dma0);
       if (t + stride < num_tiles) {
         tile_coords(t + stride, tiles_per_side, band, ty, tx);
         dma1.wait_for_dma_finish();
-        write_tile_transposed<LDS_ROW_BYTES, false, QUAD>(buf1, out, n, ty, tx, dma1);
+        write_tile_transposed<LDS_ROW_BYTES, false, QUAD, true>(buf1, out, n, ty, tx, dma1);
       }
     }
   }
@@ -333,7 +333,7 @@ transpose_not_specialized(const float* __restrict__ in, float* __restrict__ out,
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
 #pragma unroll
-      for (int k = 0; k < 4; ++k) o[(size_t)(4 * j + k) * n] = __uint_as_float(v[j][k]);
+      for (int k = 0; k < 4; ++k) __builtin_nontemporal_store(__uint_as_float(v[j][k]), o + (size_t)(4 * j + k) * n);
     }
   }
 }
@@ -777,15 +777,17 @@ extern "C" int cudadma_strided_transpose(const float* d_in, float* d_out, int n,
   const int tiles_per_side = n / kTile;
   const int tiles = tiles_per_side * tiles_per_side;
   // Variant 0 is the library's choice.  Variant 10's shape, one 16 KB tile in flight per compute unit and streaming loads and stores,
-  // is for matrices from DRAM (16384: 358 us against 456 with variant 11, 4096: 26.2 / 29.8).  Small matrices come from the
-  // Infinity Cache or leave their result there, and its short queue only costs (2112: 9.6 us against 6.8 with variant 11 from the
-  // cache, 10.2 / 8.9 from DRAM; 2496, the last below the line: 11.7 / 9.0 and 11.9 / 11.9).  Beyond it variant 11 still gains
-  // a quarter from the cache, but loses from DRAM (2560: 12.7 / 13.1, 2816: 14.5 / 16.1): the line lies where neither loses.  Up to
-  // two tiles per compute unit the tile is best moved by every wavefront, with no hand-off (variant 4; 512: 3.7 us against 2.7
-  // from DRAM, 1280: 5.6 / 4.4 and 5.6 / 5.4).
+  // is for matrices from DRAM (16384: 358 us against 449 with variant 11, 4096: 26.2 / 28.7).  Small matrices come from the
+  // Infinity Cache, and its short queue only costs (us from the caches and from DRAM, variant 10 / 11: 2112 9.6 / 5.2 and 10.2 / 7.5; 3008 16.0 / 11.3 and
+  // 15.8 / 13.0; 3712 21.8 / 17.9 and 22.4 / 22.1; beyond, variant 11 still gains from the caches and loses from DRAM: 3840 22.3 / 19.1 and 23.8 /
+  // 25.3).  Up to three tiles per compute unit the tile is best moved by every wavefront, with no hand-off (variant 4), as many workgroups as
+  // there are tiles (variant 11 / 4: 1024 3.3 / 2.8 and 3.6 / 3.5; 1408 3.8 / 3.3 and 4.5 / 4.3; 1728 4.1 / 3.8 and 6.2 / 5.7; 1984 4.6 / 4.3 and 6.7 / 8.0).
+  // All three store non-temporally.  With plain stores the output takes the place of the input in the caches: variant 11 2112 6.2
+  // and 9.4, 2496 8.3 and 12.0; variant 4, one workgroup per compute unit, 1408 3.8 and 5.9.
+  int small_per_cu = 1;
   if (variant == 0 && workloads::tuning("transpose_workgroups", 0) == 0) {
-    if (tiles <= 2 * workloads::device_cus()) variant = 4;
-    else if (8LL * n * n <= (48LL << 20)) variant = 11;
+    if (tiles <= 3 * workloads::device_cus()) { variant = 4; small_per_cu = 4; }
+    else if (8LL * n * n <= (108LL << 20)) variant = 11;
   }
   // The kernels with one LDS tile (variants 1 and 4) run best with exactly one workgroup per compute unit, i.e. one
   // 16 KB tile of loads in flight per compute unit, and with the tiles walked down the columns (the workgroups that
@@ -850,7 +852,7 @@ extern "C" int cudadma_strided_transpose(const float* d_in, float* d_out, int n,
     case 12:
     case 13: CUDADMA_REQUIRE(false, "variants 12 and 13 are sweep kernels: build the library with make EXTRA=-DHIPDMA_SWEEP_VARIANTS");
 #endif
-    default: hipLaunchKernelGGL(transpose_not_specialized, grid_for(1), block, 0, s, d_in, d_out, n, tiles, band); break;
+    default: hipLaunchKernelGGL(transpose_not_specialized, grid_for(small_per_cu), block, 0, s, d_in, d_out, n, tiles, band); break;
   }
   CUDADMA_HIP_CHECK(hipGetLastError());
   return CUDADMA_OK;

@@ -411,6 +411,12 @@ def test_default_transpose_around_its_lines(device, n):
     assert torch.equal(dst.view(torch.int32), src.t().contiguous().view(torch.int32))
 
 
+# three tiles per compute unit (27 tiles a side) and 108 MiB of both matrices (58), and the smallest
+@pytest.mark.parametrize("n", [64, 128, 1728, 1792, 3712, 3776])
+def test_default_transpose_around_its_further_lines(device, n):
+    test_default_transpose_around_its_lines(device, n)
+
+
 # the default row sums beyond 112 Ki indices: four tiles in one transfer, the last one moved back where four does not divide the tiles; one
 # transfer and several for a workgroup, and the tables at which the number of workgroups changes (256 MiB, 1 GiB; beyond 1 Mi indices)
 @pytest.mark.parametrize("n_idx", [112 << 10, (112 << 10) + 32, (112 << 10) + 64, (112 << 10) + 96, 4 * 32 * 1024 + 128, (1 << 20) + 32, 3 * (1 << 20) - 32])
