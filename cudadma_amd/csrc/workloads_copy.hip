@@ -31,7 +31,7 @@ __device__ __forceinline__ void drain_tile(const vec4_t* lds_tile, vec4_t* __res
 }
 
 // variants 0 and 3: one DMA group, two objects, two-phase calls
-template<int STORE_QUAL>
+template<int STORE_QUAL, bool STREAM = false, int LOAD_QUAL = LOAD_CACHE_ALL>
 __global__ void __launch_bounds__(kDmaThreads + kComputeThreads)
 copy_manual_double(const char* __restrict__ in, char* __restrict__ out, const int num_tiles)
 {
@@ -46,29 +46,29 @@ copy_manual_double(const char* __restrict__ in, char* __restrict__ out, const in
     if (t + 3 * stride < num_tiles) {
       // Steady state with no branch around any load, entered from a prologue that has none either:
       // the wait for one object's tile then leaves the other object's loads in flight.
-      dma0.template start_xfer_async<true, LOAD_CACHE_ALL, STORE_QUAL>(in + (size_t)t * kTileBytes);
-      dma1.template start_xfer_async<true, LOAD_CACHE_ALL, STORE_QUAL>(in + (size_t)(t + stride) * kTileBytes);
+      dma0.template start_xfer_async<true, LOAD_QUAL, STORE_QUAL>(in + (size_t)t * kTileBytes);
+      dma1.template start_xfer_async<true, LOAD_QUAL, STORE_QUAL>(in + (size_t)(t + stride) * kTileBytes);
       do {
-        dma0.template wait_xfer_finish<true, LOAD_CACHE_ALL, STORE_QUAL>(buf0);
-        dma0.template start_xfer_async<true, LOAD_CACHE_ALL, STORE_QUAL>(in + (size_t)(t + 2 * stride) * kTileBytes);
-        dma1.template wait_xfer_finish<true, LOAD_CACHE_ALL, STORE_QUAL>(buf1);
-        dma1.template start_xfer_async<true, LOAD_CACHE_ALL, STORE_QUAL>(in + (size_t)(t + 3 * stride) * kTileBytes);
+        dma0.template wait_xfer_finish<true, LOAD_QUAL, STORE_QUAL>(buf0);
+        dma0.template start_xfer_async<true, LOAD_QUAL, STORE_QUAL>(in + (size_t)(t + 2 * stride) * kTileBytes);
+        dma1.template wait_xfer_finish<true, LOAD_QUAL, STORE_QUAL>(buf1);
+        dma1.template start_xfer_async<true, LOAD_QUAL, STORE_QUAL>(in + (size_t)(t + 3 * stride) * kTileBytes);
         t += 2 * stride;
       } while (t + 3 * stride < num_tiles);
     } else {
-      if (t < num_tiles) dma0.template start_xfer_async<true, LOAD_CACHE_ALL, STORE_QUAL>(in + (size_t)t * kTileBytes);
+      if (t < num_tiles) dma0.template start_xfer_async<true, LOAD_QUAL, STORE_QUAL>(in + (size_t)t * kTileBytes);
       if (t + stride < num_tiles)
-        dma1.template start_xfer_async<true, LOAD_CACHE_ALL, STORE_QUAL>(in + (size_t)(t + stride) * kTileBytes);
+        dma1.template start_xfer_async<true, LOAD_QUAL, STORE_QUAL>(in + (size_t)(t + stride) * kTileBytes);
     }
     // the last tiles of this workgroup
     for (; t < num_tiles; t += 2 * stride) {
-      dma0.template wait_xfer_finish<true, LOAD_CACHE_ALL, STORE_QUAL>(buf0);
+      dma0.template wait_xfer_finish<true, LOAD_QUAL, STORE_QUAL>(buf0);
       if (t + 2 * stride < num_tiles)
-        dma0.template start_xfer_async<true, LOAD_CACHE_ALL, STORE_QUAL>(in + (size_t)(t + 2 * stride) * kTileBytes);
+        dma0.template start_xfer_async<true, LOAD_QUAL, STORE_QUAL>(in + (size_t)(t + 2 * stride) * kTileBytes);
       if (t + stride < num_tiles) {
-        dma1.template wait_xfer_finish<true, LOAD_CACHE_ALL, STORE_QUAL>(buf1);
+        dma1.template wait_xfer_finish<true, LOAD_QUAL, STORE_QUAL>(buf1);
         if (t + 3 * stride < num_tiles)
-          dma1.template start_xfer_async<true, LOAD_CACHE_ALL, STORE_QUAL>(in + (size_t)(t + 3 * stride) * kTileBytes);
+          dma1.template start_xfer_async<true, LOAD_QUAL, STORE_QUAL>(in + (size_t)(t + 3 * stride) * kTileBytes);
       }
     }
   } else {
@@ -76,10 +76,10 @@ copy_manual_double(const char* __restrict__ in, char* __restrict__ out, const in
     dma1.start_async_dma();
     for (int t = blockIdx.x; t < num_tiles; t += 2 * stride) {
       dma0.wait_for_dma_finish();
-      drain_tile(buf0, (vec4_t*)(out + (size_t)t * kTileBytes), dma0);
+      drain_tile<STREAM>(buf0, (vec4_t*)(out + (size_t)t * kTileBytes), dma0);
       if (t + stride < num_tiles) {
         dma1.wait_for_dma_finish();
-        drain_tile(buf1, (vec4_t*)(out + (size_t)(t + stride) * kTileBytes), dma1);
+        drain_tile<STREAM>(buf1, (vec4_t*)(out + (size_t)(t + stride) * kTileBytes), dma1);
       }
     }
   }
@@ -318,10 +318,18 @@ extern "C" int cudadma_sequential_copy(const float* d_in, float* d_out, size_t b
     case 0:
       // Two operating points, as for every read + write stream on this part: a working set that the 256 MB Infinity
       // Cache holds from launch to launch wants many tiles in flight (two LDS tiles, four workgroups per compute unit);
-      // beyond it the memory system serves a short queue better (one LDS tile, two workgroups per compute unit,
-      // streaming loads and non-temporal stores: 1 GiB in 0.353 ms against 0.408 ms).
-      if (2 * bytes <= kCacheAssistedBytes)
-        hipLaunchKernelGGL(copy_manual_double<STORE_LDS>, dim3(workloads::persistent_grid(tiles, 4)), block, 0, s, in, out, tiles);
+      // beyond it the memory system serves a short queue better (one LDS tile, two workgroups per compute unit: 1 GiB in 0.353 ms
+      // against 0.408 ms).  Stores are non-temporal throughout, which leaves the caches to the input: with plain ones, from the caches and
+      // from DRAM, 16 MiB 5.6 us and 7.5, now 4.4 and 6.2; 32 MiB 11.3 and 11.6, now 9.0 and 11.7; 64 MiB 20.9 and 25.3, now 21.1 and 24.0; 94 MiB
+      // 30.0 and 39.3, now 30.0 and 35.7.  Up to half of that cache the loads are too (94 MiB: 31.2 and 34.2, so not beyond), and up to an
+      // eighth the form with one LDS tile and four workgroups per compute unit starts sooner (16 MiB: two LDS tiles 4.4 and 6.4; 32 MiB: one
+      // 8.6 and 12.4).
+      if (2 * bytes <= kCacheAssistedBytes / 6)
+        hipLaunchKernelGGL(copy_single<true>, dim3(workloads::persistent_grid(tiles, 4)), block, 0, s, in, out, tiles);
+      else if (2 * bytes <= kCacheAssistedBytes / 3 * 2)
+        hipLaunchKernelGGL((copy_manual_double<STORE_LDS, true, LOAD_CACHE_STREAMING>), dim3(workloads::persistent_grid(tiles, 4)), block, 0, s, in, out, tiles);
+      else if (2 * bytes <= kCacheAssistedBytes)
+        hipLaunchKernelGGL((copy_manual_double<STORE_LDS, true>), dim3(workloads::persistent_grid(tiles, 4)), block, 0, s, in, out, tiles);
       else
         hipLaunchKernelGGL(copy_single<true>, dim3(workloads::persistent_grid(tiles, 2)), block, 0, s, in, out, tiles);
       break;
