@@ -320,13 +320,14 @@ extern "C" int cudadma_sequential_copy(const float* d_in, float* d_out, size_t b
       // Cache holds from launch to launch wants many tiles in flight (two LDS tiles, four workgroups per compute unit);
       // beyond it the memory system serves a short queue better (one LDS tile, two workgroups per compute unit: 1 GiB in 0.353 ms
       // against 0.408 ms).  Stores are non-temporal throughout, which leaves the caches to the input: with plain ones, from the caches and
-      // from DRAM, 16 MiB 5.6 us and 7.5, now 4.4 and 6.2; 32 MiB 11.3 and 11.6, now 9.0 and 11.7; 64 MiB 20.9 and 25.3, now 21.1 and 24.0; 94 MiB
-      // 30.0 and 39.3, now 30.0 and 35.7.  Up to half of that cache the loads are too (94 MiB: 31.2 and 34.2, so not beyond), and up to an
-      // eighth the form with one LDS tile and four workgroups per compute unit starts sooner (16 MiB: two LDS tiles 4.4 and 6.4; 32 MiB: one
-      // 8.6 and 12.4).
+      // from DRAM, 16 MiB 5.6 us and 7.5, now 4.4 and 6.2; 32 MiB 11.3 and 11.6, now 9.0 and 11.7; 64 MiB 20.9 and 25.2, now 21.1 and 25.0; 94 MiB
+      // 30.0 and 39.3, now 30.0 and 35.7.  Up to 48 MiB the loads are too (48 MiB 15.8 and 21.4, now 15.9 and 17.7; beyond, they lose from the
+      // caches: 56 MiB 18.3 / 19.5, 64 MiB 20.9 / 23.6, and with two buffers in turn, 24.3 / 23.0 where plain loads take 20.0), and up to
+      // 16 MiB the form with one LDS tile and four workgroups per compute unit starts sooner (16 MiB: two LDS tiles 4.4 and 6.4; 32 MiB:
+      // one 8.6 and 12.4).
       if (2 * bytes <= kCacheAssistedBytes / 6)
         hipLaunchKernelGGL(copy_single<true>, dim3(workloads::persistent_grid(tiles, 4)), block, 0, s, in, out, tiles);
-      else if (2 * bytes <= kCacheAssistedBytes / 3 * 2)
+      else if (2 * bytes <= kCacheAssistedBytes / 2)
         hipLaunchKernelGGL((copy_manual_double<STORE_LDS, true, LOAD_CACHE_STREAMING>), dim3(workloads::persistent_grid(tiles, 4)), block, 0, s, in, out, tiles);
       else if (2 * bytes <= kCacheAssistedBytes)
         hipLaunchKernelGGL((copy_manual_double<STORE_LDS, true>), dim3(workloads::persistent_grid(tiles, 4)), block, 0, s, in, out, tiles);
