@@ -68,10 +68,12 @@ __device__ __forceinline__ void tile_of_workgroup(const int b, const int tiles_m
 
 // The order in which the workgroups take the tiles; `per_cu` of them share a compute unit.  Every XCD has an L2 of its own, so the panels
 // of A and B behind the tiles that are in work on one XCD at a time should be few.
-//   blocks     grids that divide into 4 x 2: every XCD gets one compact block.  Not where the blocks are narrow strips with half as many panels
-//              again as a band's share (128 x 128 tiles, us in blocks and in bands, from the caches and from DRAM: 512 x 16384 x 1024 28.2 / 22.3 and
+//   blocks     grids that divide into 4 x 2: every XCD gets one compact block.  Not where the blocks are narrow strips with 1.8 times the panels
+//              of a band's share (128 x 128 tiles, us in blocks and in bands, from the caches and from DRAM: 512 x 16384 x 1024 28.2 / 22.3 and
 //              32.6 / 27.4; 1024 x 6144 x 2048 32.1 / 28.7 and 41.6 / 34.8; 512 x 8192 x 4096 43.5 / 41.0 and 46.2 / 44.3); with few K steps it is the writes of C
 //              that count (1024 x 16384 x 256, variant 1: 22.1 / 24.3), though not with tiles below 128 x 128 (256 x 5376 x 256 from DRAM 6.3 / 5.7).
+//              Between 1.5 and 1.8 times as many, only with many K steps (1536 x 7680 x 4096 from the caches 110.8 / 95.6, x 512 from DRAM 21.2 / 25.3)
+//              and where the last band is no thin rest (1024 x 5376 x 2048, eight rows in bands of seven: 28.0 / 30.3 and 31.3 / 37.8).
 //   bands      up to eight tile rows, down the columns of a band, an eighth of that walk for every XCD (dealt row-major instead:
 //              3712 x 4736 x 3712 with 128 x 128 tiles 188 us against 139, 640 x 8064 x 2048 34 / 28).  In grids that divide level or slower than
 //              blocks (8192 x 8192 x 1024, 256 x 256 tiles: 155 us against 140).
@@ -90,7 +92,8 @@ int tile_walk(const int m, const int n, const int k, const int tile_rows, const 
   int rows = 1;
   while (rows < 8 && rows * rows < each) ++rows;
   const int high = tiles_m < rows ? tiles_m : rows;
-  const bool narrow = (k >= 512 || tile_rows < 128) && tiles_m / 4 + tiles_n / 2 > 3 * (high + each / high) / 2;      // panels behind a block and behind a band's share
+  const long long of_block = tiles_m / 4 + tiles_n / 2, of_band = high + each / high;                     // panels behind a block and behind a band's share
+  const bool narrow = (5 * of_block > 9 * of_band && (k >= 512 || tile_rows < 128)) || (2 * of_block > 3 * of_band && k >= 2048 && 2 * (tiles_m % rows) >= rows);
   if ((tiles_m % 4) == 0 && (tiles_n % 2) == 0 && !narrow) return kWalkBlocks;
   const double in_work = (double)(each < per_cu * cus / 8 ? each : per_cu * cus / 8), columns = tiles_n / 8;
   const bool own_columns = (tiles_n % 8) == 0 && in_work / columns + columns <= rows + in_work / rows + 1;
@@ -1362,13 +1365,15 @@ extern "C" int cudadma_gemm_bf16(const uint16_t* d_a, const uint16_t* d_b, float
     // Grids of few tiles take the smallest tile that still gives every compute unit at most one (32 x 32, 32 x 64, 64 x 64) or, with half as
     // many wavefronts, two workgroups (64 x 64).  us with those four and with 128 x 128, from the caches: 512 x 512 x 512 3.5 / 3.7 / 4.6 / 4.6 / 6.0;
     // 640 x 512 x 1152 6.0 / 4.8 / 6.0 / 6.4 / 9.8; 768^3 6.7 / 7.0 / 5.3 / 5.5 / 7.8; 1024 x 1152 x 1920 - / - / 15.2 / 12.6 / 14.8 and from DRAM
-    // 17.0 / 14.8 / 20.4.  The last one gains 4 % from the caches (30 shapes; least 0.95, 384 x 4864 x 256 5.0 -> 5.3) and 15 % from DRAM.
+    // 17.0 / 14.8 / 20.4.  The last one has a wavefront only two or three steps below k = 512, and
+    // then 128 x 128 is as fast or faster (1152 x 1792 x 256 from the caches 5.5 / 5.1, from DRAM 5.9 / 5.7; x 512 6.4 / 6.6 and 7.0 / 7.5; x 768 7.7 / 8.1 and 8.8 / 10.0).
+    // With long rows 128 x 128 has caught up (256 x 6656 x 6144 45.0 / 42.0 and 63.4 / 61.3; 768 x 2560 x 3072 24.0 / 22.3 and 29.7 / 30.7).
     const long long t32 = (long long)(m / 32) * (n / 32);
     if (!direct_rows_fit(n, k)) variant = 1;
     else if (t32 <= cus) return launch_dealt_steps<1, 1, 8>(d_a, d_b, d_c, m, n, k, s);
     else if (t32 <= 2 * cus) return launch_dealt_steps<1, 2, 8>(d_a, d_b, d_c, m, n, k, s);
     else if (t32 <= 4 * cus) return launch_dealt_steps<2, 2, 8>(d_a, d_b, d_c, m, n, k, s);
-    else if (t32 <= 8 * cus) return launch_dealt_steps<2, 2, 4>(d_a, d_b, d_c, m, n, k, s);
+    else if (t32 <= 8 * cus && k >= 512 && k < 3072) return launch_dealt_steps<2, 2, 4>(d_a, d_b, d_c, m, n, k, s);
     else if (even && rounds((long long)(m / 256) * (n / 256), cus, cus * 5 / 8, 160, 110, 1000) < small) variant = 9;
     else {
       const long long grid = (long long)(m / 128) * (n / 128);

@@ -618,7 +618,7 @@ def test_gemm_stages(device, m, n, k):
 # small grids of the default variant, whose wavefronts take K steps of 64 in turn: both sides of the lines between its tiles (32 x 32, 32 x 64,
 # 64 x 64 with eight and with four wavefronts, then 128 x 128) on 256 compute units, fewer K steps than wavefronts, as many, and a remainder
 @pytest.mark.parametrize("m, n", [(128, 128), (512, 512), (640, 512), (512, 1024), (1152, 512), (1024, 1024), (128, 8320), (2048, 1024), (2176, 1024)])
-@pytest.mark.parametrize("k", [128, 256, 384, 512, 640, 1152])
+@pytest.mark.parametrize("k", [128, 256, 384, 512, 640, 1152, 2944, 3072])
 def test_gemm_dealt_steps(device, m, n, k):
     a = wl.fill_normal_bf16(torch.empty((m, k), dtype=torch.bfloat16, device=device), 65)
     b = wl.fill_normal_bf16(torch.empty((k, n), dtype=torch.bfloat16, device=device), 66)
