@@ -45,10 +45,10 @@ PATTERN_KERNELS = {
     "strided_even_split": "transpose_single<true, true>",
     "strided_double_buffered_lds": "transpose_double_lds<3, 1>",
     "strided_two_lds_tiles": "transpose_manual_double<272, false>",
-    "sequential": "copy_manual_double<4>",
+    "sequential": "copy_manual_double<4, true, 0>",
     "sequential_hbm": "copy_single<true, false>",
-    "gather": "gather_manual<(anonymous namespace)::RowsumConsumer, 2, true>",
-    "gather_hbm": "gather_manual<(anonymous namespace)::RowsumConsumer, 2, true>",
+    "gather": "gather_manual<(anonymous namespace)::RowsumConsumer, 1, true, 4>",
+    "gather_hbm": "gather_manual<(anonymous namespace)::RowsumConsumer, 1, true, 4>",
     "scatter": "scatter_manual<4>",
     "halo": "stencil_ws_vec4<2, 8>",
     "halo_handshake": "stencil_ws_vec4<0, 8>",
@@ -378,11 +378,11 @@ def main():
     # ---- config 3: indirect gather, row-sum consumer: the 512 MiB table of the configuration, and a 4 GiB table ----
     for name, recs, note, bound in (
             ("gather", 4 * 1024 * 1024, "CudaDMAIndirect 32 x 128 B records per tile from the configuration's 512 MiB table (4 Mi records, "
-             "each read 8 times over per launch: most reads are served by L2 and the 256 MB Infinity Cache), two objects per DMA "
-             "group with the index words requested one transfer ahead, three workgroups per compute unit, row-sum consumer",
+             "each read 8 times over per launch: most reads are served by L2 and the 256 MB Infinity Cache), one object per DMA "
+             "group that brings four tiles in a transfer, index words requested one transfer ahead, two workgroups per compute unit, row-sum consumer",
              "infinity cache + hbm"),
             ("gather_hbm", 32 * 1024 * 1024, "the same kernel and index count on a 4 GiB table (32 Mi records, each read once on "
-             "average; sixteen times the Infinity Cache), four workgroups per compute unit, row-sum consumer", "hbm")):
+             "average; sixteen times the Infinity Cache), three workgroups per compute unit, row-sum consumer", "hbm")):
         if not want(name):
             continue
         table, idx, sums = inputs.pop(name)
