@@ -1,0 +1,90 @@
+// Rules by which a default variant chooses a kernel or a launch shape from the sizes of a call: plain functions of whole numbers, free of HIP
+// calls, so that a test can evaluate them on a host.
+#pragma once
+
+#ifdef __HIPCC__
+#include <hip/hip_runtime.h>
+#define DISPATCH_FN __host__ __device__ __forceinline__
+#else
+#define DISPATCH_FN inline
+#endif
+
+namespace dispatch {
+
+// ---- GEMM: the order in which the workgroups take the tiles ----
+// Workgroup -> tile.  Workgroup b runs on XCD b % 8.  `walk` is what tile_walk() chose: blocks, row-major, or the rows of a band.
+constexpr int kWalkBlocks = 0, kWalkRowMajor = -1;
+DISPATCH_FN void tile_of_workgroup(const int b, const int tiles_m, const int tiles_n, const int walk, int& tile_m, int& tile_n)
+{
+  const int xcd = b & 7, idx = b >> 3;
+  if (walk == kWalkBlocks) {
+    const int bm = tiles_m / 4, bn = tiles_n / 2;       // block of one XCD
+    tile_m = (xcd >> 1) * bm + idx / bn;
+    tile_n = (xcd & 1) * bn + idx % bn;
+  } else if (walk == kWalkRowMajor) {
+    tile_m = b / tiles_n;
+    tile_n = b % tiles_n;
+  } else {
+    const int rows = walk, tiles = tiles_m * tiles_n, each = tiles >> 3, more = tiles & 7;
+    const int at = xcd * each + (xcd < more ? xcd : more) + idx;
+    const int band = at / (rows * tiles_n), in_band = at - band * rows * tiles_n;
+    const int height = tiles_m - band * rows < rows ? tiles_m - band * rows : rows;
+    tile_n = in_band / height;
+    tile_m = band * rows + in_band - tile_n * height;
+  }
+}
+
+// `per_cu` workgroups share one of `cus` compute units.  Every XCD has an L2 of its own, so the panels of A and B behind the tiles that are in
+// work on one XCD at a time should be few.
+//   blocks     grids that divide into 4 x 2: every XCD gets one compact block, unless the grid is narrow (below).
+//   bands      up to eight tile rows, down the columns of a band, an eighth of that walk for every XCD (dealt row-major instead:
+//              3712 x 4736 x 3712 with 128 x 128 tiles 188 us against 139, 640 x 8064 x 2048 34 / 28).  In grids that divide level or slower than
+//              blocks (8192 x 8192 x 1024, 256 x 256 tiles: 155 us against 140).
+//   row-major  where eight divides the tiles of a row, so that every XCD has columns of its own, and its rows and columns are then no more
+//              than with bands (7680 x 8192 x 384, 256 x 256 tiles: 79 us, bands 87; 640 x 8192 x 1024, 128 x 128: 15.5 / 16.8.  But
+//              16 rows and 4 columns against 8 and 8: 3712 x 4096 x 640 33.5 / 28.8 from DRAM; 15 and 2 against 6 and 5: 1920 x 2048 x 2048
+//              26.6 / 23.0); where one round of tiles is over in a few K steps and finding the place in a band counts (0.2 us: 640 x 4096 x 256
+//              5.4 / 5.6); and with two K steps of 64, when a tile is mostly its block of C and the bands scatter the writes of a large C, as long as
+//              an L2 holds B (from DRAM: 8064 x 8064 x 128 49 / 55, 4224 x 5760 x 128 20.7 / 22.9; 6528 x 896 x 128, a small C, 8.0 / 7.5;
+//              2176 x 7808 x 256 24.4 / 21.9).
+// Narrow grids: the blocks of a grid of few tile rows are strips that touch many more panels than a band's share.  What such a grid walks in
+// instead depends on what it would walk in if it did not divide.  us, from the caches and from DRAM, blocks / that walk, tiles of 128 x 128:
+//   own columns    from 13/7 times the panels (1024 x 6144 x 2048 31.7 / 28.1 and 41.4 / 35.1, 512 x 8192 x 4096 42.9 / 35.1 and 46.1 / 42.9; but 1.83
+//                  times, 1024 x 5120 x 1024, 17.9 / 16.8 and 18.1 / 20.4), or from 1.5 and k = 2048 on if the bands' last one would be no thin
+//                  rest (1536 x 8192 x 2048 19 % and 9 %, 2048 x 10240 x 2048 104 / 85 and 111 / 99).  Among grids of ten columns an XCD 1024 x 10240 x 512
+//                  still loses from DRAM (9 %; 13 % faster from the caches).
+//   bands of four  the whole height: from 1.8 times (512 x 16384 x 512 17.8 / 12.3 and 21.3 / 17.9, 512 x 8448 x 2048 22 % and 44 %).
+//   one band of    eight: from 2.5 times and k = 1024 on (1024 x 11776 x 2048 14 % and 2 %); below, the caches gain a tenth and DRAM loses
+//                  up to 18 % (1024 x 6912 x 512 1 % and -18 %, x 4096 7 % and -5 %).  Of seven and a thin rest: never (1024 x 5632 x 512 10.2 / 11.6 and
+//                  14.5 / 16.1).
+//   more bands     from 13/7 times and k = 1024 on (1536 x 11008 x 1536 15 % and 9 %; 1536 x 9984 x 512 15 % and -8 %), or from 1.5 times and k = 2048 on if
+//                  they divide the rows evenly (2048 x 8960 x 2048 91 / 79 and 101 / 95; with half a band left over 1536 x 7424 x 2048 6 % and -9 %).
+// Tiles below 128 x 128 are taken for products that are over soon: from 1.8 times at every k (128 x 4096 x 1024 6.0 / 5.0 and 9.1 / 7.7), and from 1.5
+// times and k = 2048 on without a thin rest (5376 x 256 x 2048 15.6 / 14.3 and 19.5 / 17.3).
+inline int tile_walk(const int m, const int n, const int k, const int tile_rows, const int tile_cols, const int per_cu, const int cus)
+{
+  const int tiles_m = m / tile_rows, tiles_n = n / tile_cols;
+  const long long tiles = (long long)tiles_m * tiles_n, each = tiles / 8;
+  int rows = 1;
+  while (rows < 8 && rows * rows < each) ++rows;
+  const double in_work = (double)(each < per_cu * cus / 8 ? each : per_cu * cus / 8), columns = tiles_n / 8;
+  const bool own_columns = (tiles_n % 8) == 0 && in_work / columns + columns <= rows + in_work / rows + 1;
+  const bool mostly_c = k < 256 && (long long)n * k < (3 << 19) && (long long)m * n >= (16 << 20);
+  const int other = own_columns || mostly_c || (tiles <= cus && k < 512) ? kWalkRowMajor : rows;
+  if ((tiles_m % 4) != 0 || (tiles_n % 2) != 0) return other;
+
+  const int high = tiles_m < rows ? tiles_m : rows, rest = tiles_m % rows;
+  const long long of_block = tiles_m / 4 + tiles_n / 2, of_band = high + each / high;        // panels behind a block and behind a band's share
+  const bool times_1_5 = 2 * of_block > 3 * of_band, times_1_8 = 5 * of_block > 9 * of_band, times_13_7 = 7 * of_block >= 13 * of_band,
+             times_2_5 = 2 * of_block >= 5 * of_band;
+  const bool thin_rest = rest != 0 && 2 * rest < rows;
+  bool narrow;
+  if (tile_rows < 128) narrow = times_1_8 || (times_1_5 && k >= 2048 && !thin_rest);
+  else if (tiles_m == 4) narrow = times_1_8 && k >= 512;
+  else if (other == kWalkRowMajor) narrow = (times_13_7 && k >= 512) || (times_1_5 && k >= 2048 && !thin_rest);
+  else if (tiles_m == 8) narrow = times_2_5 && k >= 1024 && rest == 0;
+  else narrow = (times_13_7 && k >= 1024) || (times_1_5 && k >= 2048 && rest == 0);
+  return narrow ? other : kWalkBlocks;
+}
+
+}  // namespace dispatch

@@ -16,6 +16,7 @@
 // Four compute wavefronts (2 x 2) share the SIMDs with the four DMA wavefronts one to
 // one and get 256 registers each; eight (2 x 4, the 256 x 256 tile) make it three
 // wavefronts per SIMD and 168 registers each, but two of them compute.
+#include "dispatch.hpp"
 #include "workloads.hpp"
 
 namespace {
@@ -44,61 +45,10 @@ struct GemmShape {
   typedef CudaDMAStrided<false, 16, kBK * kBN * 2 / kDmaWave, kBN * 2, kDmaWave, kBK> dma_b_t;   // 64 rows x 2*kBN B
 };
 
-// Workgroup -> tile.  Workgroup b runs on XCD b % 8.  `walk` is what tile_walk() chose: blocks, row-major, or the rows of a band.
-constexpr int kWalkBlocks = 0, kWalkRowMajor = -1;
-__device__ __forceinline__ void tile_of_workgroup(const int b, const int tiles_m, const int tiles_n, const int walk, int& tile_m, int& tile_n)
-{
-  const int xcd = b & 7, idx = b >> 3;
-  if (walk == kWalkBlocks) {
-    const int bm = tiles_m / 4, bn = tiles_n / 2;       // block of one XCD
-    tile_m = (xcd >> 1) * bm + idx / bn;
-    tile_n = (xcd & 1) * bn + idx % bn;
-  } else if (walk == kWalkRowMajor) {
-    tile_m = b / tiles_n;
-    tile_n = b % tiles_n;
-  } else {
-    const int rows = walk, tiles = tiles_m * tiles_n, each = tiles >> 3, more = tiles & 7;
-    const int at = xcd * each + (xcd < more ? xcd : more) + idx;
-    const int band = at / (rows * tiles_n), in_band = at - band * rows * tiles_n;
-    const int height = tiles_m - band * rows < rows ? tiles_m - band * rows : rows;
-    tile_n = in_band / height;
-    tile_m = band * rows + in_band - tile_n * height;
-  }
-}
-
-// The order in which the workgroups take the tiles; `per_cu` of them share a compute unit.  Every XCD has an L2 of its own, so the panels
-// of A and B behind the tiles that are in work on one XCD at a time should be few.
-//   blocks     grids that divide into 4 x 2: every XCD gets one compact block.  Not where the blocks are narrow strips with 1.8 times the panels
-//              of a band's share (128 x 128 tiles, us in blocks and in bands, from the caches and from DRAM: 512 x 16384 x 1024 28.2 / 22.3 and
-//              32.6 / 27.4; 1024 x 6144 x 2048 32.1 / 28.7 and 41.6 / 34.8; 512 x 8192 x 4096 43.5 / 41.0 and 46.2 / 44.3); with few K steps it is the writes of C
-//              that count (1024 x 16384 x 256, variant 1: 22.1 / 24.3), though not with tiles below 128 x 128 (256 x 5376 x 256 from DRAM 6.3 / 5.7).
-//              Between 1.5 and 1.8 times as many, only with many K steps (1536 x 7680 x 4096 from the caches 110.8 / 95.6, x 512 from DRAM 21.2 / 25.3)
-//              and where the last band is no thin rest (1024 x 5376 x 2048, eight rows in bands of seven: 28.0 / 30.3 and 31.3 / 37.8).
-//   bands      up to eight tile rows, down the columns of a band, an eighth of that walk for every XCD (dealt row-major instead:
-//              3712 x 4736 x 3712 with 128 x 128 tiles 188 us against 139, 640 x 8064 x 2048 34 / 28).  In grids that divide level or slower than
-//              blocks (8192 x 8192 x 1024, 256 x 256 tiles: 155 us against 140).
-//   row-major  where eight divides the tiles of a row, so that every XCD has columns of its own, and its rows and columns are then no more
-//              than with bands (7680 x 8192 x 384, 256 x 256 tiles: 79 us, bands 87; 640 x 8192 x 1024, 128 x 128: 15.5 / 16.8.  But
-//              16 rows and 4 columns against 8 and 8: 3712 x 4096 x 640 33.5 / 28.8 from DRAM; 15 and 2 against 6 and 5: 1920 x 2048 x 2048
-//              26.6 / 23.0); where one round of tiles is over in a few K steps and finding the place in a band counts (0.2 us: 640 x 4096 x 256
-//              5.4 / 5.6); and with two K steps of 64, when a tile is mostly its block of C and the bands scatter the writes of a large C, as long as
-//              an L2 holds B (from DRAM: 8064 x 8064 x 128 49 / 55, 4224 x 5760 x 128 20.7 / 22.9; 6528 x 896 x 128, a small C, 8.0 / 7.5;
-//              2176 x 7808 x 256 24.4 / 21.9).
+using dispatch::tile_of_workgroup;
 int tile_walk(const int m, const int n, const int k, const int tile_rows, const int tile_cols, const int per_cu)
 {
-  const int tiles_m = m / tile_rows, tiles_n = n / tile_cols;
-  const int cus = workloads::device_cus();
-  const long long tiles = (long long)tiles_m * tiles_n, each = tiles / 8;
-  int rows = 1;
-  while (rows < 8 && rows * rows < each) ++rows;
-  const int high = tiles_m < rows ? tiles_m : rows;
-  const long long of_block = tiles_m / 4 + tiles_n / 2, of_band = high + each / high;                     // panels behind a block and behind a band's share
-  const bool narrow = (5 * of_block > 9 * of_band && (k >= 512 || tile_rows < 128)) || (2 * of_block > 3 * of_band && k >= 2048 && 2 * (tiles_m % rows) >= rows);
-  if ((tiles_m % 4) == 0 && (tiles_n % 2) == 0 && !narrow) return kWalkBlocks;
-  const double in_work = (double)(each < per_cu * cus / 8 ? each : per_cu * cus / 8), columns = tiles_n / 8;
-  const bool own_columns = (tiles_n % 8) == 0 && in_work / columns + columns <= rows + in_work / rows + 1;
-  const bool mostly_c = k < 256 && (long long)n * k < (3 << 19) && (long long)m * n >= (16 << 20);
-  return own_columns || mostly_c || (tiles <= cus && k < 512) ? kWalkRowMajor : rows;
+  return dispatch::tile_walk(m, n, k, tile_rows, tile_cols, per_cu, workloads::device_cus());
 }
 
 // Order of one slice for the instruction scheduler: MFMAs matrix instructions with the READS

@@ -1,0 +1,71 @@
+"""The rules by which the default variants choose kernels and launch shapes (cudadma_amd/csrc/dispatch.hpp), evaluated on the host for the
+256 compute units of an MI355X."""
+import ctypes
+import os
+import shutil
+import subprocess
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+CUS = 256
+BLOCKS, ROW_MAJOR = 0, -1
+
+_SHIM = r"""
+#include "dispatch.hpp"
+extern "C" int tile_walk(int m, int n, int k, int rows, int cols, int per_cu, int cus) { return dispatch::tile_walk(m, n, k, rows, cols, per_cu, cus); }
+// every tile once?
+extern "C" int visits_once(int tiles_m, int tiles_n, int walk, int* seen)
+{
+  for (int b = 0; b < tiles_m * tiles_n; ++b) {
+    int i = -1, j = -1;
+    dispatch::tile_of_workgroup(b, tiles_m, tiles_n, walk, i, j);
+    if (i < 0 || i >= tiles_m || j < 0 || j >= tiles_n || seen[i * tiles_n + j]++) return 0;
+  }
+  return 1;
+}
+"""
+
+
+@pytest.fixture(scope="module")
+def rules(tmp_path_factory):
+    cxx = shutil.which("g++") or shutil.which("clang++") or shutil.which("hipcc")
+    if cxx is None:
+        pytest.skip("no C++ compiler")
+    at = tmp_path_factory.mktemp("dispatch")
+    (at / "shim.cpp").write_text(_SHIM)
+    subprocess.run([cxx, "-std=c++17", "-O2", "-Wall", "-Wextra", "-Werror", "-shared", "-fPIC", "-I", os.path.join(ROOT, "cudadma_amd", "csrc"),
+                    str(at / "shim.cpp"), "-o", str(at / "shim.so")], check=True)
+    return ctypes.CDLL(str(at / "shim.so"))
+
+
+def test_every_tile_has_one_workgroup(rules):
+    """All walks that the rule can choose, over grids of one tile to several rounds."""
+    for tiles_m in (1, 2, 3, 4, 5, 8, 11, 12, 16, 29, 60, 64):
+        for tiles_n in (1, 2, 5, 8, 17, 24, 34, 66, 128):
+            for walk in range(ROW_MAJOR, 9):
+                if walk == BLOCKS and (tiles_m % 4 or tiles_n % 2):
+                    continue
+                assert rules.visits_once(tiles_m, tiles_n, walk, (ctypes.c_int * (tiles_m * tiles_n))()), (tiles_m, tiles_n, walk)
+
+
+# m, n, k, tile, workgroups of a compute unit: grids that divide into 4 x 2, on both sides of every line
+@pytest.mark.parametrize("shape, tile, per_cu, walk", [
+    # columns of their own
+    ((1024, 6144, 2048), 128, 2, ROW_MAJOR), ((512, 8192, 1024), 128, 1, ROW_MAJOR), ((1536, 8192, 2048), 128, 2, ROW_MAJOR),
+    ((1024, 5120, 1024), 128, 2, BLOCKS), ((1024, 5120, 4096), 128, 2, BLOCKS), ((1536, 8192, 1024), 128, 2, BLOCKS), ((1024, 6144, 384), 128, 2, BLOCKS),
+    # one band of four rows
+    ((512, 16384, 512), 128, 2, 4), ((512, 8448, 2048), 128, 2, 4), ((1024, 9728, 1024), 256, 1, 4), ((512, 16384, 256), 128, 2, BLOCKS),
+    # one band of eight, and of seven with one row left over
+    ((1024, 6912, 512), 128, 2, BLOCKS), ((1024, 7936, 4096), 128, 2, BLOCKS), ((2048, 13312, 1024), 256, 1, BLOCKS), ((1024, 11776, 2048), 128, 2, 8),
+    ((1024, 11776, 512), 128, 2, BLOCKS), ((1024, 5632, 2048), 128, 2, BLOCKS),
+    # several bands: dividing the rows evenly, and with a half left over
+    ((2048, 8960, 2048), 128, 2, 8), ((2048, 8960, 1024), 128, 2, BLOCKS), ((1536, 7424, 2048), 128, 2, BLOCKS), ((1536, 11008, 1536), 128, 2, 8),
+    ((1536, 9984, 512), 128, 2, BLOCKS), ((8192, 8192, 1024), 256, 1, BLOCKS),
+    # tiles below 128 x 128
+    ((128, 2048, 768), 32, 2, ROW_MAJOR), ((256, 2176, 512), 64, 2, 4), ((3840, 256, 2048), 64, 2, 6), ((5376, 256, 2048), 64, 2, 7),
+    ((512, 2304, 2048), 64, 2, BLOCKS), ((1024, 1024, 1024), 64, 1, BLOCKS)])
+def test_walk_of_grids_in_blocks_or_narrow(rules, shape, tile, per_cu, walk):
+    got = rules.tile_walk(*shape, tile, tile, per_cu, CUS)
+    # a band is no higher than the grid
+    assert (got if got <= 0 else min(got, shape[0] // tile)) == walk

@@ -646,6 +646,16 @@ def test_gemm_long_rows(device):
     assert torch.equal(got, some.float() @ other.float())
 
 
+# grids that divide into eight blocks and walk otherwise (columns of their own, one band of four or of eight rows, bands that divide the rows evenly,
+# several bands with a rest), each beside one that stays in blocks; tiles of 128 x 128 in both variants, of 256 x 256 by default for the last row
+@pytest.mark.parametrize("shape", [(512, 8192, 512), (1024, 6144, 512), (1024, 5120, 512), (512, 8448, 512), (1024, 6912, 512), (1024, 11776, 1024),
+                                   (2048, 8448, 2048), (2048, 8448, 1920), (1536, 11008, 1024), (1536, 11008, 896),
+                                   (1024, 9728, 1024), (2048, 13312, 512)])
+@pytest.mark.parametrize("variant", [0, 1])
+def test_gemm_walks_of_narrow_grids(device, shape, variant):
+    test_gemm_tile_walks(device, shape, variant)
+
+
 def test_gemm_rejects_ragged_shapes(device):
     a = torch.zeros((100, 128), dtype=torch.bfloat16, device=device)
     b = torch.zeros((128, 128), dtype=torch.bfloat16, device=device)
