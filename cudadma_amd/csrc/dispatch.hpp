@@ -43,7 +43,9 @@ DISPATCH_FN void tile_of_workgroup(const int b, const int tiles_m, const int til
 //   row-major  where eight divides the tiles of a row, so that every XCD has columns of its own, and its rows and columns are then no more
 //              than with bands (7680 x 8192 x 384, 256 x 256 tiles: 79 us, bands 87; 640 x 8192 x 1024, 128 x 128: 15.5 / 16.8.  But
 //              16 rows and 4 columns against 8 and 8: 3712 x 4096 x 640 33.5 / 28.8 from DRAM; 15 and 2 against 6 and 5: 1920 x 2048 x 2048
-//              26.6 / 23.0); where one round of tiles is over in a few K steps and finding the place in a band counts (0.2 us: 640 x 4096 x 256
+//              26.6 / 23.0.  Tiles below 128 x 128 compare with the rows that the grid has, two or four often, in bands of which B is what counts: bands /
+//              row-major 256 x 5120 x 2432 24 % and 31 %, 256 x 7680 x 512 3 % and 21 %, 128 x 9728 x 512 3 % and 25 %; with 128 x 128 the same count would
+//              lose, 640 x 11264 x 7040 6 % and 8 %); where one round of tiles is over in a few K steps and finding the place in a band counts (0.2 us: 640 x 4096 x 256
 //              5.4 / 5.6); and with two K steps of 64, when a tile is mostly its block of C and the bands scatter the writes of a large C, as long as
 //              an L2 holds B (from DRAM: 8064 x 8064 x 128 49 / 55, 4224 x 5760 x 128 20.7 / 22.9; 6528 x 896 x 128, a small C, 8.0 / 7.5;
 //              2176 x 7808 x 256 24.4 / 21.9).
@@ -68,12 +70,12 @@ inline int tile_walk(const int m, const int n, const int k, const int tile_rows,
   int rows = 1;
   while (rows < 8 && rows * rows < each) ++rows;
   const double in_work = (double)(each < per_cu * cus / 8 ? each : per_cu * cus / 8), columns = tiles_n / 8;
-  const bool own_columns = (tiles_n % 8) == 0 && in_work / columns + columns <= rows + in_work / rows + 1;
+  const int high = tiles_m < rows ? tiles_m : rows, rest = tiles_m % rows, height = tile_rows < 128 ? high : rows;
+  const bool own_columns = (tiles_n % 8) == 0 && in_work / columns + columns <= height + in_work / height + 1;
   const bool mostly_c = k < 256 && (long long)n * k < (3 << 19) && (long long)m * n >= (16 << 20);
   const int other = own_columns || mostly_c || (tiles <= cus && k < 512) ? kWalkRowMajor : rows;
   if ((tiles_m % 4) != 0 || (tiles_n % 2) != 0) return other;
 
-  const int high = tiles_m < rows ? tiles_m : rows, rest = tiles_m % rows;
   const long long of_block = tiles_m / 4 + tiles_n / 2, of_band = high + each / high;        // panels behind a block and behind a band's share
   const bool times_1_5 = 2 * of_block > 3 * of_band, times_1_8 = 5 * of_block > 9 * of_band, times_13_7 = 7 * of_block >= 13 * of_band,
              times_2_5 = 2 * of_block >= 5 * of_band;

@@ -64,7 +64,10 @@ def test_every_tile_has_one_workgroup(rules):
     ((1536, 9984, 512), 128, 2, BLOCKS), ((8192, 8192, 1024), 256, 1, BLOCKS),
     # tiles below 128 x 128
     ((128, 2048, 768), 32, 2, ROW_MAJOR), ((256, 2176, 512), 64, 2, 4), ((3840, 256, 2048), 64, 2, 6), ((5376, 256, 2048), 64, 2, 7),
-    ((512, 2304, 2048), 64, 2, BLOCKS), ((1024, 1024, 1024), 64, 1, BLOCKS)])
+    ((512, 2304, 2048), 64, 2, BLOCKS), ((1024, 1024, 1024), 64, 1, BLOCKS),
+    # columns of their own in grids with fewer rows than a band may have
+    ((256, 7680, 512), 64, 2, ROW_MAJOR), ((256, 5120, 2432), 64, 2, ROW_MAJOR), ((128, 9728, 512), 64, 2, ROW_MAJOR), ((256, 7552, 768), 64, 2, 4),
+    ((640, 11264, 7040), 128, 2, 5)])
 def test_walk_of_grids_in_blocks_or_narrow(rules, shape, tile, per_cu, walk):
     got = rules.tile_walk(*shape, tile, tile, per_cu, CUS)
     # a band is no higher than the grid

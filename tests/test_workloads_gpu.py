@@ -647,10 +647,11 @@ def test_gemm_long_rows(device):
 
 
 # grids that divide into eight blocks and walk otherwise (columns of their own, one band of four or of eight rows, bands that divide the rows evenly,
-# several bands with a rest), each beside one that stays in blocks; tiles of 128 x 128 in both variants, of 256 x 256 by default for the last row
+# several bands with a rest), each beside one that stays in blocks; tiles of 128 x 128 in both variants, by default of 256 x 256 for the first two of
+# the last row and of 64 x 64 for the others
 @pytest.mark.parametrize("shape", [(512, 8192, 512), (1024, 6144, 512), (1024, 5120, 512), (512, 8448, 512), (1024, 6912, 512), (1024, 11776, 1024),
                                    (2048, 8448, 2048), (2048, 8448, 1920), (1536, 11008, 1024), (1536, 11008, 896),
-                                   (1024, 9728, 1024), (2048, 13312, 512)])
+                                   (1024, 9728, 1024), (2048, 13312, 512), (256, 7680, 512), (256, 7552, 512), (128, 9728, 512)])
 @pytest.mark.parametrize("variant", [0, 1])
 def test_gemm_walks_of_narrow_grids(device, shape, variant):
     test_gemm_tile_walks(device, shape, variant)
