@@ -89,4 +89,55 @@ inline int tile_walk(const int m, const int n, const int k, const int tile_rows,
   return narrow ? other : kWalkBlocks;
 }
 
+// ---- GEMM: the kernel of the default variant ----
+// Whether the rows of one round of direct-to-LDS loads (32 of A, 16 of B) span less than the 4 GiB of a lane offset.
+inline bool direct_rows_fit(const long long n, const long long k)
+{
+  return 32 * (k * 2) + 128 <= 0xffffffffLL && 16 * (n * 2) + 256 <= 0xffffffffLL;
+}
+
+enum class GemmForm { kLongRows, kDealt32x32, kDealt32x64, kDealt64x64, kDealt64x64Two, k128Far, k128, k256 };
+inline GemmForm gemm_form(const int m, const int n, const int k, const int compute_units)
+{
+  const long long cus = compute_units;
+  // Longer rows go through variant 1, whose transfers take a 64-bit offset for every row.
+  if (!direct_rows_fit(n, k)) return GemmForm::kLongRows;
+
+  // Grids of few tiles take the smallest tile that still gives every compute unit at most one (32 x 32, 32 x 64, 64 x 64) or, with half as
+  // many wavefronts, two workgroups (64 x 64).  us with those four and with 128 x 128, from the caches: 512 x 512 x 512 3.5 / 3.7 / 4.6 / 4.6 / 6.0;
+  // 640 x 512 x 1152 6.0 / 4.8 / 6.0 / 6.4 / 9.8; 768^3 6.7 / 7.0 / 5.3 / 5.5 / 7.8; 1024 x 1152 x 1920 - / - / 15.2 / 12.6 / 14.8 and from DRAM
+  // 17.0 / 14.8 / 20.4.  The last one has a wavefront only two or three steps below k = 512, and
+  // then 128 x 128 is as fast or faster (1152 x 1792 x 256 from the caches 5.5 / 5.1, from DRAM 5.9 / 5.7; x 512 6.4 / 6.6 and 7.0 / 7.5; x 768 7.7 / 8.1 and 8.8 / 10.0).
+  // With long rows 128 x 128 has caught up (256 x 6656 x 6144 45.0 / 42.0 and 63.4 / 61.3; 768 x 2560 x 3072 24.0 / 22.3 and 29.7 / 30.7); where
+  // nearly every compute unit has two of them it does so from k = 1900 on from the caches, not from DRAM (2304 x 1536 x 2304 7 % slower and 21 % faster, 1152 x 2432 x
+  // 1920 1 % faster and 18 %).  A product of two rows of more than 80 of them is nearly all B, which a tile of 64 columns fetches in pieces of
+  // 128 bytes: 128 x 128 is ahead there from k = 1024 on (128 x 11776 x 2176 10 % and 8 %, 128 x 14464 x 1664 5 % and 4 %, 128 x 16384 x 1024 0 % and 7 %; 128 x 10624 x 1536
+  // 2 % slower and 1 % faster.  With 80 128 x 10240 x 1792 is 7 % and 19 % slower).
+  const long long t32 = (long long)(m / 32) * (n / 32);
+  if (t32 <= cus) return GemmForm::kDealt32x32;
+  if (t32 <= 2 * cus) return GemmForm::kDealt32x64;
+  if (t32 <= 4 * cus) return GemmForm::kDealt64x64;
+  if (t32 <= 8 * cus && k >= 512 && k < (m == 128 && t32 > 5 * cus ? 1024 : 3072)) return GemmForm::kDealt64x64Two;
+
+  // Variant 9 with its tile of 256 x 256 or the same kernel with 128 x 128, whichever takes its rounds over the compute units in less time.
+  // `full` is the time of a K step of 64 of a whole round in units of 10 ns, `part` that of a round of few workgroups: up to one per
+  // compute unit for the small tile, of which two share one, up to five eighths of them for the large one (they get more of the
+  // clock and the memory); `once` is what a tile costs before its first and after its last K step.  Measured, 256 / 128:
+  // 1536 x 7680 x 1280 38 / 44 us, 2816 x 5888 x 1024 39 / 42, 7424 x 2304 x 2048 99 / 81, 2048^3 41 / 23, 2560 x 2560 x 1024 25 / 18.  The tiles of variants 2 and 3
+  // lie between and win nowhere.
+  auto rounds = [&](const long long tiles, const long long slots, const long long few, const int full, const int part, const int once) {
+    const long long rest = tiles % slots;
+    return (k / 64) * (tiles / slots * full + (rest == 0 ? 0 : rest <= few ? part : full)) + once;
+  };
+  const long long grid = (long long)(m / 128) * (n / 128);
+  const long long small = rounds(grid, 2 * cus, cus, 100, 58, 400);
+  const bool even = (m % 256) == 0 && (n % 256) == 0;
+  if (even && rounds((long long)(m / 256) * (n / 256), cus, cus * 5 / 8, 160, 110, 1000) < small) return GemmForm::k256;
+  // One tile or none for a compute unit: requests that run further ahead, from the k on at which <2, 4> loses from DRAM what it gained
+  // over the warp-specialised kernel (us, <2, 4> / <2, 8> from the caches, <2, 4> / <2, 8> / variant 1 from DRAM): 2048 x 2048 x 640
+  // 9.4 / 9.9, 10.2 / 10.3 / 10.6; x 768 10.3 / 10.5, 13.4 / 12.3 / 12.3; x 1280 15.1 / 15.2, 19.2 / 17.1 / 16.9; x 2048 23.3 / 20.9,
+  // 28.7 / 24.2 / 24.6; 768 x 2048 x 4736 40 / 33, 56 / 45.
+  return grid <= cus && k >= 768 ? GemmForm::k128Far : GemmForm::k128;
+}
+
 }  // namespace dispatch

@@ -1274,10 +1274,15 @@ int launch_gemm(const uint16_t* d_a, const uint16_t* d_b, float* d_c, int m, int
   return CUDADMA_OK;
 }
 
-// Whether the rows of one round of direct-to-LDS loads (32 of A, 16 of B) span less than the 4 GiB of a lane offset.
-bool direct_rows_fit(const long long n, const long long k)
+template<int B_STAGES>
+int launch_all_direct_128(const uint16_t* d_a, const uint16_t* d_b, float* d_c, int m, int n, int k, hipStream_t stream)
 {
-  return 32 * (k * 2) + 128 <= 0xffffffffLL && 16 * (n * 2) + 256 <= 0xffffffffLL;
+  const long long grid = (long long)(m / 128) * (n / 128);
+  CUDADMA_REQUIRE(grid <= 0x7fffffffLL, "grid too large");
+  hipLaunchKernelGGL((gemm_bf16_all_direct_a64<2, B_STAGES>), dim3((unsigned)grid), dim3(256), 0, stream, d_a, d_b, d_c, m, n, k,
+                     tile_walk(m, n, k, 128, 128, B_STAGES == 8 ? 1 : 2));
+  CUDADMA_HIP_CHECK(hipGetLastError());
+  return CUDADMA_OK;
 }
 
 }  // namespace
@@ -1298,44 +1303,16 @@ extern "C" int cudadma_gemm_bf16(const uint16_t* d_a, const uint16_t* d_b, float
   CUDADMA_REQUIRE((long long)k * 2 <= 0x7fffffffLL && (long long)n * 2 <= 0x7fffffffLL, "row pitch must fit an int");
   hipStream_t s = (hipStream_t)stream;
   if (variant == 0) {
-    // Variant 9 with its tile of 256 x 256 or the same kernel with 128 x 128, whichever takes its rounds over the compute units in less time.
-    // `full` is the time of a K step of 64 of a whole round in units of 10 ns, `part` that of a round of few workgroups: up to one per
-    // compute unit for the small tile, of which two share one, up to five eighths of them for the large one (they get more of the
-    // clock and the memory); `once` is what a tile costs before its first and after its last K step.  Measured, 256 / 128:
-    // 1536 x 7680 x 1280 38 / 44 us, 2816 x 5888 x 1024 39 / 42, 7424 x 2304 x 2048 99 / 81, 2048^3 41 / 23, 2560 x 2560 x 1024 25 / 18.  The tiles of variants 2 and 3
-    // lie between and win nowhere.  Both load with 32-bit lane offsets, a round of 32 rows of A or 16 of B at a time; longer rows
-    // go through variant 1, whose transfers take a 64-bit offset for every row.
-    const long long cus = workloads::device_cus();
-    auto rounds = [&](const long long tiles, const long long slots, const long long few, const int full, const int part, const int once) {
-      const long long rest = tiles % slots;
-      return (k / kBK) * (tiles / slots * full + (rest == 0 ? 0 : rest <= few ? part : full)) + once;
-    };
-    const long long small = rounds((long long)(m / 128) * (n / 128), 2 * cus, cus, 100, 58, 400);
-    const bool even = (m % 256) == 0 && (n % 256) == 0;
-    // Grids of few tiles take the smallest tile that still gives every compute unit at most one (32 x 32, 32 x 64, 64 x 64) or, with half as
-    // many wavefronts, two workgroups (64 x 64).  us with those four and with 128 x 128, from the caches: 512 x 512 x 512 3.5 / 3.7 / 4.6 / 4.6 / 6.0;
-    // 640 x 512 x 1152 6.0 / 4.8 / 6.0 / 6.4 / 9.8; 768^3 6.7 / 7.0 / 5.3 / 5.5 / 7.8; 1024 x 1152 x 1920 - / - / 15.2 / 12.6 / 14.8 and from DRAM
-    // 17.0 / 14.8 / 20.4.  The last one has a wavefront only two or three steps below k = 512, and
-    // then 128 x 128 is as fast or faster (1152 x 1792 x 256 from the caches 5.5 / 5.1, from DRAM 5.9 / 5.7; x 512 6.4 / 6.6 and 7.0 / 7.5; x 768 7.7 / 8.1 and 8.8 / 10.0).
-    // With long rows 128 x 128 has caught up (256 x 6656 x 6144 45.0 / 42.0 and 63.4 / 61.3; 768 x 2560 x 3072 24.0 / 22.3 and 29.7 / 30.7).
-    const long long t32 = (long long)(m / 32) * (n / 32);
-    if (!direct_rows_fit(n, k)) variant = 1;
-    else if (t32 <= cus) return launch_dealt_steps<1, 1, 8>(d_a, d_b, d_c, m, n, k, s);
-    else if (t32 <= 2 * cus) return launch_dealt_steps<1, 2, 8>(d_a, d_b, d_c, m, n, k, s);
-    else if (t32 <= 4 * cus) return launch_dealt_steps<2, 2, 8>(d_a, d_b, d_c, m, n, k, s);
-    else if (t32 <= 8 * cus && k >= 512 && k < 3072) return launch_dealt_steps<2, 2, 4>(d_a, d_b, d_c, m, n, k, s);
-    else if (even && rounds((long long)(m / 256) * (n / 256), cus, cus * 5 / 8, 160, 110, 1000) < small) variant = 9;
-    else {
-      const long long grid = (long long)(m / 128) * (n / 128);
-      CUDADMA_REQUIRE(grid <= 0x7fffffffLL, "grid too large");
-      // One tile or none for a compute unit: requests that run further ahead, from the k on at which <2, 4> loses from DRAM what it gained
-      // over the warp-specialised kernel (us, <2, 4> / <2, 8> from the caches, <2, 4> / <2, 8> / variant 1 from DRAM): 2048 x 2048 x 640
-      // 9.4 / 9.9, 10.2 / 10.3 / 10.6; x 768 10.3 / 10.5, 13.4 / 12.3 / 12.3; x 1280 15.1 / 15.2, 19.2 / 17.1 / 16.9; x 2048 23.3 / 20.9,
-      // 28.7 / 24.2 / 24.6; 768 x 2048 x 4736 40 / 33, 56 / 45.
-      if (grid <= cus && k >= 768) hipLaunchKernelGGL((gemm_bf16_all_direct_a64<2, 8>), dim3((unsigned)grid), dim3(256), 0, s, d_a, d_b, d_c, m, n, k, tile_walk(m, n, k, 128, 128, 1));
-      else hipLaunchKernelGGL((gemm_bf16_all_direct_a64<2, 4>), dim3((unsigned)grid), dim3(256), 0, s, d_a, d_b, d_c, m, n, k, tile_walk(m, n, k, 128, 128, 2));
-      CUDADMA_HIP_CHECK(hipGetLastError());
-      return CUDADMA_OK;
+    using dispatch::GemmForm;
+    switch (dispatch::gemm_form(m, n, k, workloads::device_cus())) {
+      case GemmForm::kDealt32x32: return launch_dealt_steps<1, 1, 8>(d_a, d_b, d_c, m, n, k, s);
+      case GemmForm::kDealt32x64: return launch_dealt_steps<1, 2, 8>(d_a, d_b, d_c, m, n, k, s);
+      case GemmForm::kDealt64x64: return launch_dealt_steps<2, 2, 8>(d_a, d_b, d_c, m, n, k, s);
+      case GemmForm::kDealt64x64Two: return launch_dealt_steps<2, 2, 4>(d_a, d_b, d_c, m, n, k, s);
+      case GemmForm::k128Far: return launch_all_direct_128<8>(d_a, d_b, d_c, m, n, k, s);
+      case GemmForm::k128: return launch_all_direct_128<4>(d_a, d_b, d_c, m, n, k, s);
+      case GemmForm::k256: variant = 9; break;
+      case GemmForm::kLongRows: variant = 1; break;
     }
   }
   switch (variant) {
@@ -1348,7 +1325,7 @@ extern "C" int cudadma_gemm_bf16(const uint16_t* d_a, const uint16_t* d_b, float
     case 6: case 7: case 8: case 9: {
       CUDADMA_REQUIRE((m % 256) == 0 && (n % 256) == 0, "this variant needs m and n multiples of 256 (got %d x %d)", m, n);
       // 6 and 7 go over to 64-bit row offsets by themselves (issue_direct), 8 and 9 are compiled for lane offsets alone
-      CUDADMA_REQUIRE(variant <= 7 || direct_rows_fit(n, k), "rows of %d x %d are too long for the lane offsets of this variant (0, 1 and 7 take them)", k, n);
+      CUDADMA_REQUIRE(variant <= 7 || dispatch::direct_rows_fit(n, k), "rows of %d x %d are too long for the lane offsets of this variant (0, 1 and 7 take them)", k, n);
       const long long grid = (long long)(m / 256) * (n / 256);
       CUDADMA_REQUIRE(grid <= 0x7fffffffLL, "grid too large");
       const int walk = tile_walk(m, n, k, 256, 256, 1);

@@ -14,6 +14,7 @@ BLOCKS, ROW_MAJOR = 0, -1
 _SHIM = r"""
 #include "dispatch.hpp"
 extern "C" int tile_walk(int m, int n, int k, int rows, int cols, int per_cu, int cus) { return dispatch::tile_walk(m, n, k, rows, cols, per_cu, cus); }
+extern "C" int gemm_form(int m, int n, int k, int cus) { return (int)dispatch::gemm_form(m, n, k, cus); }
 // every tile once?
 extern "C" int visits_once(int tiles_m, int tiles_n, int walk, int* seen)
 {
@@ -72,3 +73,17 @@ def test_walk_of_grids_in_blocks_or_narrow(rules, shape, tile, per_cu, walk):
     got = rules.tile_walk(*shape, tile, tile, per_cu, CUS)
     # a band is no higher than the grid
     assert (got if got <= 0 else min(got, shape[0] // tile)) == walk
+
+
+LONG_ROWS, DEALT_32, DEALT_32_64, DEALT_64, DEALT_64_TWO, TILE_128_FAR, TILE_128, TILE_256 = range(8)
+
+
+@pytest.mark.parametrize("shape, form", [
+    ((512, 512, 512), DEALT_32), ((640, 512, 8192), DEALT_32_64), ((1024, 1024, 128), DEALT_64), ((128, 8192, 128), DEALT_64),
+    ((1152, 1024, 384), TILE_128), ((1152, 1024, 512), DEALT_64_TWO), ((256, 8192, 3008), DEALT_64_TWO), ((256, 8192, 3072), TILE_128_FAR),
+    # two rows of 64 x 64 tiles
+    ((128, 10368, 896), DEALT_64_TWO), ((128, 10368, 1024), TILE_128_FAR), ((128, 10240, 2048), DEALT_64_TWO), ((128, 16384, 2048), TILE_128_FAR),
+    ((128, 8320, 384), TILE_128), ((2176, 1024, 640), TILE_128), ((2176, 1024, 768), TILE_128_FAR), ((2048, 2048, 1920), TILE_128_FAR),
+    ((2048, 2176, 1920), TILE_128), ((4096, 4096, 4096), TILE_256), ((1408, 2176, 1920), TILE_128_FAR), ((128, 128, 71_600_128), LONG_ROWS)])
+def test_kernel_of_the_default_gemm(rules, shape, form):
+    assert rules.gemm_form(*shape, CUS) == form

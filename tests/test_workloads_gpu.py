@@ -605,7 +605,7 @@ def test_gemm_tile_walks(device, shape, variant):
 
 # the default variant's form with eight stages of B (one tile or none for a compute unit, from 768 columns of A on): K steps that end in
 # either half of its loop, and both sides of the lines to its neighbours
-@pytest.mark.parametrize("m, n", [(128, 128), (1408, 2176), (2048, 2048), (2048, 2176)])
+@pytest.mark.parametrize("m, n", [(128, 128), (1408, 2176), (2048, 2048), (2048, 2176), (128, 10368)])
 @pytest.mark.parametrize("k", [384, 640, 768, 896, 1920])
 def test_gemm_stages(device, m, n, k):
     a = wl.fill_normal_bf16(torch.empty((m, k), dtype=torch.bfloat16, device=device), 63)
