@@ -140,4 +140,30 @@ inline GemmForm gemm_form(const int m, const int n, const int k, const int compu
   return grid <= cus && k >= 768 ? GemmForm::k128Far : GemmForm::k128;
 }
 
+// ---- copy: the kernel of the default variant ----
+// Two operating points, as for every read + write stream on this part: a working set (both buffers) that the 256 MB Infinity
+// Cache holds from launch to launch wants many tiles in flight (two LDS tiles, four workgroups per compute unit);
+// beyond it the memory system serves a short queue better (one LDS tile, two workgroups per compute unit: 1 GiB in 0.353 ms
+// against 0.408 ms).  Stores are non-temporal throughout, which leaves the caches to the input.  us from the caches, from DRAM, and with three sets of
+// buffers in turn, of which the caches hold a part:
+//            plain stores, two tiles    one tile, four workgroups    two tiles, streaming loads    two tiles, plain loads
+//   16 MiB   5.6   7.5   7.3            5.5   6.1   5.6              5.5   6.3   5.7               4.4   6.4   6.8
+//   32 MiB   11.2  11.7  10.9           11.2  12.5  12.0             9.6   11.9  11.4              8.9   11.6  11.5
+//   40 MiB   13.3  18.2  13.2           13.3  15.3  14.8             13.0  14.8  14.2              13.9  15.4  13.6
+//   44 MiB   14.5  18.4  16.5           14.7  16.6  16.0             14.4 to 15.6  16.0  15.4      15.0  16.8  14.7
+//   46 MiB   15.3  20.7  18.0           15.3  17.3  16.6             15.2 to 16.9  17.5  16.8      15.7  18.2  15.4
+//   48 MiB   15.8  21.3  20.5           16.6  17.9  17.4             15.8 to 17.5  17.7  17.2      16.2  18.3  15.9
+//   64 MiB   20.9  25.0  24.8           22.1  23.4  22.7             21.1 to 23.6  24.1  23.3      21.1  24.8  20.7
+//   96 MiB   30.6  39.0  38.3           32.2  34.0  33.2             32.5  34.4  33.0              30.7  35.9  33.9
+// Up to 16 MiB the one tile starts sooner with inputs that come from memory.  Streaming loads end at 44 MiB: beyond, they lose up to a tenth
+// with the same buffer again and again, by where it lies, and as much with three in turn.
+constexpr unsigned long long kCacheAssistedBytes = 192ull << 20;
+enum class CopyForm { kOneTileFour, kTwoTilesStreaming, kTwoTiles, kOneTileTwo };
+inline CopyForm copy_form(const unsigned long long bytes)
+{
+  if (bytes <= 16ull << 20) return CopyForm::kOneTileFour;
+  if (bytes <= 44ull << 20) return CopyForm::kTwoTilesStreaming;
+  return 2 * bytes <= kCacheAssistedBytes ? CopyForm::kTwoTiles : CopyForm::kOneTileTwo;
+}
+
 }  // namespace dispatch

@@ -45,9 +45,9 @@ int tuning(const char* name, int fallback)
 }
 
 static const VariantInfo kSequential[] = {
-  {"manual double buffer: one DMA group of 2 wavefronts, two objects, two-phase calls, registers -> ds_write_b128, non-temporal stores, four "
-   "workgroups per compute unit; for up to 16 MiB variant 5 with four of them, for more than 96 MiB (a working set beyond the Infinity "
-   "Cache) variant 5 instead"},
+  {"manual double buffer: one DMA group of 2 wavefronts, two objects, two-phase calls, registers -> ds_write_b128, non-temporal stores, up to "
+   "44 MiB streaming loads, four workgroups per compute unit; for up to 16 MiB variant 5 with four of them, for more than 96 MiB (a working "
+   "set beyond the Infinity Cache) variant 5 instead"},
   {"single buffer: one object, execute_dma"},
   {"double buffer: two DMA groups of 1 wavefront, one object each"},
   {"manual double buffer with STORE_LDS_DIRECT (global_load_lds_dwordx4, no VGPR staging)"},

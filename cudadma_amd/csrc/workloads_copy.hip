@@ -3,6 +3,7 @@
 // Kernel shapes follow src/perf/sequential/perf_sequential.cu:52-223
 // (non_specialized / single_buffer / double_buffer / manual_buffer), with a
 // consumer that really writes the tile back instead of a dead branch.
+#include "dispatch.hpp"
 #include "workloads.hpp"
 
 namespace {
@@ -13,7 +14,6 @@ constexpr int kDmaThreads = 128;
 constexpr int kComputeThreads = 128;
 constexpr int kTileVecs = kTileBytes / 16;
 constexpr int kVecsPerConsumer = kTileVecs / kComputeThreads;   // 8 ds_read_b128 per compute thread
-constexpr size_t kCacheAssistedBytes = 192u << 20;             // read + written bytes that still sit in the 256 MB Infinity Cache
 
 // Consumer: LDS tile -> registers, release the buffer, registers -> global (STREAM: non-temporal stores).
 template<bool STREAM = false, typename Dma>
@@ -316,23 +316,20 @@ extern "C" int cudadma_sequential_copy(const float* d_in, float* d_out, size_t b
   const dim3 block(kDmaThreads + kComputeThreads);
   switch (variant) {
     case 0:
-      // Two operating points, as for every read + write stream on this part: a working set that the 256 MB Infinity
-      // Cache holds from launch to launch wants many tiles in flight (two LDS tiles, four workgroups per compute unit);
-      // beyond it the memory system serves a short queue better (one LDS tile, two workgroups per compute unit: 1 GiB in 0.353 ms
-      // against 0.408 ms).  Stores are non-temporal throughout, which leaves the caches to the input: with plain ones, from the caches and
-      // from DRAM, 16 MiB 5.6 us and 7.5, now 4.4 and 6.2; 32 MiB 11.3 and 11.6, now 9.0 and 11.7; 64 MiB 20.9 and 25.2, now 21.1 and 25.0; 94 MiB
-      // 30.0 and 39.3, now 30.0 and 35.7.  Up to 48 MiB the loads are too (48 MiB 15.8 and 21.4, now 15.9 and 17.7; beyond, they lose from the
-      // caches: 56 MiB 18.3 / 19.5, 64 MiB 20.9 / 23.6, and with two buffers in turn, 24.3 / 23.0 where plain loads take 20.0), and up to
-      // 16 MiB the form with one LDS tile and four workgroups per compute unit starts sooner (16 MiB: two LDS tiles 4.4 and 6.4; 32 MiB:
-      // one 8.6 and 12.4).
-      if (2 * bytes <= kCacheAssistedBytes / 6)
-        hipLaunchKernelGGL(copy_single<true>, dim3(workloads::persistent_grid(tiles, 4)), block, 0, s, in, out, tiles);
-      else if (2 * bytes <= kCacheAssistedBytes / 2)
-        hipLaunchKernelGGL((copy_manual_double<STORE_LDS, true, LOAD_CACHE_STREAMING>), dim3(workloads::persistent_grid(tiles, 4)), block, 0, s, in, out, tiles);
-      else if (2 * bytes <= kCacheAssistedBytes)
-        hipLaunchKernelGGL((copy_manual_double<STORE_LDS, true>), dim3(workloads::persistent_grid(tiles, 4)), block, 0, s, in, out, tiles);
-      else
-        hipLaunchKernelGGL(copy_single<true>, dim3(workloads::persistent_grid(tiles, 2)), block, 0, s, in, out, tiles);
+      switch (dispatch::copy_form(bytes)) {
+        case dispatch::CopyForm::kOneTileFour:
+          hipLaunchKernelGGL(copy_single<true>, dim3(workloads::persistent_grid(tiles, 4)), block, 0, s, in, out, tiles);
+          break;
+        case dispatch::CopyForm::kTwoTilesStreaming:
+          hipLaunchKernelGGL((copy_manual_double<STORE_LDS, true, LOAD_CACHE_STREAMING>), dim3(workloads::persistent_grid(tiles, 4)), block, 0, s, in, out, tiles);
+          break;
+        case dispatch::CopyForm::kTwoTiles:
+          hipLaunchKernelGGL((copy_manual_double<STORE_LDS, true>), dim3(workloads::persistent_grid(tiles, 4)), block, 0, s, in, out, tiles);
+          break;
+        case dispatch::CopyForm::kOneTileTwo:
+          hipLaunchKernelGGL(copy_single<true>, dim3(workloads::persistent_grid(tiles, 2)), block, 0, s, in, out, tiles);
+          break;
+      }
       break;
     case 1: hipLaunchKernelGGL(copy_single<false>, dim3(workloads::persistent_grid(tiles, 8)), block, 0, s, in, out, tiles); break;
     case 5: hipLaunchKernelGGL(copy_single<true>, dim3(workloads::persistent_grid(tiles, 2)), block, 0, s, in, out, tiles); break;

@@ -15,6 +15,7 @@ _SHIM = r"""
 #include "dispatch.hpp"
 extern "C" int tile_walk(int m, int n, int k, int rows, int cols, int per_cu, int cus) { return dispatch::tile_walk(m, n, k, rows, cols, per_cu, cus); }
 extern "C" int gemm_form(int m, int n, int k, int cus) { return (int)dispatch::gemm_form(m, n, k, cus); }
+extern "C" int copy_form(unsigned long long bytes) { return (int)dispatch::copy_form(bytes); }
 // every tile once?
 extern "C" int visits_once(int tiles_m, int tiles_n, int walk, int* seen)
 {
@@ -87,3 +88,12 @@ LONG_ROWS, DEALT_32, DEALT_32_64, DEALT_64, DEALT_64_TWO, TILE_128_FAR, TILE_128
     ((2048, 2176, 1920), TILE_128), ((4096, 4096, 4096), TILE_256), ((1408, 2176, 1920), TILE_128_FAR), ((128, 128, 71_600_128), LONG_ROWS)])
 def test_kernel_of_the_default_gemm(rules, shape, form):
     assert rules.gemm_form(*shape, CUS) == form
+
+
+def test_kernel_of_the_default_copy(rules):
+    tile, mib = 16 << 10, 1 << 20
+    one_tile_four, two_tiles_streaming, two_tiles, one_tile_two = range(4)
+    rules.copy_form.argtypes = [ctypes.c_ulonglong]
+    for size, form in ((tile, one_tile_four), (16 * mib, one_tile_four), (16 * mib + tile, two_tiles_streaming), (44 * mib, two_tiles_streaming),
+                       (44 * mib + tile, two_tiles), (48 * mib, two_tiles), (96 * mib, two_tiles), (96 * mib + tile, one_tile_two), (8 << 30, one_tile_two)):
+        assert rules.copy_form(size) == form, size

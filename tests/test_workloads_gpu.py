@@ -96,8 +96,8 @@ def test_sequential_copy_beyond_four_gibibytes(device):
     assert torch.equal(dst.view(torch.int32), src.view(torch.int32))
 
 
-# the default copy around the lines between its kernels: 16, 48 and 96 MiB
-@pytest.mark.parametrize("tiles", [1023, 1024, 1025, 3072, 3073, 4096, 4097, 6144, 6145])
+# the default copy around the lines between its kernels: 16, 44 and 96 MiB
+@pytest.mark.parametrize("tiles", [1023, 1024, 1025, 2816, 2817, 3072, 3073, 4096, 4097, 6144, 6145])
 def test_default_copy_around_its_lines(device, tiles):
     src = wl.fill_uniform(torch.empty(tiles * wl.SEQ_TILE_BYTES // 4, device=device), 31)
     buf = torch.full((src.numel() + 64,), 7.0, device=device)
