@@ -166,4 +166,19 @@ inline CopyForm copy_form(const unsigned long long bytes)
   return 2 * bytes <= kCacheAssistedBytes ? CopyForm::kTwoTiles : CopyForm::kOneTileTwo;
 }
 
+// ---- row sums of a gather, four tiles in a transfer: workgroups per compute unit ----
+// Four where the Infinity Cache holds the table or the call is over soon.  A larger table wants a shorter queue; how short is a matter of a few
+// per cent (us with two / three / four, from the caches where they hold a part):
+//   384 MiB  2 Mi indices 44.3 / 44.6 / 44.7   8 Mi 162.8 / 166.8 / 168.3   32 Mi 628 / 645 / 653
+//   640 MiB  2 Mi 46.1 / 44.9 / 45.2           8 Mi 159.7 / 163.4 / 165.1   32 Mi 618 / 627 / 636
+//   768 MiB  4 Mi 84.6 / 88.6 / 88.7           8 Mi 163.2 / 161.5 / 162.1   32 Mi 637 / 627 / 636
+//   1 GiB    4 Mi 86.0 / 86.6 / 87.1           8 Mi 173.7 / 165.9 / 167.2   16 Mi 335 / 324 / 328
+//   1.5 GiB  8 Mi 182.1 / 176.0 / 177.3        4 GiB  2 Mi 45.6 / 46.4 / 47.4 (from DRAM 54.6 / 52.4 / 52.7)   16 Mi 392 / 384 / 390
+// From DRAM three are level or ahead by up to 5 % below 4 Mi indices and behind by 3 % beyond 8 Mi up to 512 MiB.
+inline int rowsum_workgroups(const unsigned long long table_bytes, const unsigned long long n_idx)
+{
+  if (table_bytes <= 256ull << 20 || n_idx <= 1ull << 20) return 4;
+  return table_bytes <= 640ull << 20 || (table_bytes <= 1ull << 30 && n_idx <= 6ull << 20) ? 2 : 3;
+}
+
 }  // namespace dispatch

@@ -5,6 +5,7 @@
 // Two consumers:
 //   copy   out[i] = table[idx[i]]                       (checks every moved byte)
 //   rowsum out[t][j] = sum_r tile[r][j], r ascending     (the reported workload)
+#include "dispatch.hpp"
 #include "workloads.hpp"
 
 namespace {
@@ -207,14 +208,12 @@ int launch_gather(const float* d_table, const int32_t* d_idx, float* d_out, size
     // The library's choice: short lists as above.  Longer ones take four tiles in one transfer, whose sums occupy all compute threads (with one
     // tile in turn a quarter of one of the two wavefronts adds while the DMA wavefronts wait for the buffer): 16 KiB in flight per
     // workgroup instead of 8, a quarter of the hand-offs.  It counts where an L2 holds the table (us, variant 6 / this: 6 Mi indices of 24000
-    // records 104 / 51, of 60000 106 / 66, 1 Mi of 24000 21 / 13); elsewhere what is in flight does, and four workgroups per compute unit become
-    // two or three where the table exceeds the Infinity Cache (4 Mi records, 32 Mi indices 632 / 619; two 617, three 639, four 646; 32 Mi records,
-    // 16 Mi indices 378, two 382, three 376, four 384).  Between 64 and 112 Ki indices the short form is 0.3 us ahead from the caches, beyond
+    // records 104 / 51, of 60000 106 / 66, 1 Mi of 24000 21 / 13); elsewhere what is in flight does.
+    // Between 64 and 112 Ki indices the short form is 0.3 us ahead from the caches, beyond
     // the long one (2 Mi records, 176 Ki indices 4.6 / 4.6 and from DRAM 7.8 / 7.4; 24000, 256 Ki 5.2 / 4.6 and 6.3 / 6.0).
     if (n_idx <= (112u << 10)) variant = 1;
     else {
-      const size_t table = n_records * (size_t)kRecBytes;
-      const int wgs = table <= (256ull << 20) || n_idx <= (1u << 20) ? 4 : table <= (1ull << 30) ? 2 : 3;
+      const int wgs = dispatch::rowsum_workgroups(n_records * (unsigned long long)kRecBytes, n_idx);
       hipLaunchKernelGGL((gather_manual<Consumer, 1, true, 4>), grid(wgs, (tiles + 3) / 4), block, 0, s, d_table, d_idx, d_out, tiles);
       CUDADMA_HIP_CHECK(hipGetLastError());
       return CUDADMA_OK;

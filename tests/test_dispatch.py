@@ -16,6 +16,7 @@ _SHIM = r"""
 extern "C" int tile_walk(int m, int n, int k, int rows, int cols, int per_cu, int cus) { return dispatch::tile_walk(m, n, k, rows, cols, per_cu, cus); }
 extern "C" int gemm_form(int m, int n, int k, int cus) { return (int)dispatch::gemm_form(m, n, k, cus); }
 extern "C" int copy_form(unsigned long long bytes) { return (int)dispatch::copy_form(bytes); }
+extern "C" int rowsum_workgroups(unsigned long long table, unsigned long long n_idx) { return dispatch::rowsum_workgroups(table, n_idx); }
 // every tile once?
 extern "C" int visits_once(int tiles_m, int tiles_n, int walk, int* seen)
 {
@@ -97,3 +98,12 @@ def test_kernel_of_the_default_copy(rules):
     for size, form in ((tile, one_tile_four), (16 * mib, one_tile_four), (16 * mib + tile, two_tiles_streaming), (44 * mib, two_tiles_streaming),
                        (44 * mib + tile, two_tiles), (48 * mib, two_tiles), (96 * mib, two_tiles), (96 * mib + tile, one_tile_two), (8 << 30, one_tile_two)):
         assert rules.copy_form(size) == form, size
+
+
+def test_workgroups_of_the_default_row_sums(rules):
+    mib, mi = 1 << 20, 1 << 20
+    rules.rowsum_workgroups.argtypes = [ctypes.c_ulonglong] * 2
+    for table, indices, workgroups in ((256 * mib, 32 * mi, 4), (4096 * mib, mi, 4), (257 * mib, mi + 32, 2), (512 * mib, 32 * mi, 2), (640 * mib, 32 * mi, 2),
+                                       (768 * mib, 6 * mi, 2), (768 * mib, 8 * mi, 3), (1024 * mib, 16 * mi, 3), (1024 * mib, 4 * mi, 2),
+                                       (1025 * mib, 2 * mi, 3), (8192 * mib, 32 * mi, 3)):
+        assert rules.rowsum_workgroups(table, indices) == workgroups, (table, indices)

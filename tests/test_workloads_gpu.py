@@ -427,7 +427,7 @@ def test_default_transpose_around_its_further_lines(device, n):
 
 
 # the default row sums beyond 112 Ki indices: four tiles in one transfer, the last one moved back where four does not divide the tiles; one
-# transfer and several for a workgroup, and the tables at which the number of workgroups changes (256 MiB, 1 GiB; beyond 1 Mi indices)
+# transfer and several for a workgroup, and the tables at which the number of workgroups changes (256 MiB, 1 GiB; beyond 1 Mi indices; 640 MiB beyond 6 Mi)
 @pytest.mark.parametrize("n_idx", [112 << 10, (112 << 10) + 32, (112 << 10) + 64, (112 << 10) + 96, 4 * 32 * 1024 + 128, (1 << 20) + 32, 3 * (1 << 20) - 32])
 @pytest.mark.parametrize("recs", [1, 3000, (2 << 20) + 1, (8 << 20) + 1])
 def test_default_gather_rowsum_transfers(device, n_idx, recs):
@@ -441,6 +441,11 @@ def test_default_gather_rowsum_transfers(device, n_idx, recs):
         want += rows[:, r]
     assert torch.equal(got, want)
     assert bool(torch.isnan(buf[n_idx // 32:]).all())
+
+
+@pytest.mark.parametrize("recs", [5 << 20, (5 << 20) + 1])
+def test_default_gather_rowsum_of_many_indices(device, recs):
+    test_default_gather_rowsum_transfers(device, 6 * (1 << 20) + 96, recs)
 
 
 @pytest.mark.parametrize("n_idx", [1 << 18, (1 << 18) + 32])
