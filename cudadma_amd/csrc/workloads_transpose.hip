@@ -295,6 +295,10 @@ transpose_double_groups(const float* __restrict__ in, float* __restrict__ out, c
 // all four wavefronts move the tile into LDS, meet, and all four write it out
 // transposed.  The next tile is requested (two-phase call) before the current one
 // is consumed, so its loads are in flight under the LDS reads and the stores.
+// ALL_AT_ONCE: as many workgroups as tiles, none of which has a next one.  Requesting a tile that is never used all the same doubled the loads (us
+// from the caches and from DRAM, with and without: 1024 2.80 / 2.72 and 3.53 / 3.38; 1152 3.43 / 3.12 and 3.89 / 3.80; 1536 4.16 / 3.61 and 5.9 / 5.6; 1728 3.94 /
+// 3.61 and 5.78 / 5.82; 1280 and 1408 3.47 / 3.21 and 3.54 / 3.34, from DRAM 4.42 / 4.63 and 4.45 / 4.60).
+template<bool ALL_AT_ONCE>
 __global__ void __launch_bounds__(kDmaThreads + kComputeThreads)
 transpose_not_specialized(const float* __restrict__ in, float* __restrict__ out, const int n, const int num_tiles,
                           const int band)
@@ -319,9 +323,11 @@ transpose_not_specialized(const float* __restrict__ in, float* __restrict__ out,
   for (; t < num_tiles; t += stride) {
     dma.template wait_xfer_finish<true, LOAD_CACHE_ALL, STORE_LDS>(buf);
     __syncthreads();
-    // past the last tile the last one is requested again: the loads stay unconditional
-    const int tn = (t + stride < num_tiles) ? (t + stride) : last;
-    dma.template start_xfer_async<true, LOAD_CACHE_ALL, STORE_LDS>(src_of(tn));
+    if constexpr (!ALL_AT_ONCE) {
+      // past the last tile the last one is requested again: the loads stay unconditional
+      const int tn = (t + stride < num_tiles) ? (t + stride) : last;
+      dma.template start_xfer_async<true, LOAD_CACHE_ALL, STORE_LDS>(src_of(tn));
+    }
     vec4_t v[4];
     const vec4_t* row = (const vec4_t*)(buf + lane * kLdsRow) + w * 4;
 #pragma unroll
@@ -781,7 +787,7 @@ extern "C" int cudadma_strided_transpose(const float* d_in, float* d_out, int n,
   // Infinity Cache, and its short queue only costs (us from the caches and from DRAM, variant 10 / 11: 2112 9.6 / 5.2 and 10.2 / 7.5; 3008 16.0 / 11.3 and
   // 15.8 / 13.0; 3712 21.8 / 17.9 and 22.4 / 22.1; beyond, variant 11 still gains from the caches and loses from DRAM: 3840 22.3 / 19.1 and 23.8 /
   // 25.3).  Up to three tiles per compute unit the tile is best moved by every wavefront, with no hand-off (variant 4), as many workgroups as
-  // there are tiles (variant 11 / 4: 1024 3.3 / 2.8 and 3.6 / 3.5; 1408 3.8 / 3.3 and 4.5 / 4.3; 1728 4.1 / 3.8 and 6.2 / 5.7; 1984 4.6 / 4.3 and 6.7 / 8.0).
+  // there are tiles (variant 11 / 4: 1024 3.3 / 2.7 and 3.6 / 3.4; 1408 3.8 / 3.3 and 4.5 / 4.6; 1728 4.1 / 3.6 and 6.2 / 5.8; 1984, beyond, 4.6 / 4.3 and 6.7 / 8.0).
   // All three store non-temporally.  With plain stores the output takes the place of the input in the caches: variant 11 2112 6.2
   // and 9.4, 2496 8.3 and 12.0; variant 4, one workgroup per compute unit, 1408 3.8 and 5.9.
   int small_per_cu = 1;
@@ -789,9 +795,10 @@ extern "C" int cudadma_strided_transpose(const float* d_in, float* d_out, int n,
     if (tiles <= 3 * workloads::device_cus()) { variant = 4; small_per_cu = 4; }
     else if (8LL * n * n <= (108LL << 20)) variant = 11;
   }
-  // The kernels with one LDS tile (variants 1 and 4) run best with exactly one workgroup per compute unit, i.e. one
-  // 16 KB tile of loads in flight per compute unit, and with the tiles walked down the columns (the workgroups that
-  // run together then write whole output rows); the others with four workgroups and bands of 16 tile rows.
+  // The kernels with one LDS tile (variants 1 and 4) run best with exactly one workgroup per compute unit where the matrix comes from DRAM, i.e.
+  // one 16 KB tile of loads in flight per compute unit, and with the tiles walked down the columns (the workgroups that
+  // run together then write whole output rows); the others with four workgroups and bands of 16 tile rows.  Up to three tiles per compute
+  // unit variant 0 has them all in flight at once.
   const bool one_tile = variant == 0 || variant == 1 || variant == 4 || variant == 10 || variant == 14;
   int band = workloads::tuning("transpose_band", one_tile ? tiles_per_side : kDefaultBand);
   if (band > tiles_per_side) band = tiles_per_side;
@@ -852,7 +859,12 @@ extern "C" int cudadma_strided_transpose(const float* d_in, float* d_out, int n,
     case 12:
     case 13: CUDADMA_REQUIRE(false, "variants 12 and 13 are sweep kernels: build the library with make EXTRA=-DHIPDMA_SWEEP_VARIANTS");
 #endif
-    default: hipLaunchKernelGGL(transpose_not_specialized, grid_for(small_per_cu), block, 0, s, d_in, d_out, n, tiles, band); break;
+    default: {
+      const dim3 grid = grid_for(small_per_cu);
+      if ((int)grid.x >= tiles) hipLaunchKernelGGL(transpose_not_specialized<true>, grid, block, 0, s, d_in, d_out, n, tiles, band);
+      else hipLaunchKernelGGL(transpose_not_specialized<false>, grid, block, 0, s, d_in, d_out, n, tiles, band);
+      break;
+    }
   }
   CUDADMA_HIP_CHECK(hipGetLastError());
   return CUDADMA_OK;

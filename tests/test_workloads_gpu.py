@@ -426,6 +426,19 @@ def test_default_transpose_around_its_further_lines(device, n):
     test_default_transpose_around_its_lines(device, n)
 
 
+@pytest.mark.parametrize("workgroups_per_cu", [0, 1])
+@pytest.mark.parametrize("n", [1024, 1088, 1728])
+def test_default_transpose_of_few_tiles_in_one_round_and_in_several(device, n, workgroups_per_cu):
+    """As many workgroups as tiles, which request no second one, and one per compute unit, which do."""
+    wl.set_workgroups_per_cu(workgroups_per_cu)
+    try:
+        test_default_transpose_around_its_lines(device, n)
+        src = wl.fill_uniform(torch.empty((n, n), device=device), 45)
+        assert torch.equal(wl.strided_transpose(src, torch.zeros((n, n), device=device), 4), src.t())
+    finally:
+        wl.set_workgroups_per_cu(0)
+
+
 # the default row sums beyond 112 Ki indices: four tiles in one transfer, the last one moved back where four does not divide the tiles; one
 # transfer and several for a workgroup, and the tables at which the number of workgroups changes (256 MiB, 1 GiB; beyond 1 Mi indices; 640 MiB beyond 6 Mi)
 @pytest.mark.parametrize("n_idx", [112 << 10, (112 << 10) + 32, (112 << 10) + 64, (112 << 10) + 96, 4 * 32 * 1024 + 128, (1 << 20) + 32, 3 * (1 << 20) - 32])
