@@ -236,7 +236,8 @@ __device__ __forceinline__ void load_to_lds_scalar_base(const char* scalar_base,
 #undef HIPDMA_LOAD_TO_LDS_ASM
 #pragma clang diagnostic pop
 
-// Wait until every global -> LDS move of this wavefront has landed.
+// Wait until every global -> LDS move of this wavefront has landed.  The builtin counts as an access to any memory: plain LDS reads that
+// follow it in the source stay behind it, with no barrier or fence.
 __device__ __forceinline__ void wait_lds_direct()
 {
   // s_waitcnt vmcnt(0): simm16 = vmcnt[3:0] | expcnt[6:4] | lgkmcnt[11:8] | vmcnt[15:14]

@@ -257,6 +257,36 @@ def test_headers_compile_standalone_for_gfx950(tmp_path, header, flags):
     assert res.returncode == 0, res.stderr[-2000:]
 
 
+_WAIT_KERNEL = r"""
+#include "hipDMA.h"
+__global__ void k(const float* in, float* out)
+{
+  __shared__ float buf[64];
+  buf[threadIdx.x ^ 1] = in[threadIdx.x];
+  __syncthreads();
+  const float before = buf[threadIdx.x];
+  hipdma::%s;
+  out[threadIdx.x] = before + 3.0f * buf[threadIdx.x];
+}
+"""
+
+
+@pytest.mark.parametrize("wait, counter", [("wait_direct_loads<0>()", "vmcnt(0)"), ("wait_direct_loads<5>()", "vmcnt(5)"), ("detail::wait_lds_direct()", "vmcnt(0)")])
+def test_plain_lds_reads_stay_behind_the_wait_for_direct_loads(tmp_path, wait, counter):
+    """The compiler does not see what a direct-to-LDS load writes.  Kernels whose wavefronts read their own stage right after the wait, with no
+    barrier between, rely on the wait being read as an access to any memory: the same word read before and after it is read twice."""
+    import shutil
+    hipcc = shutil.which("hipcc") or "/opt/rocm/bin/hipcc"
+    if not os.path.exists(hipcc):
+        pytest.skip("no hipcc")
+    (tmp_path / "wait.hip").write_text(_WAIT_KERNEL % wait)
+    subprocess.run([hipcc, "-std=c++17", "-O3", "--offload-arch=gfx950", "--cuda-device-only", "-S", str(tmp_path / "wait.hip"), "-o", str(tmp_path / "wait.s"),
+                    "-I", os.path.join(ROOT, "include"), "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops"], check=True, capture_output=True, timeout=300)
+    text = (tmp_path / "wait.s").read_text().split("s_endpgm")[0]
+    order = re.findall(r"ds_read_b32|s_waitcnt " + re.escape(counter), text.split("s_barrier")[-1])
+    assert order.count("ds_read_b32") == 2 and order.index("s_waitcnt " + counter) == 1, order
+
+
 # ---- the harness refuses, on the host, a run whose transfer would leave the caller's buffers ----
 def _fake_run(case_id, case, io, **over):
     """cudadma_run_case with pointers that are never dereferenced: every refusal tested here happens before
