@@ -488,7 +488,7 @@ def main():
                 "ceiling": ceiling, "frac_of_ceiling": round(value / ceiling, 4) if ceiling else None,
                 "ceiling_kind": "best read + write yardstick of this run on the same buffers (plain copy, hipMemcpyDtoDAsync, "
                                 "copy at its best launch shape)",
-                "counters_collected_at": counters.get("collected_at_commit")}
+                "counters_collected_at": (counters.get("patterns", {}).get("strided") or {}).get("collected_at_commit")}
     if "read_only" in yardsticks and "write_only" in yardsticks:
         r, w = yardsticks["read_only"]["GB/s"], yardsticks["write_only"]["GB/s"]
         roofline["read_then_write_bound"] = round(2.0 / (1.0 / r + 1.0 / w), 1)     # 1 GiB read alone, then 1 GiB written alone

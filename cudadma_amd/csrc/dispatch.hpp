@@ -109,8 +109,8 @@ inline GemmForm gemm_form(const int m, const int n, const int k, const int compu
   // 17.0 / 14.8 / 20.4.  The last one has a wavefront only two or three steps below k = 512, and
   // then 128 x 128 is as fast or faster (1152 x 1792 x 256 from the caches 5.5 / 5.1, from DRAM 5.9 / 5.7; x 512 6.4 / 6.6 and 7.0 / 7.5; x 768 7.7 / 8.1 and 8.8 / 10.0).
   // With long rows 128 x 128 has caught up (256 x 6656 x 6144 45.0 / 42.0 and 63.4 / 61.3; 768 x 2560 x 3072 24.0 / 22.3 and 29.7 / 30.7); where
-  // nearly every compute unit has two of them it does so from k = 1900 on from the caches, not from DRAM (2304 x 1536 x 2304 7 % slower and 21 % faster, 1152 x 2432 x
-  // 1920 1 % faster and 18 %).  A product of two rows of more than 80 of them is nearly all B, which a tile of 64 columns fetches in pieces of
+  // nearly every compute unit has two of them it does so from k = 1900 on from the caches, not from DRAM (1152 x 1536 x 2304 18.8 / 17.4 and 19.7 / 23.8,
+  // 768 x 2432 x 1920 15.7 / 15.2 and 18.5 / 20.5, 3968 x 512 x 2176 16.9 / 16.8 and 19.6 / 23.3).  A product of two rows of more than 80 of them is nearly all B, which a tile of 64 columns fetches in pieces of
   // 128 bytes: 128 x 128 is ahead there from k = 1024 on (128 x 11776 x 2176 10 % and 8 %, 128 x 14464 x 1664 5 % and 4 %, 128 x 16384 x 1024 0 % and 7 %; 128 x 10624 x 1536
   // 2 % slower and 1 % faster.  With 80 128 x 10240 x 1792 is 7 % and 19 % slower).
   const long long t32 = (long long)(m / 32) * (n / 32);

@@ -59,6 +59,8 @@ void launch_sgemv_ring(hipStream_t s, int n, int m, float alpha, const float* a,
 // Narrower matrices and longer leading dimensions go through small panels, and so do those with more rows than 64 per compute
 // unit: several workgroups then share a compute unit and hide each other's hand-offs (20480 x 4096 64 us, ring of 64 rows 72; 32768 x 4096 85 and
 // 95), and narrow ones from 40 on (12288 x 224 from DRAM 5.7, ring of 16 rows 6.3).
+// With 256 to about 300 columns and more than 32 rows per compute unit no shape is ahead in both states (10496 x 256: rings 3.8 / 4.6 / 4.5 and 6.4 / 6.2 /
+// 5.7, panels of 32 columns 5.3 and 6.1; a lane per row with panels of 128 columns 4.3 and 5.9).
 // From 112 rows on the longer pieces of 128 rows count, in bursts of 64 bytes a thread (64 / 128 rows: 32768 x 2048 42 / 39 us, 98304 x 1024
 // 76 / 72).
 void launch_sgemv_double(hipStream_t s, int n, int m, float alpha, const float* a, int lda, const float* x, float* y)

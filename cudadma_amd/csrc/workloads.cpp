@@ -130,7 +130,7 @@ static const VariantInfo kHalo[] = {
 static const VariantInfo kGemm[] = {
   {"the library's choice: variant 9, or its kernel with a 128 x 128 tile (80 KB of LDS and two workgroups per compute unit, or 144 KB "
    "and one with requests further ahead), whichever takes its rounds over the compute units in less time; for up to two 64 x 64 tiles per "
-   "compute unit (beyond one, for k from 512 to 3071) tiles of 64 x 64, 32 x 64 or 32 x 32 whose wavefronts take K steps in turn and add their partial sums"},
+   "compute unit (beyond one, for k from 512 to 3071, with m = 128 and n > 10240 to 1023) tiles of 64 x 64, 32 x 64 or 32 x 32 whose wavefronts take K steps in turn and add their partial sums"},
   {"warp-specialised: two DMA wavefronts per operand with two CudaDMAStrided objects each (two LDS stages, tile two K "
    "steps ahead in flight), four compute wavefronts with v_mfma_f32_32x32x16_bf16, B fragments through "
    "ds_read_b64_tr_b16; 128 x 128 workgroup tile, 64 x 64 per compute wavefront, two workgroups per compute unit"},

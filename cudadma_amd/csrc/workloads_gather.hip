@@ -26,21 +26,19 @@ typedef dma_of<1> dma_t;
 struct CopyConsumer {
   static constexpr bool kWritesEveryRecord = true;
   template<int TILES>
-  static __device__ __forceinline__ void run(const char* lds_tiles, float* __restrict__ out, const long long tile, const dma_of<TILES>& dma)
+  static __device__ __forceinline__ void run(const char* lds_tile, float* __restrict__ out, const long long tile, const dma_of<TILES>& dma)
   {
-    constexpr int kEach = TILES * kTileBytes / 16 / kComputeThreads;
-    vec4_t v[kEach];
-    const vec4_t* src = (const vec4_t*)lds_tiles;
-#pragma unroll
-    for (int i = 0; i < kEach; ++i) v[i] = src[threadIdx.x + i * kComputeThreads];
+    static_assert(TILES == 1 && kTileBytes == 2 * 16 * kComputeThreads, "two vectors per compute thread");
+    vec4_t v[2];
+    const vec4_t* src = (const vec4_t*)lds_tile;
+    v[0] = src[threadIdx.x];
+    v[1] = src[threadIdx.x + kComputeThreads];
     dma.start_async_dma();
     // Non-temporal: the records written are not read again, and lines of them would push those of the table out of the L2 (us, plain /
     // non-temporal: 6 Mi records from a table of 24000 248 / 136, 24000 x 512 Ki from DRAM 23 / 15; 8 Mi from one of 4 Mi 367 / 319).
     vec4_t* dst = (vec4_t*)(out + tile * (kTileBytes / 4));
-#pragma unroll
-    for (int i = 0; i < kEach; ++i) {
-      __builtin_nontemporal_store(v[i], &dst[threadIdx.x + i * kComputeThreads]);
-    }
+    __builtin_nontemporal_store(v[0], &dst[threadIdx.x]);
+    __builtin_nontemporal_store(v[1], &dst[threadIdx.x + kComputeThreads]);
   }
 };
 

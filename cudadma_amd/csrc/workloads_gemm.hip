@@ -1103,8 +1103,9 @@ gemm_bf16_all_direct_a64(const unsigned short* __restrict__ a, const unsigned sh
 // wavefront brings its own operands with direct-to-LDS loads into a stage of its own and is the only one to read them, so nothing in the loop
 // waits for another wavefront: no barrier, no hand-off, s_waitcnt alone.  It takes a whole stage into registers, and while it multiplies
 // it the next one is on its way into the same place.  At the end the partial tiles are added through LDS.
-// What bounds the loop is the LDS: direct loads land at about 100 B a cycle, fragments are read at 128, and the two share it.  32 x 32 takes 70
-// cycles per K = 32, 64 x 64 takes 126 to 144, against 434 of a 128 x 128 tile with four wavefronts, which is 4 to 16 times the work.
+// What bounds the loop is the way into the LDS: direct loads land at 64 B a cycle of a compute unit, however many wavefronts issue them (16 cycles
+// per KB; fragment reads take 4).  32 x 32 brings 4 KB per K = 32, 64 cycles, and takes 70; 64 x 64 brings 8 KB, 128 cycles, and takes 126 to
+// 144, against 417 to 434 of a 128 x 128 tile with four wavefronts, which is 4 to 16 times the work.
 // Measured (us, former choice -> this, from the caches and from DRAM): 512^3 6.0 -> 3.5 and 7.2 -> 4.0; 128 x 128 x 8192 48.7 -> 9.9 and 48.9 ->
 // 16.6; 1024^3 9.2 -> 6.2 and 10.1 -> 7.3; 2560 x 384 x 6528 40.7 -> 22.4 and 60 -> 28.
 // Stages of K = 32, two per wavefront, read A in pieces of 64 B, half a cache line: 1024 x 1024 x 4096 18.5 us, 16.4 so.  Four wavefronts with four

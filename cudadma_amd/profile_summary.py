@@ -81,15 +81,15 @@ def summarise(root):
     import bench
     out = {"patterns": {}, "calibration": {}}
     try:
-        out["collected_at_commit"] = subprocess.check_output(["git", "-C", ROOT, "rev-parse", "--short", "HEAD"], text=True).strip()
+        commit = subprocess.check_output(["git", "-C", ROOT, "rev-parse", "--short", "HEAD"], text=True).strip()
     except (OSError, subprocess.CalledProcessError):
-        out["collected_at_commit"] = None
+        commit = None
     for name in sorted(os.listdir(root)):
         pdir = os.path.join(root, name)
         kernel = bench.PATTERN_KERNELS.get(name)
         if not os.path.isdir(pdir) or kernel is None:
             continue
-        row = {"kernel": kernel}
+        row = {"kernel": kernel, "collected_at_commit": commit}
         algorithmic = None
         tj = os.path.join(pdir, "trace.json")
         if os.path.exists(tj):

@@ -607,7 +607,8 @@ def test_gemm_full_size(device, variant):
 
 
 # tile grids that divide into eight blocks and that do not (fewer tiles than XCDs, bands of tile rows with a remainder, rows of tiles
-# that eight divides, a large C of few K steps), both tiles of the default variant, one and several rounds
+# that eight divides, a large C of few K steps), one and several rounds: with 128 x 128 tiles in variant 1, by default with both of its large tiles
+# and, for the grids of few tiles, with those whose wavefronts share the K steps
 @pytest.mark.parametrize("shape", [(128, 128, 128), (128, 896, 256), (384, 1152, 128), (1152, 1408, 384), (2944, 2432, 128), (2816, 2816, 256),
                                    (3072, 3072, 128), (3328, 3840, 128), (2176, 3072, 256), (4224, 4224, 128), (1280, 4096, 256), (640, 2048, 1024),
                                    (768, 4096, 128)])
@@ -622,7 +623,8 @@ def test_gemm_tile_walks(device, shape, variant):
 
 
 # the default variant's form with eight stages of B (one tile or none for a compute unit, from 768 columns of A on): K steps that end in
-# either half of its loop, and both sides of the lines to its neighbours
+# either half of its loop, and both sides of the lines to its neighbours, among them, for two rows of many 64 x 64 tiles, the dealt K steps below
+# 1024 (128 x 128 is all theirs)
 @pytest.mark.parametrize("m, n", [(128, 128), (1408, 2176), (2048, 2048), (2048, 2176), (128, 10368)])
 @pytest.mark.parametrize("k", [384, 640, 768, 896, 1920])
 def test_gemm_stages(device, m, n, k):
